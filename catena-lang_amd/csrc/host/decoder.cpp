@@ -271,7 +271,7 @@ int forward(catena_decoder& m, const uint32_t* tokens, uint32_t batch, uint32_t 
       TRY(gemm_bf16_rope_qkv(XN, wqkv, static_cast<const float*>(m.rope_tab), lens, Q, kc, vc, rows, d,
                              tq, c.n_heads, c.max_len));
     } else {
-      TRY(catena_mi355x_gemm_bf16(XN, wqkv, QKV, rows, 3 * d, d, 1));
+      TRY(gemm_bf16(XN, wqkv, QKV, rows, 3 * d, d, 1, false));
       TRY(catena_mi355x_rope_qkv_bf16(QKV, inv, lens, Q, kc, vc, batch, tq, c.n_heads, c.head_dim,
                                       c.max_len));
     }
@@ -290,7 +290,7 @@ int forward(catena_decoder& m, const uint32_t* tokens, uint32_t batch, uint32_t 
       else
         TRY(residual_parts_rmsnorm_bf16(X, P, parts_o, AP, nullptr, H, HN, rows, rows, d));
     } else {
-      TRY(catena_mi355x_gemm_bf16(ATT, static_cast<const uint16_t*>(m.w_o[l]), AP, rows, d, d, 1));
+      TRY(gemm_bf16(ATT, static_cast<const uint16_t*>(m.w_o[l]), AP, rows, d, d, 1, false));
       TRY(catena_mi355x_residual_rmsnorm_bf16(X, AP, nullptr, H, HN, rows, d));
     }
     const uint16_t* wgu = static_cast<const uint16_t*>(m.w_gu[l]);
@@ -308,7 +308,7 @@ int forward(catena_decoder& m, const uint32_t* tokens, uint32_t batch, uint32_t 
       // (4x the bytes of act) is never written
       TRY(catena_mi355x_gemm_bf16_silu(HN, wgu, ACT, rows, 2 * f, d));
     } else {
-      TRY(catena_mi355x_gemm_bf16(HN, wgu, GU, rows, 2 * f, d, 1));
+      TRY(gemm_bf16(HN, wgu, GU, rows, 2 * f, d, 1, false));
       TRY(catena_mi355x_silu_mul_bf16(GU, ACT, rows, (uint32_t)f, 64));
     }
     if (step)
@@ -319,7 +319,7 @@ int forward(catena_decoder& m, const uint32_t* tokens, uint32_t batch, uint32_t 
     else if (down_split)
       TRY(gemm_bf16_f32_ksplit(ACT, static_cast<const uint16_t*>(m.w_down[l]), PF, rows, d, f, kPfSplits));
     else
-      TRY(catena_mi355x_gemm_bf16(ACT, static_cast<const uint16_t*>(m.w_down[l]), FO, rows, d, f, 1));
+      TRY(gemm_bf16(ACT, static_cast<const uint16_t*>(m.w_down[l]), FO, rows, d, f, 1, false));
   }
   float* FH = static_cast<float*>(A(CATENA_DEC_FINAL_H));
   uint16_t* FXN = static_cast<uint16_t*>(A(CATENA_DEC_FINAL_XN));
@@ -344,7 +344,7 @@ int forward(catena_decoder& m, const uint32_t* tokens, uint32_t batch, uint32_t 
     }
     TRY(gemm_bf16_decode(FXN, wlm, LG, batch, c.vocab, d, DecodeEpilogue::Argmax, e));
   } else {
-    TRY(catena_mi355x_gemm_bf16(FXN, wlm, LG, batch, c.vocab, d, 1));
+    TRY(gemm_bf16(FXN, wlm, LG, batch, c.vocab, d, 1, false));
     TRY(catena_mi355x_argmax_f32(LG, next, batch, c.vocab));
   }
   return CATENA_OK;

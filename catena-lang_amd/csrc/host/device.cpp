@@ -56,6 +56,19 @@ const KernelSpec kKernels[] = {
     {KernelId::GemmF32ExactQ16, "gemm_f32_exact", "catena_gemm_f32_exact_q16"},
     {KernelId::GemmBf16EdgeBf16, "gemm_bf16", "catena_gemm_bf16_edge_bf16out"},
     {KernelId::GemmBf16EdgeF32, "gemm_bf16", "catena_gemm_bf16_edge_f32out"},
+    {KernelId::GemmBf16Any128x128F32, "gemm_bf16_any", "catena_gemm_bf16_any_128x128_f32out"},
+    {KernelId::GemmBf16Any128x128Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_128x128_bf16out"},
+    {KernelId::GemmBf16Any64x128F32, "gemm_bf16_any", "catena_gemm_bf16_any_64x128_f32out"},
+    {KernelId::GemmBf16Any64x128Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_64x128_bf16out"},
+    {KernelId::GemmBf16Any64x64F32, "gemm_bf16_any", "catena_gemm_bf16_any_64x64_f32out"},
+    {KernelId::GemmBf16Any64x64Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_64x64_bf16out"},
+    {KernelId::GemmBf16Any32x64F32, "gemm_bf16_any", "catena_gemm_bf16_any_32x64_f32out"},
+    {KernelId::GemmBf16Any32x64Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_32x64_bf16out"},
+    {KernelId::GemmBf16Any32x32F32, "gemm_bf16_any", "catena_gemm_bf16_any_32x32_f32out"},
+    {KernelId::GemmBf16Any32x32Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_32x32_bf16out"},
+    {KernelId::PackRowsBf16, "gemm_bf16_any", "catena_pack_rows_bf16"},
+    {KernelId::GemmBf16K32EdgeF32, "gemm_bf16_k32", "catena_gemm_bf16_k32_edge_f32out"},
+    {KernelId::GemmBf16K32EdgeBf16, "gemm_bf16_k32", "catena_gemm_bf16_k32_edge_bf16out"},
     {KernelId::GemmBf16LdsBf16, "gemm_bf16_lds", "catena_gemm_bf16_lds_bf16out"},
     {KernelId::GemmBf16LdsF32, "gemm_bf16_lds", "catena_gemm_bf16_lds_f32out"},
     {KernelId::GemmBf16K32Bf16, "gemm_bf16_k32", "catena_gemm_bf16_k32_bf16out"},

@@ -16,8 +16,21 @@ enum class KernelId : int {
   GemmF32Exact = 0,
   GemmF32ExactT16,  // 16x16 tiles for small outputs (gemm_f32_exact.hip)
   GemmF32ExactQ16,  // 16x16 tiles, A by DPP row broadcast: k % 16 == 0, m % 4 == 0
-  GemmBf16EdgeBf16,  // general shapes, bounds-checked (gemm_bf16.hip)
+  GemmBf16EdgeBf16,  // no alignment, no scratch, any size (gemm_bf16.hip)
   GemmBf16EdgeF32,
+  GemmBf16Any128x128F32,  // ragged and small shapes (gemm_bf16_any.hip), f32 / bf16 per tile
+  GemmBf16Any128x128Bf16,
+  GemmBf16Any64x128F32,
+  GemmBf16Any64x128Bf16,
+  GemmBf16Any64x64F32,
+  GemmBf16Any64x64Bf16,
+  GemmBf16Any32x64F32,
+  GemmBf16Any32x64Bf16,
+  GemmBf16Any32x32F32,
+  GemmBf16Any32x32Bf16,
+  PackRowsBf16,  // an operand copied to 16-byte rows (gemm_bf16_any.hip)
+  GemmBf16K32EdgeF32,  // the 256 x 256 tile kernel on ragged shapes
+  GemmBf16K32EdgeBf16,
   GemmBf16LdsBf16,  // aligned tiles with K % 128 != 0: two 64-k stages (gemm_bf16_lds.hip)
   GemmBf16LdsF32,
   GemmBf16K32Bf16,  // four 32-k stages, spread buffer loads, LDS-staged epilogue (default)
@@ -172,6 +185,11 @@ int pool_alloc(uint64_t len, void** out);
 int pool_free(void* ptr);
 uint64_t pool_capacity(void* ptr);
 int workspace(uint64_t bytes, void** out);
+
+// catena_mi355x_gemm_bf16 (kernels.cpp); may_split: the product may be folded
+// as k groups whose partials are added (another order of the same sum).
+int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_t m, uint64_t k,
+              int out_f32, bool may_split);
 
 // Extra operands of the fused decode-GEMM epilogues; layout shared with
 // struct DecodeEpi in gemm_bf16_decode.hip (passed by value as a kernel

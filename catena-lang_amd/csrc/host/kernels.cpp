@@ -1,4 +1,6 @@
 // Kernel ABI: shape checks, kernel selection and launches.
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -61,6 +63,94 @@ uint32_t decode_kw(uint64_t n_cols, uint64_t k, bool regs_path) {
   }
   if (kw > k) kw = ceil_div(k, 32) * 32;
   return (uint32_t)kw;
+}
+// The tile kernels of a product, with what the choice between them weighs.
+// `alone` and `shared`: microseconds per 32-k slab of one workgroup that has
+// its CU to itself, and of each of the `fit` workgroups that share a CU;
+// `stream`: GB/s at which one CU brings a weight in from HBM (the narrower
+// the tile's rows, the less).  Fitted to 2,900 timings of the five general
+// kernels and the ragged 256 x 256 one over n = 17 .. 4000, widths 256 ..
+// 11264 and depths 512 .. 11008, 1 to 16 k groups: the tile it picks is on
+// average 2.4 % from the fastest (1.22x at worst, 0.5 % without k groups).
+struct GemmTile {
+  KernelId f32, bf16;
+  uint32_t bm, bn, waves, stages, stage_k, fit;
+  double alone, shared, stream;
+};
+constexpr GemmTile kGemmTiles[] = {
+    {KernelId::GemmBf16Any128x128F32, KernelId::GemmBf16Any128x128Bf16, 128, 128, 4, 2, 64, 2, 0.358, 0.211, 36.3},
+    {KernelId::GemmBf16Any64x128F32, KernelId::GemmBf16Any64x128Bf16, 64, 128, 4, 3, 64, 2, 0.217, 0.158, 36.3},
+    {KernelId::GemmBf16Any64x64F32, KernelId::GemmBf16Any64x64Bf16, 64, 64, 4, 2, 128, 2, 0.169, 0.105, 33.5},
+    {KernelId::GemmBf16Any32x64F32, KernelId::GemmBf16Any32x64Bf16, 32, 64, 4, 6, 128, 1, 0.120, 0.120, 33.5},
+    {KernelId::GemmBf16Any32x32F32, KernelId::GemmBf16Any32x32Bf16, 32, 32, 4, 4, 128, 2, 0.075, 0.067, 24.8},
+    {KernelId::GemmBf16K32EdgeF32, KernelId::GemmBf16K32EdgeBf16, 256, 256, 8, 4, 32, 1, 0.705, 0.705, 36.3},
+};
+constexpr int kTileRagged256 = 5;
+// k groups a product may be split into (with 1: whole)
+constexpr uint32_t kGemmSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+// row strides up to which the general kernels' 32-bit offsets reach (a stage
+// of 128 rows)
+constexpr uint64_t kGemmMaxStride = 1ull << 22;
+// most scratch one product takes: packed operands and partials (a product
+// that needs more runs on the kernel that needs none)
+constexpr uint64_t kGemmScratchMax = 1ull << 30;
+
+// k per group, in whole stages
+uint64_t gemm_k_len(uint64_t k, uint32_t splits, uint32_t stage_k) {
+  return ceil_div(ceil_div(k, splits), stage_k) * stage_k;
+}
+
+// Estimated microseconds.  A function of the shape alone (kDecodeSpread
+// stands for the CUs), so that the k groups, which fix the order of a sum,
+// are the same on every device.
+double gemm_cost(const GemmTile& t, uint64_t n, uint64_t m, uint64_t k, uint32_t splits) {
+  const double wgs = (double)ceil_div(n, t.bm) * (double)ceil_div(m, t.bn) * splits;
+  const double per_cu = std::ceil(wgs / kDecodeSpread);
+  const double whole = std::floor(per_cu / t.fit) * t.fit, left = per_cu - whole;
+  const double slab = whole * t.shared + (left > 0 ? std::max(t.alone, left * t.shared) : 0.0);
+  const double fold = (double)gemm_k_len(k, splits, t.stage_k) / 32 * slab;
+  const double weight = 2.0 * (double)k * (double)m / (std::min(wgs, (double)kDecodeSpread) * t.stream * 1e3);
+  const double out = 4.0 * (double)n * (double)m / 4.8e6;  // one f32 pass over the output
+  double us = 2.5 + std::max(fold, weight) + out * splits;
+  if (splits > 1) us += 2.8 + out * (splits + 1);  // the launch that adds the partials
+  return us;
+}
+
+struct GemmPlan {
+  int tile = 0;
+  uint32_t splits = 1;
+  double us = 0;
+};
+GemmPlan gemm_plan(uint64_t n, uint64_t m, uint64_t k, bool ragged256, bool may_split) {
+  GemmPlan best;
+  best.us = -1;
+  for (int i = 0; i < (int)(sizeof(kGemmTiles) / sizeof(kGemmTiles[0])); ++i) {
+    const GemmTile& t = kGemmTiles[i];
+    if (i == kTileRagged256 && !ragged256) continue;
+    if (ceil_div(n, t.bm) * ceil_div(m, t.bn) > 0x7FFFFFFFull) continue;
+    for (uint32_t s : kGemmSplits) {
+      if (s > 1 && (!may_split || i == kTileRagged256 || n * m * 4 * s > kGemmScratchMax / 4 ||
+                    ceil_div(k, gemm_k_len(k, s, t.stage_k)) != s))
+        continue;
+      const double us = gemm_cost(t, n, m, k, s);
+      if (best.us < 0 || us < best.us) best = GemmPlan{i, s, us};
+    }
+  }
+  return best;
+}
+
+// Y = P[0] + P[1] + ... + P[S-1] in ascending order, f32 or bf16
+int reduce_parts(const float* P, uint64_t S, uint64_t elems, void* Y, bool bf16) {
+  uint64_t stride4 = elems / 4;
+  uint32_t S32 = (uint32_t)S, b = bf16 ? 1u : 0u;
+  void* args[] = {&P, &stride4, &S32, &Y, &elems, &b};
+  return launch(KernelId::DecodeReduce, dim3((unsigned)ceil_div(elems, 1024)), dim3(256), 0, args);
+}
+
+int pack_rows(const uint16_t* src, uint64_t rows, uint64_t cols, uint16_t* dst, uint64_t ld) {
+  const uint64_t g = ceil_div(rows * (ld / 8), 256);
+  void* args[] = {&src, &rows, &cols, &dst, &ld};
+  return launch(KernelId::PackRowsBf16, dim3((unsigned)(g < 16384 ? g : 16384)), dim3(256), 0, args);
 }
 }  // namespace
 
@@ -169,10 +259,7 @@ int gemm_bf16_decode(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, 
     // instead of a completion ticket)
     st = launch(KernelId::GemmBf16DecodePartsNt, dim3((unsigned)gx, (unsigned)S), dim3(256), lds, args);
     if (st) return st;
-    uint64_t part_elems = (uint64_t)M * m, n4 = part_elems / 4;
-    uint32_t S32 = (uint32_t)S, bf16 = epi == DecodeEpilogue::StoreBf16 ? 1u : 0u;
-    void* rargs[] = {&P, &part_elems, &S32, &Y, &n4, &bf16};
-    return launch(KernelId::DecodeReduce, dim3((unsigned)ceil_div(n4, 256)), dim3(256), 0, rargs);
+    return reduce_parts(P, S, (uint64_t)M * m, Y, epi == DecodeEpilogue::StoreBf16);
   }
   return launch(id, dim3((unsigned)gx, (unsigned)S), dim3(256), lds, args);
 }
@@ -295,6 +382,138 @@ int gemm_bf16_rope_qkv(const uint16_t* a, const uint16_t* w, const float* tab, c
   return launch(KernelId::GemmBf16K32N128Rope, dim3((unsigned)grid), dim3(512), lds, args);
 }
 
+// bf16 product of any shape.  Every kernel below adds the same 32-k MFMA
+// steps in the same ascending order per output element, so which one runs
+// never changes the bits, except where a product is split into k groups
+// (f32 partials added in ascending order): ragged shapes with few tiles
+// only, never the aligned shapes, whose bits the fused projections share.
+// may_split = false keeps the one order throughout (the decoder).
+int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_t m, uint64_t k,
+              int out_f32, bool may_split) {
+  int st = ensure_init();
+  if (st) return st;
+  if (n == 0 || m == 0) return CATENA_OK;
+  if (!c || (k > 0 && (!a || !b))) return fail(CATENA_ERR_INVALID_ARGUMENT, "null operand");
+  Device& d = device();
+
+  // decode shape: <= 16 rows of activations against a K x N weight
+  if (n <= 16 && k > 0 && m % 8 == 0 && k % 8 == 0 && aligned16(a) && aligned16(b) &&
+      aligned16(c))
+    return gemm_bf16_decode(a, b, c, n, m, k,
+                            out_f32 ? DecodeEpilogue::StoreF32 : DecodeEpilogue::StoreBf16,
+                            DecodeEpiArgs{}, nullptr, 0);
+
+  const bool ptr_ok = aligned16(a) && aligned16(b) && aligned16(c);
+  const bool tile_ok = n % 256 == 0 && m % 256 == 0 && k % 64 == 0 && k > 0 && ptr_ok;
+  // the 32-k stage kernels need K % 128 == 0 (whole groups of 4 stages);
+  // they address A's 256-row tile and B's 32-row slab with
+  // 32-bit buffer offsets
+  const bool k32_ok = k % 128 == 0 && k > 0 && k <= (1ull << 22) && m <= (1ull << 24);
+  const bool n128_ok = n % 256 == 0 && m % 128 == 0 && k32_ok && ptr_ok;
+  const uint64_t tiles = ceil_div(n, 256) * ceil_div(m, 256);
+  if (ceil_div(n, 256) * ceil_div(m, 128) > 0x7FFFFFFFu)
+    return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
+  const bool strides_ok = k <= kGemmMaxStride && m <= kGemmMaxStride;
+  // Aligned shapes: direct-to-LDS kernels (8 waves): the four-stage 32-k
+  // kernel on 256 x 256 tiles, or on 256 x 128 tiles when N % 256 == 128 or
+  // when that takes fewer rounds of the chip; the two-stage 64-k kernel when
+  // K % 128 != 0.  With fewer than 160 of the narrow tiles most CUs would be
+  // idle: then the general kernels' smaller tiles are faster (256 x 2048 x
+  // 2048: 16 narrow tiles take 38 us, 256 tiles of 32 x 64 10 us; 1024 x
+  // 6144 x 2048: 192 narrow tiles and 128 x 128 tiles both 35 us).
+  if ((tile_ok || n128_ok) && !((n / 256) * ceil_div(m, 128) < 160 && strides_ok)) {
+    void* args[] = {&a, &b, &c, &n, &m, &k};
+    KernelId id;
+    size_t lds;
+    uint64_t grid;
+    if (k32_ok && (!tile_ok || prefer_n128(n, m, d.cu_count))) {
+      id = out_f32 ? KernelId::GemmBf16K32N128F32 : KernelId::GemmBf16K32N128Bf16;
+      lds = 4ull * (256 + 128) * 32 * sizeof(uint16_t);  // 98304 B
+      grid = (n / 256) * (m / 128);
+    } else if (k32_ok) {
+      id = out_f32 ? KernelId::GemmBf16K32F32 : KernelId::GemmBf16K32Bf16;
+      lds = 4ull * (256 + 256) * 32 * sizeof(uint16_t);  // 131072 B
+      grid = tiles;
+    } else {
+      id = out_f32 ? KernelId::GemmBf16LdsF32 : KernelId::GemmBf16LdsBf16;
+      lds = 2ull * (256 * 64 + 64 * 256) * sizeof(uint16_t);  // 131072 B
+      grid = tiles;
+    }
+    if (lds > d.max_lds) return fail(CATENA_ERR_UNSUPPORTED, "device LDS %zu < %zu", d.max_lds, lds);
+    return launch(id, dim3((unsigned)grid), dim3(512), lds, args);
+  }
+
+  // General shapes.  An operand whose rows do not all start on 16 bytes is
+  // packed into the library's scratch first (A's rows to whole 32-k slabs);
+  // partials of k groups go there too.  Where there is no scratch -- the
+  // stream is being captured (a graph would keep the address, and growing the
+  // block is not allowed), the product would need too much, or the device has
+  // none left -- a product runs unsplit, or, if it needs packing, on the
+  // bounds-checked kernel of gemm_bf16.hip, which also takes strides past the
+  // 32-bit offsets here.
+  const bool pack_a = k > 0 && (k % 8 != 0 || !aligned16(a));
+  const bool pack_b = k > 0 && (m % 8 != 0 || !aligned16(b));
+  if (strides_ok) {
+    const uint64_t lda = pack_a ? ceil_div(k, 32) * 32 : k, ldb = pack_b ? ceil_div(m, 8) * 8 : m;
+    const uint64_t a_bytes = pack_a ? ceil_div(n * lda * 2, 256) * 256 : 0;
+    const uint64_t b_bytes = pack_b ? ceil_div(k * ldb * 2, 256) * 256 : 0;
+    const bool ragged256 = k > 0 && (k % 32 == 0 || pack_a);
+    const bool splittable = may_split && !tile_ok && !n128_ok && n * m % 4 == 0;
+    GemmPlan p = gemm_plan(n, m, k, ragged256, splittable);
+    uint64_t need = a_bytes + b_bytes + (p.splits > 1 ? p.splits * n * m * 4 : 0);
+    std::unique_lock<std::mutex> ws_guard(d.ws_mu, std::defer_lock);
+    char* ws = nullptr;
+    if (need > 0) {
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      const bool scratch_ok = need <= kGemmScratchMax &&
+                              hipStreamIsCapturing(d.stream, &cap) == hipSuccess &&
+                              cap == hipStreamCaptureStatusNone;
+      ws_guard.lock();  // the block stays ours until everything is launched
+      void* w = nullptr;
+      if (scratch_ok && workspace(need, &w) == CATENA_OK) {
+        ws = static_cast<char*>(w);
+      } else {
+        p = gemm_plan(n, m, k, ragged256, false);
+      }
+    }
+    if (ws || !(pack_a || pack_b)) {
+      const uint16_t *pa = a, *pb = b;
+      if (pack_a) {
+        st = pack_rows(a, n, k, reinterpret_cast<uint16_t*>(ws), lda);
+        if (st) return st;
+        pa = reinterpret_cast<uint16_t*>(ws);
+      }
+      if (pack_b) {
+        st = pack_rows(b, k, m, reinterpret_cast<uint16_t*>(ws + a_bytes), ldb);
+        if (st) return st;
+        pb = reinterpret_cast<uint16_t*>(ws + a_bytes);
+      }
+      const GemmTile& t = kGemmTiles[p.tile];
+      const size_t lds = (size_t)t.stages * t.stage_k * (t.bm + t.bn) * sizeof(uint16_t);
+      if (lds > d.max_lds) return fail(CATENA_ERR_UNSUPPORTED, "device LDS %zu < %zu", d.max_lds, lds);
+      const dim3 grid((unsigned)(ceil_div(n, t.bm) * ceil_div(m, t.bn)), p.splits);
+      float* parts = p.splits > 1 ? reinterpret_cast<float*>(ws + a_bytes + b_bytes) : nullptr;
+      void* out = parts ? parts : c;
+      const bool store_f32 = out_f32 || parts;
+      // four columns to a store of the general kernels, eight bf16 ones to one of the 256 x 256 kernel's
+      uint32_t vec = (parts || aligned16(c)) && m % (p.tile == kTileRagged256 && !store_f32 ? 8 : 4) == 0;
+      uint64_t k_len = p.splits > 1 ? gemm_k_len(k, p.splits, t.stage_k) : k;
+      uint64_t sa = lda, sb = ldb;
+      void* any_args[] = {&pa, &pb, &out, &n, &m, &k, &sa, &sb, &k_len, &vec};
+      void* edge_args[] = {&pa, &pb, &out, &n, &m, &k, &sa, &sb, &vec};
+      st = launch(store_f32 ? t.f32 : t.bf16, grid, dim3(64 * t.waves), lds,
+                  p.tile == kTileRagged256 ? edge_args : any_args);
+      if (st || !parts) return st;
+      return reduce_parts(parts, p.splits, n * m, c, !out_f32);
+    }
+  }
+  void* args[] = {&a, &b, &c, &n, &m, &k};
+  const size_t lds = 2ull * 2 * 256 * 72 * sizeof(uint16_t);  // 147456 B
+  if (lds > d.max_lds) return fail(CATENA_ERR_UNSUPPORTED, "device LDS %zu < %zu", d.max_lds, lds);
+  return launch(out_f32 ? KernelId::GemmBf16EdgeF32 : KernelId::GemmBf16EdgeBf16,
+                dim3((unsigned)tiles), dim3(256), lds, args);
+}
+
 }  // namespace catena
 
 extern "C" {
@@ -325,59 +544,7 @@ int catena_mi355x_gemm_f32_exact(const float* a, const float* b, float* c, uint6
 
 int catena_mi355x_gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_t m,
                             uint64_t k, int out_f32) {
-  int st = ensure_init();
-  if (st) return st;
-  if (n == 0 || m == 0) return CATENA_OK;
-  if (!c || (k > 0 && (!a || !b))) return fail(CATENA_ERR_INVALID_ARGUMENT, "null operand");
-  Device& d = device();
-
-  // decode shape: <= 16 rows of activations against a K x N weight
-  if (n <= 16 && k > 0 && m % 8 == 0 && k % 8 == 0 && aligned16(a) && aligned16(b) &&
-      aligned16(c))
-    return gemm_bf16_decode(a, b, c, n, m, k,
-                            out_f32 ? DecodeEpilogue::StoreF32 : DecodeEpilogue::StoreBf16,
-                            DecodeEpiArgs{}, nullptr, 0);
-
-  const bool ptr_ok = aligned16(a) && aligned16(b) && aligned16(c);
-  const bool tile_ok = n % 256 == 0 && m % 256 == 0 && k % 64 == 0 && k > 0 && ptr_ok;
-  // the 32-k stage kernels need K % 128 == 0 (whole groups of 4 stages);
-  // they address A's 256-row tile and B's 32-row slab with
-  // 32-bit buffer offsets
-  const bool k32_ok = k % 128 == 0 && k > 0 && k <= (1ull << 22) && m <= (1ull << 24);
-  const bool n128_ok = n % 256 == 0 && m % 128 == 0 && k32_ok && ptr_ok;
-  const uint64_t tiles = ceil_div(n, 256) * ceil_div(m, 256);
-  if (ceil_div(n, 256) * ceil_div(m, 128) > 0x7FFFFFFFu)
-    return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
-  void* args[] = {&a, &b, &c, &n, &m, &k};
-  // Aligned shapes: direct-to-LDS kernels (8 waves), all with the same
-  // per-accumulator k32 order, so the choice between them never changes the
-  // bits: the four-stage 32-k kernel on 256 x 256 tiles, or on 256 x 128
-  // tiles when N % 256 == 128 or when that takes fewer rounds of the chip;
-  // the two-stage 64-k kernel when K % 128 != 0.
-  if (tile_ok || n128_ok) {
-    KernelId id;
-    size_t lds;
-    uint64_t grid;
-    if (k32_ok && (!tile_ok || prefer_n128(n, m, d.cu_count))) {
-      id = out_f32 ? KernelId::GemmBf16K32N128F32 : KernelId::GemmBf16K32N128Bf16;
-      lds = 4ull * (256 + 128) * 32 * sizeof(uint16_t);  // 98304 B
-      grid = (n / 256) * (m / 128);
-    } else if (k32_ok) {
-      id = out_f32 ? KernelId::GemmBf16K32F32 : KernelId::GemmBf16K32Bf16;
-      lds = 4ull * (256 + 256) * 32 * sizeof(uint16_t);  // 131072 B
-      grid = tiles;
-    } else {
-      id = out_f32 ? KernelId::GemmBf16LdsF32 : KernelId::GemmBf16LdsBf16;
-      lds = 2ull * (256 * 64 + 64 * 256) * sizeof(uint16_t);  // 131072 B
-      grid = tiles;
-    }
-    if (lds > d.max_lds) return fail(CATENA_ERR_UNSUPPORTED, "device LDS %zu < %zu", d.max_lds, lds);
-    return launch(id, dim3((unsigned)grid), dim3(512), lds, args);
-  }
-  const size_t lds = 2ull * 2 * 256 * 72 * sizeof(uint16_t);  // 147456 B
-  if (lds > d.max_lds) return fail(CATENA_ERR_UNSUPPORTED, "device LDS %zu < %zu", d.max_lds, lds);
-  return launch(out_f32 ? KernelId::GemmBf16EdgeF32 : KernelId::GemmBf16EdgeBf16,
-                dim3((unsigned)tiles), dim3(256), lds, args);
+  return gemm_bf16(a, b, c, n, m, k, out_f32, true);
 }
 
 int catena_mi355x_gemm_bf16_silu(const uint16_t* a, const uint16_t* b, uint16_t* act, uint64_t n,

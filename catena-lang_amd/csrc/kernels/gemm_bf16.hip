@@ -1,7 +1,10 @@
 // bf16 GEMM on gfx950 MFMA with a fixed, data-independent reduction order:
-// the general-shape (edge) kernel, for shapes the aligned tile kernels do not
-// take (M or N not a multiple of 256, K not a multiple of 64, unaligned
-// pointers).  Every load and store is bounds-checked; out-of-range A and B
+// the kernel that needs nothing: no alignment, no scratch memory, no limit on
+// the strides.  It loads by the element, so the general kernels of
+// gemm_bf16_any.hip (which pack unaligned operands into scratch) are 10 to 70
+// times faster; it runs when the row strides pass their 32-bit offsets, and
+// for unaligned operands while the stream is captured or when no scratch can
+// be had.  Every load and store is bounds-checked; out-of-range A and B
 // elements read as +0.
 //
 // Semantics: the reference's f32.matmul.row-major.materialize contraction

@@ -659,28 +659,29 @@ CATENA_DECODE_KERNEL(catena_gemm_bf16_decode_silu, EPI_SILU, 0)
 CATENA_DECODE_KERNEL(catena_gemm_bf16_decode_argmax, EPI_ARGMAX, 2)
 CATENA_DECODE_KERNEL(catena_gemm_bf16_decode_parts, EPI_PARTIALS, 0)
 
-// The split-K reduction of a plain decode GEMM, as a launch of its own after
-// the partials kernel (catena_gemm_bf16_decode_parts_nt): Y = ((P[0] + P[1]) + ...) + P[S-1]
-// elementwise, ascending s -- the adds the last-arriving workgroup of the
+// The split-K reduction of a plain GEMM, as a launch of its own after the
+// partials kernel: Y = ((P[0] + P[1]) + ...) + P[S-1] elementwise, ascending s
+// -- for the decode shapes the adds the last-arriving workgroup of the
 // ticketed form makes, so the same bits -- stored as f32 or as bf16 (RNE).
 // The launch boundary orders the partials before these loads, which takes
 // the place of the ticket's agent-scope release / acquire (an L2 write-back
 // per workgroup and an L2 invalidate per column block).  Four elements per
-// thread; n4 = M * N / 4.
+// thread; n = M * N, the partials stride4 * 4 elements apart.  Y that four
+// elements cannot be stored to at once (unaligned, or the last n % 4) is
+// written by the element.
 extern "C" __global__ __launch_bounds__(256) void catena_decode_reduce(const float* __restrict__ P,
-                                                                       uint64_t part_elems, uint32_t S,
-                                                                       void* __restrict__ Y, uint64_t n4,
+                                                                       uint64_t stride4, uint32_t S,
+                                                                       void* __restrict__ Y, uint64_t n,
                                                                        uint32_t out_bf16) {
   const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n4) return;
+  if (4 * i >= n) return;
   const f32x4_t* p4 = reinterpret_cast<const f32x4_t*>(P) + i;
-  const uint64_t st4 = part_elems / 4;
   f32x4_t sum = p4[0];
   for (uint32_t s0 = 1; s0 < S; s0 += 8) {
     f32x4_t v[8];
 #pragma unroll
     for (uint32_t u = 0; u < 8; ++u)
-      if (s0 + u < S) v[u] = p4[(s0 + u) * st4];
+      if (s0 + u < S) v[u] = p4[(s0 + u) * stride4];
 #pragma unroll
     for (uint32_t u = 0; u < 8; ++u)
       if (s0 + u < S) {
@@ -688,13 +689,26 @@ extern "C" __global__ __launch_bounds__(256) void catena_decode_reduce(const flo
         for (int q = 0; q < 4; ++q) sum[q] = sum[q] + v[u][q];
       }
   }
+  const bool whole = 4 * i + 4 <= n;
   if (out_bf16) {
     uint2 o;
     o.x = pack_bf16x2(sum[0], sum[1]);
     o.y = pack_bf16x2(sum[2], sum[3]);
-    reinterpret_cast<uint2*>(Y)[i] = o;
+    uint16_t* y = static_cast<uint16_t*>(Y) + 4 * i;
+    if (whole && (reinterpret_cast<uintptr_t>(Y) & 7u) == 0) {
+      *reinterpret_cast<uint2*>(y) = o;
+    } else {
+      const uint32_t left = n - 4 * i < 4 ? (uint32_t)(n - 4 * i) : 4u;
+      for (uint32_t q = 0; q < left; ++q) y[q] = (uint16_t)((q < 2 ? o.x : o.y) >> (16 * (q & 1)));
+    }
   } else {
-    reinterpret_cast<f32x4_t*>(Y)[i] = sum;
+    float* y = static_cast<float*>(Y) + 4 * i;
+    if (whole && (reinterpret_cast<uintptr_t>(Y) & 15u) == 0) {
+      *reinterpret_cast<f32x4_t*>(y) = sum;
+    } else {
+      const uint32_t left = n - 4 * i < 4 ? (uint32_t)(n - 4 * i) : 4u;
+      for (uint32_t q = 0; q < left; ++q) y[q] = q == 0 ? sum[0] : q == 1 ? sum[1] : q == 2 ? sum[2] : sum[3];
+    }
   }
 }
 

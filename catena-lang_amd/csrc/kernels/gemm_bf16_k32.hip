@@ -83,6 +83,9 @@ CATENA_DEV void tile_of(uint32_t bid, uint32_t tiles_m, uint32_t tiles_n, uint32
 // buffer descriptor word 3 for raw (unswizzled, stride 0) 32-bit access
 constexpr int kRsrcWord3 = 0x00020000;
 
+// Bytes of a descriptor over `n` elements, in 31 bits
+CATENA_DEV int records(uint64_t n) { return n > 0x3FFFFFF8ull ? 0x7FFFFFF0 : (int)(2 * n); }
+
 // The RoPE epilogue's operands (a fused q / k / v projection, one head per
 // 128-column tile): the rotation table [positions][64][2] (cos, sin), the
 // per-sequence lengths, q [M][H * 128] and the caches [B][H][L][128], bf16.
@@ -97,12 +100,21 @@ struct RopeQkv {
 
 // K is the depth this workgroup folds; lda (0: K) is A's row stride, which a
 // k-split launch sets to the whole depth (A and B then start at the split's
-// first k).
-template <bool OUT_BF16, int BN, bool SILU = false, bool ROPE = false>
+// first k).  EDGE: M, N and K need not be multiples of the tile.  Each slab's
+// descriptors then end at the operands' last rows, so rows past M and k rows
+// past K arrive as zeros without touching memory (A's columns K .. of the last
+// slab are zeros in memory: the host pads A's rows when K % 32 != 0), columns
+// past N read the next row and are not stored, and a part-filled last group of
+// S slabs runs on zeros, which leave every accumulator as it is.  B's row
+// stride is ldb; vec: C's rows take 16-byte stores.
+template <bool OUT_BF16, int BN, bool SILU = false, bool ROPE = false, bool EDGE = false>
 CATENA_DEV void gemm_k32_body(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                               void* __restrict__ C, uint64_t M, uint64_t N, uint64_t K,
-                              const RopeQkv& rq = RopeQkv{}, uint64_t lda = 0) {
+                              const RopeQkv& rq = RopeQkv{}, uint64_t lda = 0, uint64_t ldb = 0,
+                              uint32_t vec = 1) {
   const uint64_t LDA = lda ? lda : K;
+  const uint64_t LDB = EDGE ? ldb : N;
+  static_assert(!EDGE || (!SILU && !ROPE), "the fused epilogues take whole tiles");
   static_assert(!ROPE || BN == 128, "the RoPE epilogue pairs the two column waves of a 128-wide tile");
   static_assert(BN == 256 || BN == 128, "tile widths 256 and 128");
   constexpr int B_ST = BK * BN;                // elements per B stage
@@ -117,7 +129,8 @@ CATENA_DEV void gemm_k32_body(const uint16_t* __restrict__ A, const uint16_t* __
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, 0..7
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const uint32_t tiles_m = (uint32_t)(M / BM), tiles_n = (uint32_t)(N / BN);
+  const uint32_t tiles_m = (uint32_t)(EDGE ? (M + BM - 1) / BM : M / BM);
+  const uint32_t tiles_n = (uint32_t)(EDGE ? (N + BN - 1) / BN : N / BN);
   uint32_t tm, tn;
   tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const uint64_t m0 = (uint64_t)tm * BM, n0 = (uint64_t)tn * BN;
@@ -133,7 +146,7 @@ CATENA_DEV void gemm_k32_body(const uint16_t* __restrict__ A, const uint16_t* __
     aoff = (uint32_t)((r * LDA + 8 * q) * 2);
     const uint32_t kr = (64 / B_LANES) * wave + (uint32_t)lane / B_LANES;
     const uint32_t qb = (uint32_t)(lane % B_LANES) ^ hB(kr);
-    boff = (uint32_t)((kr * N + 8 * qb) * 2);
+    boff = (uint32_t)((kr * LDB + 8 * qb) * 2);
   }
   // Load idx (0, 1: A; 2 .. LOADS-1: B) of slab `slab` into stage `stage`.
   auto issue_one = [&](uint64_t slab, int stage, int idx) {
@@ -141,17 +154,19 @@ CATENA_DEV void gemm_k32_body(const uint16_t* __restrict__ A, const uint16_t* __
     const bool live = k0 < K;
     if (idx < 2) {
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(A + m0 * LDA + (live ? k0 : 0)), (short)0, live ? (int)(BM * LDA * 2) : 0, kRsrcWord3);
+          (void*)(A + m0 * LDA + (live ? k0 : 0)), (short)0,
+          !live ? 0 : EDGE ? records((M - m0 < BM ? M - m0 : BM) * LDA - k0) : (int)(BM * LDA * 2), kRsrcWord3);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rs, (lds_void*)(smem + stage * A_ST + (32 * wave + 16 * idx) * BK), 16, (int)aoff,
           idx ? (int)(16 * LDA * 2) : 0, 0, 0);
     } else {
       const int b = idx - 2;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(B + (live ? k0 : 0) * N + n0), (short)0, live ? (int)(BK * N * 2) : 0, kRsrcWord3);
+          (void*)(B + (live ? k0 : 0) * LDB + n0), (short)0,
+          !live ? 0 : EDGE ? records((K - k0 < BK ? K - k0 : BK) * LDB - n0) : (int)(BK * N * 2), kRsrcWord3);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rs, (lds_void*)(smem + S * A_ST + stage * B_ST + ((64 / B_LANES) * wave + 16 * b) * BN), 16,
-          (int)boff, b ? (int)(16 * N * 2) : 0, 0, 0);
+          (int)boff, b ? (int)(16 * LDB * 2) : 0, 0, 0);
     }
   };
 
@@ -298,7 +313,8 @@ CATENA_DEV void gemm_k32_body(const uint16_t* __restrict__ A, const uint16_t* __
     asm volatile("" ::: "memory");
   };
 
-  const uint64_t nk = K / BK;  // host guarantees nk % S == 0
+  // aligned shapes: the host guarantees nk % S == 0
+  const uint64_t nk = EDGE ? (K + BK - 1) / BK : K / BK;
 #pragma unroll
   for (int t = 0; t < S; ++t)
 #pragma unroll
@@ -498,17 +514,33 @@ CATENA_DEV void gemm_k32_body(const uint16_t* __restrict__ A, const uint16_t* __
       const u32x4_t v = *reinterpret_cast<const u32x4_t*>(wt + r * 128 + 16 * (cc ^ ((r >> 1) & 7u)));
       const uint64_t gr = m0 + wm * 16 * WI + r;
       const uint64_t gc = n0 + wn * 64 + 8 * cc;
-      *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(C) + gr * N + gc) = v;
+      uint16_t* dst = static_cast<uint16_t*>(C) + gr * N + gc;
+      if (EDGE && gr >= M) continue;
+      if (!EDGE || vec) {
+        if (!EDGE || gc < N) *reinterpret_cast<u32x4_t*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (gc + e < N) dst[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+      }
     }
   } else {
     // acc[i][j] lane (G, s) holds C[row 16 i + s][cols 16 j + 4G .. +3]
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
       const uint64_t gr = m0 + wm * 16 * WI + 16 * i + s;
+      if (EDGE && gr >= M) continue;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint64_t gc = n0 + wn * 64 + 16 * j + 4 * G;
-        *reinterpret_cast<f32x4_t*>(static_cast<float*>(C) + gr * N + gc) = acc[i][j];
+        float* dst = static_cast<float*>(C) + gr * N + gc;
+        if (!EDGE || vec) {
+          if (!EDGE || gc < N) *reinterpret_cast<f32x4_t*>(dst) = acc[i][j];
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (gc + q < N) dst[q] = acc[i][j][q];
+        }
       }
     }
   }
@@ -527,6 +559,18 @@ CATENA_GEMM_K32_KERNEL(catena_gemm_bf16_k32_bf16out, true, 256)
 CATENA_GEMM_K32_KERNEL(catena_gemm_bf16_k32_f32out, false, 256)
 CATENA_GEMM_K32_KERNEL(catena_gemm_bf16_k32n128_bf16out, true, 128)
 CATENA_GEMM_K32_KERNEL(catena_gemm_bf16_k32n128_f32out, false, 128)
+
+// Ragged shapes: grid = ceil(M / 256) * ceil(N / 256), same block and LDS.  lda,
+// ldb >= K, N: row strides, multiples of 8; A's row r holds zeros in columns
+// K .. the next multiple of 32.
+#define CATENA_GEMM_K32_EDGE_KERNEL(NAME, OUTB)                                           \
+  extern "C" __global__ __launch_bounds__(512) void NAME(                                 \
+      const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, void* __restrict__ C, \
+      uint64_t M, uint64_t N, uint64_t K, uint64_t lda, uint64_t ldb, uint32_t vec) {     \
+    gemm_k32_body<OUTB, 256, false, false, true>(A, B, C, M, N, K, RopeQkv{}, lda, ldb, vec); \
+  }
+CATENA_GEMM_K32_EDGE_KERNEL(catena_gemm_bf16_k32_edge_bf16out, true)
+CATENA_GEMM_K32_EDGE_KERNEL(catena_gemm_bf16_k32_edge_f32out, false)
 
 // SwiGLU-fused: C = act [M][N / 2] bf16 (N % 128 == 0), dynamic LDS the larger
 // of the stages and 4 up slots of 16 WI rows x 68 floats

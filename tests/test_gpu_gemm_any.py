@@ -1,0 +1,117 @@
+"""gemm_bf16 on shapes and addresses no aligned tile kernel takes: the general
+tile kernels, their k groups, the packing of rows that do not start on 16
+bytes, and the kernel that needs neither, at the sizes where they change."""
+import numpy as np
+import pytest
+
+import catena_amd as ca
+import oracle
+from gpu_util import as_f32, gemm_within_bound, say
+
+pytestmark = pytest.mark.gpu
+
+NAN16 = 0x7FC1  # what surrounds every operand: a value read past one shows in the product
+
+
+def _placed(bits: np.ndarray, shift: int):
+    """`bits` in a device buffer of NaNs, `shift` elements past a 256-byte line."""
+    flat = np.full(bits.size + 512, NAN16, np.uint16)
+    flat[128 + shift:128 + shift + bits.size] = bits.reshape(-1)
+    buf = ca.Buffer.from_array(flat)
+    return buf, buf.ptr + 2 * (128 + shift)
+
+
+def _product(a16, b16, out_f32, shifts=(0, 0, 0)):
+    """gemm_bf16 into the middle of a buffer whose other bytes must not move."""
+    n, k = a16.shape
+    m = b16.shape[1]
+    es = 4 if out_f32 else 2
+    (ab, ap), (bb, bp) = _placed(a16, shifts[0]), _placed(b16, shifts[1])
+    pad, fill = 256 + es * shifts[2], 0xA5
+    cb = ca.Buffer.from_array(np.full(n * m * es + 512 + es * shifts[2], fill, np.uint8))
+    ca.gemm_bf16(ap, bp, cb.ptr + pad, n, m, k, out_f32=out_f32)
+    raw = cb.read(np.uint8)
+    got = raw[pad:pad + n * m * es].copy().view(np.float32 if out_f32 else np.uint16).reshape(n, m)
+    assert np.all(raw[:pad] == fill) and np.all(raw[pad + n * m * es:] == fill)
+    return got
+
+
+def _inputs(n, m, k, seed):
+    rng = np.random.default_rng(seed)
+    return (oracle.f32_to_bf16_bits_np(rng.normal(0, 1, (n, k)).astype(np.float32)),
+            oracle.f32_to_bf16_bits_np(rng.normal(0, 1, (k, m)).astype(np.float32)))
+
+
+def _check(n, m, k, shifts=(0, 0, 0)):
+    say(f"bf16 gemm general {n}x{m}x{k} shifts {shifts}")
+    a16, b16 = _inputs(n, m, k, n + 3 * m + 7 * k)
+    g32 = _product(a16, b16, True, shifts)
+    gemm_within_bound(a16, b16, g32)
+    g16 = _product(a16, b16, False, shifts)
+    assert np.array_equal(g16, oracle.f32_to_bf16_bits_np(g32))
+    assert np.array_equal(_product(a16, b16, True, shifts).view(np.uint32), g32.view(np.uint32))
+    return a16, b16, g32
+
+
+# rows at the edges of 32, 64, 128 and 256-row tiles; widths and depths one off
+# a tile, a 16-byte chunk, a k step; from one tile to several rounds of them
+@pytest.mark.parametrize("n,m,k", [
+    (17, 8, 8), (31, 40, 32), (32, 32, 40), (33, 64, 120), (63, 72, 136), (64, 128, 96), (65, 136, 264),
+    (127, 248, 512), (129, 264, 1032), (255, 520, 96), (257, 256, 160), (513, 1032, 1000), (1000, 2056, 72),
+    (700, 3000, 232), (1, 1, 1), (3, 7, 1000), (16, 9, 64), (5, 64, 9), (40, 33, 31), (100, 127, 129),
+    (257, 511, 255), (300, 1000, 2), (20, 4096, 3), (256, 256, 128), (256, 384, 256), (512, 512, 640)])
+def test_general_shapes(n, m, k):
+    _check(n, m, k)
+
+
+# few tiles and a deep k: folded as 2 .. 16 k groups, the last one shorter
+@pytest.mark.parametrize("n,m,k", [(17, 256, 8192), (24, 96, 4104), (48, 4096, 2888), (64, 512, 8200), (100, 1024, 5000),
+                                   (33, 64, 16384), (20, 60, 4099)])
+def test_k_groups(n, m, k):
+    _check(n, m, k)
+
+
+# every address a caller may pass: 2, 4 and 8-byte aligned operands and outputs
+@pytest.mark.parametrize("shifts", [(1, 0, 0), (0, 1, 0), (0, 0, 1), (3, 5, 7), (4, 2, 2), (8, 8, 4)])
+@pytest.mark.parametrize("n,m,k", [(8, 136, 64), (130, 264, 192), (256, 256, 128)])
+def test_unaligned_operands(n, m, k, shifts):
+    _check(n, m, k, shifts)
+
+
+@pytest.mark.parametrize("n,m,k", [(999, 768, 256), (200, 1024, 544), (333, 1536, 160), (1000, 2048, 96)])
+def test_unsplit_bits_equal_the_aligned_kernels(n, m, k):
+    """A product that is not split has the bits of the same product padded to
+    whole tiles: rows and k rows of zeros change no other cell's MFMA steps."""
+    a16, b16, g32 = _check(n, m, k)
+    pn, pk = -(-n // 256) * 256, -(-k // 128) * 128
+    ap, bp = np.zeros((pn, pk), np.uint16), np.zeros((pk, m), np.uint16)
+    ap[:n, :k], bp[:k] = a16, b16
+    say(f"bf16 gemm padded {pn}x{m}x{pk}")
+    full = _product(np.concatenate([ap] * 5)[:5 * pn], bp, True)[:n]
+    assert np.array_equal(full.view(np.uint32), g32.view(np.uint32))
+
+
+def test_special_values_stay_in_their_row_and_column():
+    """An infinity or NaN of row i reaches row i only, also where k ends inside
+    a k step and the next row's values lie behind it (and so for columns)."""
+    n, m, k = 70, 200, 72
+    a16, b16 = _inputs(n, m, k, 5)
+    clean = _product(a16, b16, True)
+    a16[10, 0], a16[41, k - 1], b16[3, 77] = 0x7F80, 0x7FC0, 0xFF80
+    got = _product(a16, b16, True)
+    hit = np.zeros((n, m), bool)
+    hit[[10, 41]], hit[:, 77] = True, True
+    assert not np.isfinite(got[hit]).any()
+    assert np.array_equal(got[~hit].view(np.uint32), clean[~hit].view(np.uint32))
+
+
+def test_strides_past_the_32_bit_offsets():
+    """k past 2^22: the kernel with 64-bit addressing (small integers: every
+    partial sum exact, so any order gives the same bits)."""
+    n, m, k = 17, 8, (1 << 22) + 64
+    rng = np.random.default_rng(9)
+    a16 = oracle.f32_to_bf16_bits_np(rng.integers(-1, 2, (n, k)).astype(np.float32))
+    b16 = oracle.f32_to_bf16_bits_np(rng.integers(-1, 2, (k, m)).astype(np.float32))
+    say(f"bf16 gemm {n}x{m}x{k}")
+    got = _product(a16, b16, True)
+    assert np.array_equal(got, as_f32(a16) @ as_f32(b16).astype(np.float64))
