@@ -1,6 +1,7 @@
 // Kernel ABI of the decoder-block pieces (block.hip, causal attention) and
 // the program ABI of the two stdlib ops they mirror (nn.rmsnorm,
 // tensor.argmax-f32).
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
@@ -117,23 +118,52 @@ int attn_causal(const uint16_t* q, const uint16_t* k, const uint16_t* v, const u
   if (!aligned16(k) || !aligned16(v))
     return fail(CATENA_ERR_INVALID_ARGUMENT, "K/V caches must be 16-byte aligned");
   if (blocks > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "too many queries");
-  // Many queries per sequence: the block-of-16-queries kernel, which reads
-  // each K / V row once per block (its score buffer holds whole 64-key
-  // blocks of rows up to the longest prefix, bounded by len_bound (every
-  // lens[b] <= len_bound) and max_len, so it is used while two workgroups
-  // still fit a CU, bound <= 1088, and four share one for bounds up to 512;
-  // it reads q rows with 16-byte loads); otherwise the one-query-per-
-  // workgroup kernel.  Both give the same bits.
+  // Many queries per sequence: the block-of-16-queries kernels, which read
+  // each K / V row once per block and hold a block's scores in LDS, one row
+  // per key up to the longest prefix (bounded by len_bound: every lens[b] <=
+  // len_bound, and by max_len).  All of them, and the one-query-per-workgroup
+  // kernel, give the same bits.
+  //   * at most 64 blocks: one query per workgroup, since 16 times as many
+  //     workgroups then still find CUs (128 queries x 8 heads over 1028 keys:
+  //     56 us against 64 in 64 blocks; 200 queries, 104 blocks: 98 against 67);
+  //   * four waves while at least three workgroups share a CU (up to 704
+  //     rows) and there are more than two for each CU; eight otherwise, which
+  //     finish a block sooner and keep a CU busier where two blocks or one
+  //     fit (336 blocks of 333 x 400: 30 us against 34; 1408 of 700 x 828: 275
+  //     against 300; 2000 of 2000 x 2048: 470 against 583);
+  //   * up to 1088 rows two workgroups share a CU, up to 2304 one fits.  When
+  //     blocks with at most 1088 rows alone fill the chip's 512 places, they
+  //     get a launch with that buffer (500 queries after 500 cached, in 1100:
+  //     608 us against 824).
   const uint32_t rows_bound = len_bound < max_len ? len_bound : max_len;
-  const size_t lds_pf =
-      16 * 136 * 2 + 3 * 16 * 4 + 3 * 4 * 16 * 4 + (size_t)ceil_div(rows_bound, 64) * 64 * 17 * 4;
-  if (tq >= 8 && lds_pf <= 80 * 1024 && aligned16(q)) {
-    const uint64_t nqb = ceil_div(tq, 16);
-    const uint64_t grid = (uint64_t)batch * heads * nqb;
+  auto pf_lds = [](uint32_t waves, uint32_t rows) {
+    return 16 * 136 * 2 + 3 * 16 * 4 + (size_t)3 * waves * 16 * 4 + (size_t)ceil_div(rows, 64) * 64 * 17 * 4;
+  };
+  const uint64_t bh = (uint64_t)batch * heads, grid = bh * ceil_div(tq, 16);
+  if (tq >= 8 && grid > 64 && aligned16(q) && pf_lds(8, rows_bound) <= device().max_lds) {
     if (grid > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "too many query blocks");
-    void* pargs[] = {&q, &k, &v, &lens, &o, &batch, &heads, &max_len, &tq, &scale};
-    return launch(out_f32 ? KernelId::AttnPrefillD128F32 : KernelId::AttnPrefillD128Bf16,
-                  dim3((unsigned)grid), dim3(256), lds_pf, pargs);
+    const uint32_t nqb = (uint32_t)ceil_div(tq, 16);
+    // keys the queries before block qb may see: the last of them is followed
+    // by tq - 16 qb others
+    auto rows_before = [&](uint32_t qb) {
+      const uint64_t later = tq - std::min<uint64_t>(tq, 16ull * qb);
+      return rows_bound > later ? (uint32_t)(rows_bound - later) : 0u;
+    };
+    auto blocks_of = [&](uint32_t waves, uint32_t qb0, uint32_t n) {
+      const KernelId id = waves == 4 ? (out_f32 ? KernelId::AttnPrefillD128F32 : KernelId::AttnPrefillD128Bf16)
+                                     : (out_f32 ? KernelId::AttnPrefillW8D128F32 : KernelId::AttnPrefillW8D128Bf16);
+      void* pargs[] = {&q, &k, &v, &lens, &o, &batch, &heads, &max_len, &tq, &scale, &qb0, &n};
+      return launch(id, dim3((unsigned)(bh * n)), dim3(64 * waves), pf_lds(waves, rows_before(qb0 + n)), pargs);
+    };
+    if (rows_bound <= 704 && grid > 512) return blocks_of(4, 0, nqb);
+    uint32_t split = 0;  // query blocks below it have at most 1088 rows
+    if (rows_bound > 1088) {
+      while (split < nqb && rows_before(split + 1) <= 1088) ++split;
+      if (split * bh < 512) split = 0;
+    }
+    st = blocks_of(8, split, nqb - split);
+    if (st || split == 0) return st;
+    return blocks_of(8, 0, split);
   }
   const size_t lds = attn_lds_bytes(max_len);
   if (lds > device().max_lds)

@@ -97,6 +97,8 @@ const KernelSpec kKernels[] = {
     {KernelId::AttnCausalD128Bf16, "attn_decode", "catena_attn_causal_bf16_d128_bf16out"},
     {KernelId::AttnPrefillD128F32, "attn_prefill", "catena_attn_prefill_bf16_d128_f32out"},
     {KernelId::AttnPrefillD128Bf16, "attn_prefill", "catena_attn_prefill_bf16_d128_bf16out"},
+    {KernelId::AttnPrefillW8D128F32, "attn_prefill", "catena_attn_prefill_w8_bf16_d128_f32out"},
+    {KernelId::AttnPrefillW8D128Bf16, "attn_prefill", "catena_attn_prefill_w8_bf16_d128_bf16out"},
     {KernelId::EmbedRowsBf16, "block", "catena_embed_rows_bf16"},
     {KernelId::RmsnormRows, "block", "catena_rmsnorm_rows"},
     {KernelId::RopeQkvStore, "block", "catena_rope_qkv_store"},

@@ -59,6 +59,8 @@ enum class KernelId : int {
   AttnCausalD128Bf16,
   AttnPrefillD128F32,
   AttnPrefillD128Bf16,
+  AttnPrefillW8D128F32,  // eight waves a workgroup (attn_prefill.hip)
+  AttnPrefillW8D128Bf16,
   EmbedRowsBf16,
   RmsnormRows,
   RopeQkvStore,

@@ -8,14 +8,14 @@
 // math.hex:148-199), so every output is bitwise equal to the decode kernel
 // run on that query's prefix.
 //
-// One workgroup (4 waves) per (batch, head, block of QB = 16 consecutive
+// One workgroup (4 or 8 waves) per (batch, head, block of QB = 16 consecutive
 // queries); the queries of a block share every K and V row they read.
 // Query tq of sequence b attends to the first lens[b] - (Tq - 1 - tq)
 // positions (clamped to [0, L]).
 //
 // Scores: waves take 64-key blocks round robin; lane l owns key kb*64 + l
-// and holds its K row in registers (chunk c of the next block's row is
-// loaded as soon as chunk c of the current one is folded).  The fold over d
+// and holds its K row in registers (the eight chunks of a 128-byte line of the
+// next block's row are loaded once the current block's are folded).  The fold over d
 // runs on the matrix cores: v_mfma_f32_16x16x1_4b_f32 with A = the 16
 // queries' q_d (lane l: query l % 16, every block) and B = the 64 keys'
 // k_d (lane l: key l) adds q_d * k_{t,d} to each of the 16 x 64
@@ -34,10 +34,11 @@
 // Softmax: per query, the exact parallel form of the max fold (FirstMax,
 // common.h): each lane tracks the first maximum and the last NaN of the
 // scores it produces, rows of 16 lanes combine them by DPP and the max
-// phase combines the four waves' partials; exp~ elementwise; the
+// phase combines the waves' partials; exp~ elementwise; the
 // denominators are 16 independent serial folds, one lane per query;
 // p = e / den elementwise.
-// Output: wave w owns columns 32w .. 32w + 31 of all 16 queries.  The
+// Output: wave w owns columns 32w .. 32w + 31 of all 16 queries (of eight
+// waves, the even or the odd ones of such a range).  The
 // products p_t * v_{t,c} come from v_mfma_f32_16x16x1_4b_f32 with a zero
 // accumulator (one product, one rounding: fl(p * v)), four keys per
 // instruction; the VALU adds them to the running sums in ascending key
@@ -46,6 +47,16 @@
 // three workgroups share a CU at the C5 shape.  Keys below the shortest
 // prefix of the block need no mask; past it, a key beyond a query's prefix
 // leaves that query's sums untouched.
+//
+// What bounds it: issue on the VALU, which the f32 matrix instructions occupy
+// too (measured: 32 cycles of a SIMD per 16x16x1 instruction and about 2.4 per
+// add, added up, at four waves per SIMD; 2.6 to 4.2 per add at two).  At C5's
+// 512 keys and four workgroups per CU that is 90 % filled.  Where the score
+// buffer leaves one or two workgroups to a CU, eight waves instead of four keep
+// the SIMDs busier, and each load, LDS read and matrix instruction is issued
+// ahead of the adds it would hold up: 2000 queries x 16 heads in a 2048-row
+// cache 1400 us (one query per workgroup) -> 583 (four waves) -> 470 (eight) ->
+// 455 (blocks of up to 1088 keys two to a CU).
 #include "common.h"
 
 namespace {
@@ -53,7 +64,6 @@ constexpr int D = 128;
 constexpr int QH = D + 8;            // qh row stride (bf16): the MFMA A-operand reads (16 rows,
                                      // 16 bytes each) cover the 64 banks once
 constexpr int QB = 16;               // queries per workgroup
-constexpr int HALF = QB / 2;         // queries per score item / output thread
 constexpr int ST = QB + 1;           // sT row stride (floats)
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
@@ -94,22 +104,24 @@ CATENA_DEV uint32_t query_len(uint32_t lens_b, uint32_t L, uint32_t Tq, uint32_t
 }
 }  // namespace
 
-template <bool OUT_BF16>
+// NW: waves of the workgroup, 4 or 8
+template <bool OUT_BF16, int NW>
 CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                              const uint16_t* __restrict__ v, const uint32_t* __restrict__ lens,
                              void* __restrict__ o, uint32_t B, uint32_t H, uint32_t L,
-                             uint32_t Tq, float scale) {
+                             uint32_t Tq, float scale, uint32_t qb0, uint32_t nqb) {
+  constexpr int NT = 64 * NW;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   uint16_t* qh = reinterpret_cast<uint16_t*>(smem);                // [QB][QH] bf16
   float* red = reinterpret_cast<float*>(smem + QB * QH * 2);       // [QB] max, [QB] den
-  float* part = red + 3 * QB;  // [3][4 waves][QB]: first-max value, its index, last NaN
-  float* sT = part + 3 * 4 * QB;                                   // [Lmax][ST]
+  float* part = red + 3 * QB;  // [3][NW waves][QB]: first-max value, its index, last NaN
+  float* sT = part + 3 * NW * QB;                                   // [Lmax][ST]
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t BH = B * H;
-  const uint32_t nqb = (Tq + QB - 1) / QB;
-  // longest query blocks first; the blocks of one (b, h) are BH apart
-  const uint32_t qb = nqb - 1 - blockIdx.x / BH;
+  // query blocks qb0 .. qb0 + nqb - 1, longest first; the blocks of one (b, h)
+  // are BH apart
+  const uint32_t qb = qb0 + nqb - 1 - blockIdx.x / BH;
   const uint32_t bh = blockIdx.x % BH;
   const uint32_t b = bh / H, h = bh % H;
   const uint32_t t0 = qb * QB;
@@ -127,7 +139,7 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
   // `unsafe` notes a value outside the MFMA fold's exact range
   // thread t: row t / 16, values 8 (t % 16) .. +7 (one 16-byte load)
   int unsafe = 0;
-  {
+  if (NW == 4 || tid < 256) {
     const uint32_t i = (uint32_t)tid / 16, d0 = 8 * ((uint32_t)tid % 16);
     const u32x4_t w = i < nq ? *reinterpret_cast<const u32x4_t*>(q + (((uint64_t)b * Tq + t0 + i) * H + h) * D + d0)
                              : u32x4_t{0u, 0u, 0u, 0u};
@@ -182,10 +194,15 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
     // wave's next block (zeros past the rows) is loaded as soon as chunk c
     // of the current one has been folded, a whole block ahead of its use
     u32x4_t raw[D / 8];
+    // in chunk order: the waits inside the loop then leave 15 loads in flight
+    // (any other order here and they leave as few as it has after chunk 0's)
 #pragma unroll
-    for (int c = 0; c < D / 8; ++c) raw[c] = kchunk((uint32_t)wave * 64 + lane, c);
-    for (uint32_t kblk = wave; kblk < nkb; kblk += 4) {
-      const uint32_t jn = (kblk + 4) * 64 + lane;
+    for (int c = 0; c < D / 8; ++c) {
+      raw[c] = kchunk((uint32_t)wave * 64 + lane, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (uint32_t kblk = wave; kblk < nkb; kblk += NW) {
+      const uint32_t jn = (kblk + NW) * 64 + lane;
       f32x16_t acc;
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] = __uint_as_float(0u);
@@ -203,7 +220,13 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
           acc = __builtin_amdgcn_mfma_f32_16x16x1f32(bf16lo(qword), bf16lo(word), acc, 0, 0, 0);
           acc = __builtin_amdgcn_mfma_f32_16x16x1f32(bf16hi(qword), bf16hi(word), acc, 0, 0, 0);
         }
-        raw[c] = kchunk(jn, c);
+        // the eight chunks of a 128-byte line are requested together: one miss
+        // and seven hits per line (a chunk at a time, other rows' lines have
+        // pushed it out of the L1 before its next chunk is asked for)
+        if (c % 8 == 7) {
+#pragma unroll
+          for (int h = 7; h >= 0; --h) raw[c - h] = kchunk(jn, c - h);
+        }
         // one chunk at a time: its conversions and range check are not
         // hoisted ahead, nor the next block's load of it sunk behind
         __builtin_amdgcn_sched_barrier(0);
@@ -244,8 +267,8 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
       if ((lane & 15) == 0) {
         const int qi = 4 * (lane >> 4) + u;
         part[wave * QB + qi] = f.v;
-        part[4 * QB + wave * QB + qi] = __uint_as_float(f.i);
-        part[8 * QB + wave * QB + qi] = __int_as_float(n);
+        part[NW * QB + wave * QB + qi] = __uint_as_float(f.i);
+        part[2 * NW * QB + wave * QB + qi] = __int_as_float(n);
       }
     }
     // x - 1 wraps a zero to 0xFFFF: a minimum below kSafeLo - 1 is a nonzero
@@ -260,7 +283,7 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
     // (bf16 pairs, widened at each use) folded against each of the 16
     // queries (LDS broadcasts of the bf16 q rows), v_mul_f32 then v_add_f32
     // per product, d ascending
-    for (uint32_t kblk = wave; kblk < nkb; kblk += 4) {
+    for (uint32_t kblk = wave; kblk < nkb; kblk += NW) {
       u32x4_t raw[D / 8];
       kload(kblk, raw);
       const uint32_t j = kblk * 64 + lane;
@@ -293,8 +316,8 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
   __syncthreads();
 
   // ---------------------------------------------------------------- max per query
-  // Wave w takes queries w, w + 4, w + 8, w + 12: the last NaN position and
-  // the first max of the query's scores, from the four waves' partials of
+  // Wave w takes queries w, w + NW, ...: the last NaN position and
+  // the first max of the query's scores, from the waves' partials of
   // the matrix-core fold, or (after a VALU refold) from one pass over the
   // scores in which each lane keeps them for the positions it reads
   // (ascending).  Without a NaN in the query's prefix, the first-max combine
@@ -302,21 +325,22 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
   // as in the two-pass form; a query with a NaN takes that form (first max
   // after the last NaN, or the NaN itself when it is the last position).
   {
-    uint32_t len4[4];
-    int ln4[4];
-    FirstMax fm4[4];
+    constexpr int U = QB / NW;  // queries per wave
+    uint32_t len4[U];
+    int ln4[U];
+    FirstMax fm4[U];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) len4[u] = qlen[wave + 4 * u];
+    for (int u = 0; u < U; ++u) len4[u] = qlen[wave + NW * u];
     if (!refold) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = wave + 4 * u;
+      for (int u = 0; u < U; ++u) {
+        const int i = wave + NW * u;
         FirstMax f{__uint_as_float(0xFF800000u), 0xFFFFFFFFu};
         int n = -1;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          f = first_max_combine(f, FirstMax{part[w * QB + i], __float_as_uint(part[4 * QB + w * QB + i])});
-          const int nw = __float_as_int(part[8 * QB + w * QB + i]);
+        for (int w = 0; w < NW; ++w) {
+          f = first_max_combine(f, FirstMax{part[w * QB + i], __float_as_uint(part[NW * QB + w * QB + i])});
+          const int nw = __float_as_int(part[2 * NW * QB + w * QB + i]);
           n = nw > n ? nw : n;
         }
         fm4[u] = f;
@@ -325,14 +349,14 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
     } else {
       uint32_t lmx = 0;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) lmx = len4[u] > lmx ? len4[u] : lmx;
+      for (int u = 0; u < U; ++u) lmx = len4[u] > lmx ? len4[u] : lmx;
       // per lane the positions ascend, so its first maximum is kept by a
       // strict comparison (a NaN never replaces it; a lane holding only
       // -inf stays empty, which the combine treats as -inf)
-      float bv[4];
-      uint32_t bi[4];
+      float bv[U];
+      uint32_t bi[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < U; ++u) {
         bv[u] = __uint_as_float(0xFF800000u);
         bi[u] = 0xFFFFFFFFu;
         ln4[u] = -1;
@@ -340,9 +364,9 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
       for (uint32_t t = lane; t < lmx; t += 64) {
         const float* row = sT + t * ST + wave;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
           if (t < len4[u]) {
-            const float sv = row[4 * u];
+            const float sv = row[NW * u];
             if (sv != sv) ln4[u] = (int)t;
             if (sv > bv[u]) {
               bv[u] = sv;
@@ -352,12 +376,12 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
         }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) fm4[u] = FirstMax{bv[u], bi[u]};
-      // the four queries' butterflies interleaved (independent shuffle chains)
+      for (int u = 0; u < U; ++u) fm4[u] = FirstMax{bv[u], bi[u]};
+      // the queries' butterflies interleaved (independent shuffle chains)
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
           const int o = __shfl_xor(ln4[u], off, 64);
           ln4[u] = o > ln4[u] ? o : ln4[u];
           FirstMax b;
@@ -368,8 +392,8 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
       }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = wave + 4 * u;
+    for (int u = 0; u < U; ++u) {
+      const int i = wave + NW * u;
       const uint32_t len = len4[u];
       const int J = ln4[u];
       FirstMax fm;
@@ -395,19 +419,19 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
 
   // ---------------------------------------------------------------- exp~
   // four elements per thread in flight (each element's arithmetic unchanged)
-  for (uint32_t e0 = tid; e0 < lmax * QB; e0 += 4 * 256) {
+  for (uint32_t e0 = tid; e0 < lmax * QB; e0 += 4 * NT) {
     float sv[4], mv[4];
     bool live[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const uint32_t e = e0 + 256u * u, t = e / QB, i = e % QB;
+      const uint32_t e = e0 + (uint32_t)NT * u, t = e / QB, i = e % QB;
       live[u] = e < lmax * QB && t < qlen[i];
       sv[u] = live[u] ? sT[t * ST + i] : 0.0f;
       mv[u] = red[i];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const uint32_t e = e0 + 256u * u, t = e / QB, i = e % QB;
+      const uint32_t e = e0 + (uint32_t)NT * u, t = e / QB, i = e % QB;
       if (live[u]) {
         const float shifted = sv[u] - mv[u];
         sT[t * ST + i] = exp_approx(shifted);
@@ -463,28 +487,28 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
     red[QB + i] = den;
   }
   __syncthreads();
-  for (uint32_t e0 = tid; e0 < lmax * QB; e0 += 4 * 256) {
+  for (uint32_t e0 = tid; e0 < lmax * QB; e0 += 4 * NT) {
     float sv[4], dv[4];
     bool live[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const uint32_t e = e0 + 256u * u, t = e / QB, i = e % QB;
+      const uint32_t e = e0 + (uint32_t)NT * u, t = e / QB, i = e % QB;
       live[u] = e < lmax * QB && t < qlen[i];
       sv[u] = live[u] ? sT[t * ST + i] : 0.0f;
       dv[u] = red[QB + i];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const uint32_t e = e0 + 256u * u, t = e / QB, i = e % QB;
+      const uint32_t e = e0 + (uint32_t)NT * u, t = e / QB, i = e % QB;
       if (live[u]) sT[t * ST + i] = sv[u] / dv[u];
     }
   }
   __syncthreads();
 
   // ---------------------------------------------------------------- P V
-  // Wave w owns output columns 32w .. 32w + 31 of the 16 queries.  For each
-  // group of 4 keys t .. t + 3, two v_mfma_f32_16x16x1_4b_f32 with a zero
-  // accumulator form the 16 x 16 x 4 products (K = 1: one product, one
+  // Four waves: wave w owns output columns 32w .. 32w + 31 of the 16 queries.
+  // For each group of 4 keys t .. t + 3, two v_mfma_f32_16x16x1_4b_f32 with a
+  // zero accumulator form the 16 x 16 x 4 products (K = 1: one product, one
   // rounding, so each is fl(p * v), the reference's product; a -0 product
   // comes out +0, which no add below can tell apart: every sum starts at +0
   // and never becomes -0): block b = key t + b, row i = query i (A: lane
@@ -493,59 +517,105 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
   // Lane l receives in register 4kk + u the product of key t + kk, query
   // 4(l / 16) + u and its column pair l % 16, and adds it to that query's
   // two sums on the VALU, keys in ascending order (a key past the query's
-  // prefix is skipped).
+  // prefix is skipped).  Eight waves: wave w takes the even (w < 4) or odd
+  // column of each pair of wave w % 4's columns, one MFMA a group.
+  constexpr int NX = 8 / NW;  // columns per lane
   const uint32_t jp = (uint32_t)lane & 15, kq = (uint32_t)lane >> 4;
+  const uint32_t cw = (uint32_t)wave & 3u;
+  const uint32_t up = NW == 8 && wave < 4 ? 16u : 0u;  // the even column's bits move up
   uint32_t glen[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) glen[u] = qlen[4 * kq + u];
   // every real query of the block sees at least qlen[0] keys (padding rows'
   // sums are never stored)
   const uint32_t ng = (lmax + 3) / 4, nfull = qlen[0] / 4;
-  float s0[4], s1[4];
+  float sum[NX][4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) s0[u] = s1[u] = __uint_as_float(0u);
+  for (int x = 0; x < NX; ++x)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) sum[x][u] = __uint_as_float(0u);
   // V words by range-checked buffer loads (keys past lmax read zeros),
   // eight groups ahead of their use
   const __amdgpu_buffer_rsrc_t vrs =
       __builtin_amdgcn_make_buffer_rsrc((void*)vb, (short)0,
                                         __builtin_amdgcn_readfirstlane((int)(lmax * (uint32_t)D * 2u)), kRsrcWord3);
-  const int voff = (int)((kq * D + 32 * (uint32_t)wave + 2 * jp) * 2u);
+  const int voff = (int)((kq * D + 32 * cw + 2 * jp) * 2u);
   auto vload = [&](uint32_t t) -> uint32_t {
     return __builtin_amdgcn_raw_buffer_load_b32(vrs, voff + (int)(t * (uint32_t)D * 2u), 0, 0);
   };
   const float* pcol = sT + kq * ST + jp;  // p[jp][t + kq] at pcol[t * ST]
   const f32x16_t zero16 = {};
+  struct Products {
+    f32x16_t x[NX];
+  };
+  auto products = [&](float pv, uint32_t w) {
+    Products r;
+    r.x[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(pv, NW == 4 ? bf16lo(w) : bf16hi(w << up), zero16, 0, 0, 0);
+    if constexpr (NX == 2) r.x[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(pv, bf16hi(w), zero16, 0, 0, 0);
+    return r;
+  };
   uint32_t vw[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) vw[i] = vload(4u * i);
-  for (uint32_t g = 0; g < ng; g += 8) {
+  uint32_t g = 0;
+  // Eight groups at a time while every query sees all their keys: the V words
+  // and p values of the next eight are requested first, and each group's
+  // products are formed before the previous group's are added, so no load, LDS
+  // read or matrix instruction is waited for.  (What is formed ahead past the
+  // last whole eight is dropped; its p rows are clamped to the score rows.)
+  if (nfull >= 8) {
+    const uint32_t rlast = nkb * 64 - 32;
+    float pv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) pv[i] = pcol[4 * i * ST];
+    Products cur = products(pv[0], vw[0]);
+    for (; g + 8 <= nfull; g += 8) {
+      uint32_t vn[8];
+      float pn[8];
+      const uint32_t tn = 4 * (g + 8);
+      const float* pnext = pcol + (tn < rlast ? tn : rlast) * ST;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) vn[i] = vload(tn + 4u * i);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pn[i] = pnext[4 * i * ST];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        Products nxt = i < 7 ? products(pv[(i + 1) & 7], vw[(i + 1) & 7]) : products(pn[0], vn[0]);
+        // formed here, not where it is used
+#pragma unroll
+        for (int x = 0; x < NX; ++x) asm volatile("" : "+v"(nxt.x[x]));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int x = 0; x < NX; ++x) sum[x][u] = sum[x][u] + cur.x[x][4 * kk + u];
+        __builtin_amdgcn_sched_barrier(0);
+        cur = nxt;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        pv[i] = pn[i];
+        vw[i] = vn[i];
+      }
+    }
+  }
+  for (; g < ng; g += 8) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t t = 4 * (g + i);
       const uint32_t w = vw[i];
       vw[i] = vload(t + 32);
       if (g + i < ng) {
-        const float pv = pcol[t * ST];
-        const f32x16_t x0 = __builtin_amdgcn_mfma_f32_16x16x1f32(pv, bf16lo(w), zero16, 0, 0, 0);
-        const f32x16_t x1 = __builtin_amdgcn_mfma_f32_16x16x1f32(pv, bf16hi(w), zero16, 0, 0, 0);
-        if (g + i < nfull) {
+        const Products pr = products(pcol[t * ST], w);
 #pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
+        for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              s0[u] = s0[u] + x0[4 * kk + u];
-              s1[u] = s1[u] + x1[4 * kk + u];
-            }
-          }
-        } else {
+          for (int u = 0; u < 4; ++u) {
+            const bool in = t + kk < glen[u];
 #pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const bool in = t + kk < glen[u];
-              s0[u] = in ? s0[u] + x0[4 * kk + u] : s0[u];
-              s1[u] = in ? s1[u] + x1[4 * kk + u] : s1[u];
-            }
+            for (int x = 0; x < NX; ++x) sum[x][u] = in ? sum[x][u] + pr.x[x][4 * kk + u] : sum[x][u];
           }
         }
       }
@@ -555,11 +625,18 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
   for (int u = 0; u < 4; ++u) {
     const uint32_t qi = 4 * kq + u;
     if (qi >= nq) continue;
-    const uint64_t off = (((uint64_t)b * Tq + t0 + qi) * H + h) * D + 32 * (uint32_t)wave + 2 * jp;
-    if (OUT_BF16)
-      *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(o) + off) = pack_bf16x2(s0[u], s1[u]);
-    else
-      *reinterpret_cast<float2*>(static_cast<float*>(o) + off) = make_float2(s0[u], s1[u]);
+    const uint64_t off = (((uint64_t)b * Tq + t0 + qi) * H + h) * D + 32 * cw + 2 * jp + (NW == 8 ? (uint32_t)wave >> 2 : 0u);
+    if constexpr (NX == 2) {
+      if (OUT_BF16)
+        *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(o) + off) = pack_bf16x2(sum[0][u], sum[1][u]);
+      else
+        *reinterpret_cast<float2*>(static_cast<float*>(o) + off) = make_float2(sum[0][u], sum[1][u]);
+    } else {
+      if (OUT_BF16)
+        static_cast<uint16_t*>(o)[off] = (uint16_t)f32_to_bf16_bits(sum[0][u]);
+      else
+        static_cast<float*>(o)[off] = sum[0][u];
+    }
   }
 }
 
@@ -567,19 +644,19 @@ CATENA_DEV void prefill_body(const uint16_t* __restrict__ q, const uint16_t* __r
 // results in ordinary VGPRs, no AGPR copies before the VALU adds; one value
 // spilled to 8 bytes of scratch), so four workgroups share a CU when the
 // score buffer allows (up to 512 rows): C5 prefill 256 -> 234 us.
-// grid = B * H * ceil(Tq / 16), block = 256, dynamic LDS =
-// 16*136*2 + 3*16*4 + 3*4*16*4 + R*17*4 with R >= min(max lens, L) rounded up
-// to a multiple of 64 (the score rows of whole 64-key blocks).
-extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void catena_attn_prefill_bf16_d128_f32out(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const uint32_t* __restrict__ lens, float* __restrict__ o, uint32_t B, uint32_t H, uint32_t L,
-    uint32_t Tq, float scale) {
-  prefill_body<false>(q, k, v, lens, o, B, H, L, Tq, scale);
-}
-
-extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void catena_attn_prefill_bf16_d128_bf16out(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const uint32_t* __restrict__ lens, uint16_t* __restrict__ o, uint32_t B, uint32_t H, uint32_t L,
-    uint32_t Tq, float scale) {
-  prefill_body<true>(q, k, v, lens, o, B, H, L, Tq, scale);
-}
+// grid = B * H * nqb, block = 64 NW, dynamic LDS = 16*136*2 + 3*16*4 +
+// 3*NW*16*4 + R*17*4 with R >= the longest prefix of query blocks qb0 .. qb0
+// + nqb - 1, rounded up to a multiple of 64 (the score rows of whole 64-key
+// blocks).
+#define CATENA_PREFILL_KERNEL(NAME, OUTB, OT, NW, EU)                                                          \
+  extern "C" __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(EU))) void NAME(       \
+      const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,        \
+      const uint32_t* __restrict__ lens, OT* __restrict__ o, uint32_t B, uint32_t H, uint32_t L,             \
+      uint32_t Tq, float scale, uint32_t qb0, uint32_t nqb) {                                                \
+    prefill_body<OUTB, NW>(q, k, v, lens, o, B, H, L, Tq, scale, qb0, nqb);                                  \
+  }
+CATENA_PREFILL_KERNEL(catena_attn_prefill_bf16_d128_f32out, false, float, 4, 4)
+CATENA_PREFILL_KERNEL(catena_attn_prefill_bf16_d128_bf16out, true, uint16_t, 4, 4)
+// Eight waves, for score buffers that leave room for one workgroup per CU
+CATENA_PREFILL_KERNEL(catena_attn_prefill_w8_bf16_d128_f32out, false, float, 8, 4)
+CATENA_PREFILL_KERNEL(catena_attn_prefill_w8_bf16_d128_bf16out, true, uint16_t, 8, 4)
