@@ -525,21 +525,39 @@ int catena_mi355x_gemm_f32_exact(const float* a, const float* b, float* c, uint6
   if (n == 0 || m == 0) return CATENA_OK;
   if (!c || (k > 0 && (!a || !b))) return fail(CATENA_ERR_INVALID_ARGUMENT, "null operand");
   void* args[] = {&a, &b, &c, &n, &m, &k};
-  // 64x64 tiles (16 cells per thread) unless they would leave CUs idle; then
-  // 16x16 tiles with one cell per thread: A by DPP row broadcast and B through
-  // LDS when k % 16 == 0, B's rows are 16-byte aligned and the buffer offsets
-  // fit 31 bits, else A and B both through LDS.  Every cell is the same
-  // k-ascending chain in all three, so the choice never changes the bits.
+  // Every cell is the same k-ascending chain in every form, so the choice
+  // never changes the bits.
   const uint64_t gx = ceil_div(m, 64), gy = ceil_div(n, 64);
-  if (gx * gy < kDecodeSpread) {
-    const uint64_t sx = ceil_div(m, 16), sy = ceil_div(n, 16);
-    if (k > 0 && k % 16 == 0 && m % 4 == 0 && aligned16(b) && reinterpret_cast<uintptr_t>(a) % 4 == 0 &&
-        (n + 16) * k * 4 < (1ull << 31) && (k + 256) * m * 4 < (1ull << 31) && sy <= 65535)
-      return launch(KernelId::GemmF32ExactQ16, dim3((unsigned)sx, (unsigned)sy), dim3(256), 256 * 16 * 4, args);
-    return launch(KernelId::GemmF32ExactT16, dim3((unsigned)sx, (unsigned)sy), dim3(256), 0, args);
+  if (gx * gy >= kDecodeSpread && (gx > 0x7FFFFFFFu || gy > 65535u))
+    return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
+  const uint64_t t16 = ceil_div(m, 16) * ceil_div(n, 16);
+  const bool words = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 3u) == 0;
+  // One cell per thread on 16 x 16 tiles: A by DPP row broadcast and B through
+  // LDS (k % 16 == 0, 16-byte rows of B, 31-bit buffer offsets) up to four
+  // tiles for each CU (512^3: 13.0 us against 13.9), else A and B both through
+  // LDS while each CU gets one tile (255^3: 6.9 us against 8.6; 300 x 300 x 301,
+  // 361 tiles: 10.2 against 9.5) or operands are not word-aligned or too wide
+  // for the offsets below.
+  if (t16 <= 4 * kDecodeSpread && k > 0 && k % 16 == 0 && m % 4 == 0 && aligned16(b) && words &&
+      (n + 16) * k * 4 < (1ull << 31) && (k + 256) * m * 4 < (1ull << 31) && ceil_div(n, 16) <= 65535)
+    return launch(KernelId::GemmF32ExactQ16, dim3((unsigned)ceil_div(m, 16), (unsigned)ceil_div(n, 16)), dim3(256),
+                  256 * 16 * 4, args);
+  if (t16 <= kDecodeSpread || !words || k >= (1ull << 26) || m >= (1ull << 25)) {
+    if (t16 > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
+    return launch(KernelId::GemmF32ExactT16, dim3((unsigned)t16), dim3(256), 0, args);
   }
-  if (gx > 0x7FFFFFFFu || gy > 65535u) return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
-  return launch(KernelId::GemmF32Exact, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, args);
+  // Rows and columns per lane: 8 x 2 from 700 workgroups on (2.7 waves per
+  // SIMD: 1800 x 1700 x 1500, 798 of them, 233 us against 243 with 4 x 1; 1500^3,
+  // 564, 197 against 172), 4 x 1 from 600 on (300 x 2000 x 500, 608: 21.6 us
+  // against 26.9 with 2 x 1; 1024 x 512 x 1024, 512: 48 against 42), else 2 x 1.
+  const uint64_t g82 = ceil_div(m, 128) * ceil_div(n, 32), g41 = gx * ceil_div(n, 16), g21 = gx * ceil_div(n, 8);
+  const KernelId id = g82 >= 700 ? KernelId::GemmF32Exact8x2 : g41 >= 600 ? KernelId::GemmF32Exact4x1
+                                                                          : KernelId::GemmF32Exact2x1;
+  const uint64_t grid = id == KernelId::GemmF32Exact8x2 ? g82 : id == KernelId::GemmF32Exact4x1 ? g41 : g21;
+  if (grid > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
+  uint32_t m32 = (uint32_t)m, k32 = (uint32_t)k;
+  void* rargs[] = {&a, &b, &c, &n, &m32, &k32};
+  return launch(id, dim3((unsigned)grid), dim3(256), 0, rargs);
 }
 
 int catena_mi355x_gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_t m,

@@ -7,90 +7,203 @@
 //     acc = +0.0f; for kk = 0 .. k-1 ascending: acc = acc + A[i,kk] * B[kk,j]
 // with the multiply and the add separately rounded.  The reference runs one
 // thread per cell that streams a row of A and a column of B from global
-// memory.  Here a 64x64 output tile is staged through LDS 16 k-values at a
-// time and every thread owns a 4x4 block of cells; each cell keeps its own
-// k-ascending chain of v_mul_f32 then v_add_f32, so the result is bitwise the
-// reference's.  No split-K, no atomics.
+// memory.  Here each cell keeps its own k-ascending chain of v_mul_f32 then
+// v_add_f32 in one lane, so the result is bitwise the reference's.  No split-K,
+// no atomics.
+//
+// Large outputs: a wave owns ROWS consecutive rows and 64 COLS consecutive
+// columns, a lane all rows of its COLS columns.  A row of A is then uniform
+// across the wave: its next KB values are scalar loads, and each multiply takes
+// its A value as the scalar operand, with no LDS, no broadcast and no vector
+// register; a lane's own B values come straight from memory (256 contiguous
+// bytes per row and wave), KB rows ahead of their use.  No barrier, no alignment
+// beyond 4 bytes, any size: rows past n repeat the last row and are not stored,
+// k % KB values are folded one at a time.
+// What bounds it: VALU issue.  A SIMD issues such a multiply or add every 2.4
+// cycles with eight waves and every 2.9 with four (measured: 66 and 55 T lane
+// operations per second on the chip), so the rows and columns of a wave are as
+// many as leave each SIMD about four waves (host); the scalar loads cost a
+// request per row, hence 8 or 16 values each.  Waves run ahead in the order of
+// their age and the last ones would finish alone: priority falls with progress
+// (404 -> 347 us at 2048^3 on one box).
+// Measured on one box against 64 x 64 tiles staged through LDS (4 x 4 cells per
+// thread, eight LDS reads per 16 multiply-adds): 2048^3 535 -> 347 us (49.5 T
+// operations/s), 1000 x 1531 x 771 172 -> 59, 1000^3 230 -> 53, 500 x 500 x 501
+// 24 -> 14 (one cell per thread before).  Tried: A by DPP row broadcast (a DPP
+// multiply issues at less than half rate: 480 us), products on the f32 matrix
+// instructions (they occupy the VALU: 32 cycles for 16 adds' worth of products),
+// scalar loads a batch ahead (more requests: 459 us with 4 rows).
 #include "common.h"
 
 namespace {
-constexpr int TM = 64, TN = 64, TK = 16;
+typedef const __attribute__((address_space(4))) char scalar_bytes;
+typedef const __attribute__((address_space(4))) float scalar_float;
+typedef float f32x8_t __attribute__((ext_vector_type(8)));
+
+// The next values of rows p, p + stride, ... (at most p + last: rows past the
+// end repeat the last one), waited for in the same block: scalar loads return
+// out of order, so nothing is gained by leaving some in flight.
+CATENA_DEV void rows_of_a(f32x8_t (&a)[8], scalar_bytes* p, uint32_t stride, uint32_t last) {
+  uint32_t o;
+  asm volatile(
+      "s_load_dwordx8 %0, %9, 0x0\n\ts_min_u32 %8, %10, %11\n\t"
+      "s_load_dwordx8 %1, %9, %8 offset:0\n\ts_add_u32 %8, %8, %10\n\ts_min_u32 %8, %8, %11\n\t"
+      "s_load_dwordx8 %2, %9, %8 offset:0\n\ts_add_u32 %8, %8, %10\n\ts_min_u32 %8, %8, %11\n\t"
+      "s_load_dwordx8 %3, %9, %8 offset:0\n\ts_add_u32 %8, %8, %10\n\ts_min_u32 %8, %8, %11\n\t"
+      "s_load_dwordx8 %4, %9, %8 offset:0\n\ts_add_u32 %8, %8, %10\n\ts_min_u32 %8, %8, %11\n\t"
+      "s_load_dwordx8 %5, %9, %8 offset:0\n\ts_add_u32 %8, %8, %10\n\ts_min_u32 %8, %8, %11\n\t"
+      "s_load_dwordx8 %6, %9, %8 offset:0\n\ts_add_u32 %8, %8, %10\n\ts_min_u32 %8, %8, %11\n\t"
+      "s_load_dwordx8 %7, %9, %8 offset:0\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(a[0]), "=&s"(a[1]), "=&s"(a[2]), "=&s"(a[3]), "=&s"(a[4]), "=&s"(a[5]), "=&s"(a[6]), "=&s"(a[7]),
+        "=&s"(o)
+      : "s"(p), "s"(stride), "s"(last)
+      : "scc");
+}
+CATENA_DEV void rows_of_a(f32x16_t (&a)[4], scalar_bytes* p, uint32_t stride, uint32_t last) {
+  uint32_t o;
+  asm volatile(
+      "s_load_dwordx16 %0, %5, 0x0\n\ts_min_u32 %4, %6, %7\n\t"
+      "s_load_dwordx16 %1, %5, %4 offset:0\n\ts_add_u32 %4, %4, %6\n\ts_min_u32 %4, %4, %7\n\t"
+      "s_load_dwordx16 %2, %5, %4 offset:0\n\ts_add_u32 %4, %4, %6\n\ts_min_u32 %4, %4, %7\n\t"
+      "s_load_dwordx16 %3, %5, %4 offset:0\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(a[0]), "=&s"(a[1]), "=&s"(a[2]), "=&s"(a[3]), "=&s"(o)
+      : "s"(p), "s"(stride), "s"(last)
+      : "scc");
+}
+CATENA_DEV void rows_of_a(f32x16_t (&a)[2], scalar_bytes* p, uint32_t stride, uint32_t last) {
+  uint32_t o;
+  asm volatile(
+      "s_load_dwordx16 %0, %3, 0x0\n\ts_min_u32 %2, %4, %5\n\t"
+      "s_load_dwordx16 %1, %3, %2 offset:0\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(a[0]), "=&s"(a[1]), "=&s"(o)
+      : "s"(p), "s"(stride), "s"(last)
+      : "scc");
 }
 
-extern "C" __global__ __launch_bounds__(256) void catena_gemm_f32_exact(
-    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
-    uint64_t n, uint64_t m, uint64_t k) {
-  __shared__ float As[TK][TM + 1];
-  __shared__ float Bs[TK][TN];
+// The workgroup's 4 waves stack their rows over the same columns.  32-bit
+// offsets: (ROWS - 1) k and KB m floats stay below 2^31 bytes (host).
+template <int ROWS, int COLS, int KB>
+CATENA_DEV void rows_body(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
+                          uint64_t n, uint32_t m, uint32_t k) {
+  typedef float a_t __attribute__((ext_vector_type(KB)));
+  typedef float b_t __attribute__((ext_vector_type(COLS)));
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t gx = (m + 64 * COLS - 1) / (64 * COLS);
+  const uint64_t row0 = ((uint64_t)(blockIdx.x / gx) * 4 + wave) * ROWS;
+  if (row0 >= n) return;
+  const uint32_t col0 = (blockIdx.x % gx * 64 + lane) * COLS;
+  const uint32_t rowb = m * 4;
+  const uint32_t bvo = (col0 < m ? col0 : m - 1) * 4;
+  scalar_bytes* ap = (scalar_bytes*)(A + row0 * k);
+  const uint32_t stride = k * 4;
+  const uint32_t last = (n - 1 - row0 < (uint64_t)(ROWS - 1) ? (uint32_t)(n - 1 - row0) : ROWS - 1) * stride;
+  float acc[ROWS][COLS];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) acc[r][c] = __uint_as_float(0u);
 
-  const int tid = threadIdx.x;
-  const int tx = tid % 16;  // column group: cols tx + 16*jj
-  const int ty = tid / 16;  // row group: rows ty + 16*ii
-  const uint64_t row0 = (uint64_t)blockIdx.y * TM;
-  const uint64_t col0 = (uint64_t)blockIdx.x * TN;
-
-  float acc[4][4];
+  // B rows k0 .. k0 + KB - 1 of this lane's columns (zeros, untouched memory,
+  // when not live; a second column past m reads the next row's first value,
+  // and zero past the last row's end, and is not stored)
+  auto rows_of_b = [&](b_t (&b)[KB], uint32_t k0, bool live) {
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(B + (uint64_t)k0 * m), (short)0, live ? (int)(KB * rowb) : 0, 0x00020000);
 #pragma unroll
-  for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) acc[ii][jj] = __uint_as_float(0u);
-
-  for (uint64_t k0 = 0; k0 < k; k0 += TK) {
-    const int kt = (k - k0) < (uint64_t)TK ? (int)(k - k0) : TK;
-    // A tile: 64 rows x 16 k (row-major in A) -> As[kk][row]
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      int idx = tid + 256 * e;  // 0..1023
-      int r = idx / TK, kk = idx % TK;
-      uint64_t gi = row0 + r;
-      float v = 0.0f;
-      if (gi < n && kk < kt) v = A[gi * k + k0 + kk];
-      As[kk][r] = v;
+    for (int u = 0; u < KB; ++u) {
+      const int o = (int)(bvo + u * rowb);
+      if constexpr (COLS == 1)
+        b[u] = b_t{__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0))};
+      else
+        b[u] = __builtin_bit_cast(b_t, __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 0));
     }
-    // B tile: 16 k x 64 cols -> Bs[kk][col]
+  };
+  const uint32_t km = k / KB * KB;
+  uint32_t kk = 0;
+  if (km > 0) {
+    b_t b[KB];
+    rows_of_b(b, 0, true);
+    auto fold_to = [&](uint32_t kend) {
+      for (; kk < kend; kk += KB) {
+        b_t bn[KB];
+        const bool more = kk + KB < km;
+        rows_of_b(bn, more ? kk + KB : kk, more);
+        a_t a[ROWS];
+        __builtin_amdgcn_sched_barrier(0);
+        rows_of_a(a, ap, stride, last);
+        ap += 4 * KB;
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      int idx = tid + 256 * e;
-      int kk = idx / TN, c = idx % TN;
-      uint64_t gj = col0 + c;
-      float v = 0.0f;
-      if (gj < m && kk < kt) v = B[(k0 + kk) * m + gj];
-      Bs[kk][c] = v;
-    }
-    __syncthreads();
-    // Only the kt live k-values are folded: the chain sees exactly
-    // k = 0 .. k-1 in ascending order.
-    for (int kk = 0; kk < kt; ++kk) {
-      float a[4], b[4];
+        for (int u = 0; u < KB; ++u)
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) a[ii] = As[kk][ty + 16 * ii];
+          for (int c = 0; c < COLS; ++c) {
+            float prod[ROWS];
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) b[jj] = Bs[kk][tx + 16 * jj];
+            for (int r = 0; r < ROWS; ++r) prod[r] = a[r][u] * b[u][c];
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii)
+            for (int r = 0; r < ROWS; ++r) acc[r][c] = acc[r][c] + prod[r];
+          }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          float prod = a[ii] * b[jj];
-          acc[ii][jj] = acc[ii][jj] + prod;
-        }
-    }
-    __syncthreads();
+        for (int u = 0; u < KB; ++u) b[u] = bn[u];
+      }
+    };
+    const uint32_t quarter = km / (4 * KB) * KB;
+    __builtin_amdgcn_s_setprio(3);
+    fold_to(quarter);
+    __builtin_amdgcn_s_setprio(2);
+    fold_to(2 * quarter);
+    __builtin_amdgcn_s_setprio(1);
+    fold_to(3 * quarter);
+    __builtin_amdgcn_s_setprio(0);
+    fold_to(km);
   }
-
+  for (; kk < k; ++kk) {
+    float b[COLS];
 #pragma unroll
-  for (int ii = 0; ii < 4; ++ii) {
-    uint64_t gi = row0 + ty + 16 * ii;
-    if (gi >= n) continue;
+    for (int c = 0; c < COLS; ++c) b[c] = B[(uint64_t)kk * m + (col0 + c < m ? col0 + c : m - 1)];
+    uint32_t o = 0;
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      uint64_t gj = col0 + tx + 16 * jj;
-      if (gj < m) C[gi * m + gj] = acc[ii][jj];
+    for (int r = 0; r < ROWS; ++r) {
+      const float av = *(scalar_float*)(ap + o);
+      o = o + stride < last ? o + stride : last;
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) {
+        const float prod = av * b[c];
+        acc[r][c] = acc[r][c] + prod;
+      }
     }
+    ap += 4;
+  }
+  // (opaque here, so that the stores' tests do not take registers in the loop)
+  uint32_t rows = n - row0 < (uint64_t)ROWS ? (uint32_t)(n - row0) : ROWS, cols = m;
+  asm volatile("" : "+s"(rows), "+s"(cols));
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    if ((uint32_t)r >= rows) continue;
+#pragma unroll
+    for (int c = 0; c < COLS; ++c)
+      if (col0 + c < cols) C[(row0 + r) * cols + col0 + c] = acc[r][c];
   }
 }
+}  // namespace
 
-// The same contraction for small outputs, where 64x64 tiles would leave most
-// CUs idle (256^3 is 16 tiles of 64x64 on a 256-CU device): a 16x16 output
+// grid = ceil(m / (64 COLS)) * ceil(n / (4 ROWS)), block = 256.  (The register
+// budget is set for four waves per SIMD so that all scalar registers can be
+// used; the vector registers leave room for eight.)
+#define CATENA_GEMM_F32_ROWS(NAME, ROWS, COLS, KB)                                                        \
+  extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void NAME(         \
+      const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, uint64_t n,        \
+      uint32_t m, uint32_t k) {                                                                           \
+    rows_body<ROWS, COLS, KB>(A, B, C, n, m, k);                                                          \
+  }
+CATENA_GEMM_F32_ROWS(catena_gemm_f32_exact_8x2, 8, 2, 8)
+CATENA_GEMM_F32_ROWS(catena_gemm_f32_exact_4x1, 4, 1, 16)
+CATENA_GEMM_F32_ROWS(catena_gemm_f32_exact_2x1, 2, 1, 16)
+
+// The same contraction for small outputs, where whole waves of columns would
+// leave most CUs idle (256^3 is 128 workgroups of the smallest form above): a 16x16 output
 // tile per workgroup of 256 threads, one cell per thread, so 256^3 launches
 // 256 workgroups.  A 16-row x 128-k slab of A and a 128-k x 16-column slab of
 // B are staged in LDS k-contiguous per row / per column ([row][k] and
@@ -102,7 +215,7 @@ extern "C" __global__ __launch_bounds__(256) void catena_gemm_f32_exact(
 // requested into registers before the current one is folded.  The cell's
 // chain is the one above: acc = +0, then for kk ascending
 // acc = acc + fl(A[i,kk] * B[kk,j]), separately rounded -- bitwise the same
-// result as the 64x64 instance and the reference.
+// result as the forms above and the reference.
 namespace {
 constexpr int S_T = 16, S_K = 128, S_PAD = 4;
 
@@ -178,8 +291,9 @@ extern "C" __global__ __launch_bounds__(256) void catena_gemm_f32_exact_t16(
   const int tid = threadIdx.x;
   const int tx = tid % S_T;  // column of the cell
   const int ty = tid / S_T;  // row of the cell
-  const uint64_t row0 = (uint64_t)blockIdx.y * S_T;
-  const uint64_t col0 = (uint64_t)blockIdx.x * S_T;
+  const uint32_t gx = (uint32_t)((m + S_T - 1) / S_T);
+  const uint64_t row0 = (uint64_t)(blockIdx.x / gx) * S_T;
+  const uint64_t col0 = (uint64_t)(blockIdx.x % gx) * S_T;
 
   float acc = __uint_as_float(0u);
   Slab sl;

@@ -1,0 +1,59 @@
+"""The exact-order f32 GEMM's row forms (A by scalar loads) at the sizes where
+they and the 16 x 16 tiles change over, bitwise against the oracle's ascending
+chain, with operands at any 4-byte address between NaNs."""
+import numpy as np
+import pytest
+
+import catena_amd as ca
+import oracle
+from gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+SPECIALS = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-20, -1e-20, 3e-39, 1.0, -2.5], np.float32)
+
+
+def _placed(a, shift_bytes):
+    raw = np.full(a.nbytes + 1024, 0xFF, np.uint8)  # all-ones words are NaNs
+    raw[256 + shift_bytes:256 + shift_bytes + a.nbytes] = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+    buf = ca.Buffer.from_array(raw)
+    return buf, buf.ptr + 256 + shift_bytes
+
+
+def _check(n, m, k, shift=0, special=False):
+    rng = np.random.default_rng(n + 3 * m + 7 * k + shift)
+    a = rng.uniform(-1, 1, (n, k)).astype(np.float32)
+    b = rng.uniform(-1, 1, (k, m)).astype(np.float32)
+    if special:
+        for x in (a, b):
+            hit = rng.random(x.shape) < 0.01
+            x[hit] = rng.choice(SPECIALS, int(hit.sum()))
+        b[:, :3] *= np.float32(1e-19)
+    say(f"gemm f32 exact rows {n}x{m}x{k} shift {shift} special {special}")
+    (ab, ap), (bb, bp) = _placed(a, shift), _placed(b, shift)
+    fill = 0xA5
+    cb = ca.Buffer.from_array(np.full(n * m * 4 + 512, fill, np.uint8))
+    ca.gemm_f32_exact(ap, bp, cb.ptr + 256, n, m, k)
+    raw = cb.read(np.uint8)
+    assert np.all(raw[:256] == fill) and np.all(raw[-256:] == fill)
+    got, want = raw[256:-256].copy().view(np.float32).reshape(n, m), oracle.matmul_f32(a, b)
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
+# 2 x 1: more than 256 tiles of 16 x 16 and fewer than 600 workgroups of 4 x 1;
+# 4 x 1; 8 x 2 from 700 workgroups on; one row or column past a wave's
+@pytest.mark.parametrize("n,m,k", [
+    (257, 257, 1), (272, 257, 7), (273, 259, 16), (300, 301, 17), (1000, 70, 33), (70, 1000, 47), (5, 20000, 31),
+    (385, 1537, 15), (400, 1600, 16), (401, 1601, 48), (9600, 63, 19), (9601, 65, 16),
+    (1089, 2561, 8), (1120, 2560, 9), (33, 90000, 7), (1121, 2562, 24),
+    (512, 512, 16), (512, 516, 16), (516, 512, 32)])
+def test_row_forms(n, m, k):
+    _check(n, m, k)
+
+
+@pytest.mark.parametrize("n,m,k", [(300, 301, 50), (401, 1601, 37), (1089, 2561, 21)])
+@pytest.mark.parametrize("shift,special", [(4, False), (12, True), (0, True), (2, False)])
+def test_addresses_and_special_values(n, m, k, shift, special):
+    _check(n, m, k, shift, special)
