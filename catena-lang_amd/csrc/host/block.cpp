@@ -45,9 +45,20 @@ int rmsnorm_launch(const float* x, const float* resid, const uint32_t* row_index
                 (unsigned long long)n, rmsnorm_lds_bytes(n));
   if (resid_parts == 0 || (resid_parts > 1 && (!resid || (n % 4 == 0 && resid_stride % 4 != 0))))
     return fail(CATENA_ERR_INVALID_ARGUMENT, "rmsnorm residual partials");
-  uint32_t n32 = (uint32_t)n;
-  void* args[] = {&x,      &resid, &row_index, &h_out,       &y_f32,       &y_bf16,   &n32,
-                  &tokens, &table, &vocab,     &resid_parts, &resid_stride, &resid_out};
+  uint32_t n32 = (uint32_t)n, rows32 = (uint32_t)rows;
+  // Four rows to a workgroup (their folds then cost the VALU a quarter) once
+  // there are more rows than one round of one-row workgroups takes, and two of
+  // the larger ones fit a CU.  Measured, one against four: 2048 x 2048 14.1 / 14.9
+  // us, 4096 x 2048 25.8 / 19.1, 32001 x 2048 148 / 111, 16384 x 512 28.7 / 19.7,
+  // 1536 x 4096 28.8 / 23.1, 8192 x 6000 219 / 246.
+  const uint64_t round = (uint64_t)device().cu_count * std::min<uint64_t>(8, device().max_lds / rmsnorm_lds_bytes(n));
+  uint32_t slot = rows > round ? rows4_slot(n) : 0;
+  if (slot && rows4_per_cu(slot) < 2) slot = 0;
+  void* args[] = {&x,     &resid, &row_index,   &h_out,        &y_f32,     &y_bf16, &n32, &tokens,
+                  &table, &vocab, &resid_parts, &resid_stride, &resid_out, &rows32, &slot};
+  if (slot)
+    return launch(KernelId::RmsnormRows4, dim3((unsigned)ceil_div(rows, 4)), dim3(256),
+                  4 * (size_t)slot * sizeof(float), args);
   return launch(KernelId::RmsnormRows, dim3((unsigned)rows), dim3(256), lds, args);
 }
 }  // namespace

@@ -103,6 +103,7 @@ const KernelSpec kKernels[] = {
     {KernelId::AttnPrefillW8D128Bf16, "attn_prefill", "catena_attn_prefill_w8_bf16_d128_bf16out"},
     {KernelId::EmbedRowsBf16, "block", "catena_embed_rows_bf16"},
     {KernelId::RmsnormRows, "block", "catena_rmsnorm_rows"},
+    {KernelId::RmsnormRows4, "block", "catena_rmsnorm_rows4"},
     {KernelId::RopeQkvStore, "block", "catena_rope_qkv_store"},
     {KernelId::RopeTable, "block", "catena_rope_table"},
     {KernelId::SiluMulBf16, "block", "catena_silu_mul_bf16"},
@@ -111,9 +112,15 @@ const KernelSpec kKernels[] = {
     {KernelId::ArangeF32, "tensor", "catena_arange_f32"},
     {KernelId::CopyF32, "tensor", "catena_copy_f32"},
     {KernelId::SumRowsF32, "tensor", "catena_sum_rows_f32"},
+    {KernelId::SumRows4VecF32, "tensor", "catena_sum_rows4_vec_f32"},
+    {KernelId::SumRows4F32, "tensor", "catena_sum_rows4_f32"},
     {KernelId::MaxRowsF32, "tensor", "catena_max_rows_f32"},
     {KernelId::SumRowsU64, "tensor", "catena_sum_rows_u64"},
     {KernelId::SoftmaxRows, "softmax", "catena_softmax_rows_f32"},
+    {KernelId::SoftmaxRowVec, "softmax", "catena_softmax_row_vec_f32"},
+    {KernelId::SoftmaxRow, "softmax", "catena_softmax_row_f32"},
+    {KernelId::SoftmaxRows4Vec, "softmax", "catena_softmax_rows4_vec_f32"},
+    {KernelId::SoftmaxRows4, "softmax", "catena_softmax_rows4_f32"},
     {KernelId::ExpApprox, "softmax", "catena_exp_approx_f32"},
     {KernelId::MapF32, "softmax", "catena_map_f32"},
     {KernelId::FillNormalBf16, "fill", "catena_fill_normal_bf16"},

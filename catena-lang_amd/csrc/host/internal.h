@@ -65,6 +65,7 @@ enum class KernelId : int {
   AttnPrefillW8D128Bf16,
   EmbedRowsBf16,
   RmsnormRows,
+  RmsnormRows4,  // four rows a workgroup
   RopeQkvStore,
   RopeTable,
   SiluMulBf16,
@@ -73,9 +74,15 @@ enum class KernelId : int {
   ArangeF32,
   CopyF32,
   SumRowsF32,
+  SumRows4VecF32,  // four rows a workgroup, in LDS (tensor.hip)
+  SumRows4F32,
   MaxRowsF32,
   SumRowsU64,
   SoftmaxRows,
+  SoftmaxRowVec,  // rows in LDS (softmax.hip): one row a workgroup
+  SoftmaxRow,
+  SoftmaxRows4Vec,  // four rows a workgroup
+  SoftmaxRows4,
   ExpApprox,
   MapF32,
   FillNormalBf16,
@@ -179,6 +186,18 @@ inline size_t rmsnorm_lds_bytes(uint64_t n) {
 }
 
 Device& device();
+
+// LDS slot, in floats, of a row in a four-row workgroup (pad32 of common.h: 36
+// floats for 32 values, rows rounded up to 4 values); 0 when four such rows do
+// not fit (n over about 9,088)
+inline uint32_t rows4_slot(uint64_t n) {
+  const uint64_t n4 = (n + 3) / 4 * 4, slot = n4 + n4 / 32 * 4 + 4;
+  return n4 <= 16384 && 4 * slot * sizeof(float) + 64 <= device().max_lds ? (uint32_t)slot : 0;
+}
+// such workgroups that one CU's LDS holds
+inline uint32_t rows4_per_cu(uint32_t slot) {
+  return (uint32_t)(device().max_lds / (4 * (size_t)slot * sizeof(float) + 64));
+}
 int ensure_init();
 int fail(int status, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 void clear_error();

@@ -663,6 +663,22 @@ int catena_mi355x_softmax_f32(const float* x, float* y, uint64_t rows, uint64_t 
   if (!x || !y) return fail(CATENA_ERR_INVALID_ARGUMENT, "null operand");
   if (n >= 0x7FFFFFFFull) return fail(CATENA_ERR_UNSUPPORTED, "softmax length too large");
   if (rows > 0x7FFFFFFFull) return fail(CATENA_ERR_UNSUPPORTED, "too many rows");
+  // Rows that fit LDS: one to a workgroup while the latency of a row is what
+  // counts, four once the folds' adds do (a wave's add advances four rows): from
+  // six rows a CU, where three such workgroups fit one.  Measured, one against
+  // four: 1024 x 2048 11.6 / 12.7 us, 2048 x 2048 21.0 / 18.7, 16384 x 512 36.1 /
+  // 24.2, 4096 x 4096 58.9 / 59.4, 8192 x 6000 173 / 302.  Longer rows: one row
+  // per workgroup through memory.
+  const bool vec = n % 4 == 0 && aligned16(x) && aligned16(y);
+  uint32_t n32 = (uint32_t)n, slot = rows4_slot(n);
+  void* lds_args[] = {&x, &y, &rows, &n32, &slot};
+  if (slot && rows4_per_cu(slot) >= 3 && rows >= 6ull * (unsigned)device().cu_count)
+    return launch(vec ? KernelId::SoftmaxRows4Vec : KernelId::SoftmaxRows4, dim3((unsigned)ceil_div(rows, 4)),
+                  dim3(256), 4 * (size_t)slot * sizeof(float), lds_args);
+  if (n <= (device().max_lds - 64) / sizeof(float)) {
+    return launch(vec ? KernelId::SoftmaxRowVec : KernelId::SoftmaxRow, dim3((unsigned)rows), dim3(256),
+                  ceil_div(n, 4) * 4 * sizeof(float), lds_args);
+  }
   void* args[] = {&x, &y, &n};
   return launch(KernelId::SoftmaxRows, dim3((unsigned)rows), dim3(256), 0, args);
 }

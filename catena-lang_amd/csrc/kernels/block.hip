@@ -87,11 +87,14 @@ extern "C" __global__ __launch_bounds__(256) void catena_embed_rows_bf16(
 // moved with 16-byte accesses when n % 4 == 0 (pointers 16-byte aligned),
 // element by element otherwise.
 namespace {
+template <int ROWS>
 CATENA_DEV void rms_finish_row(const float* hs, uint32_t n, uint64_t row, float rms,
                                float* __restrict__ y_f32, uint16_t* __restrict__ y_bf16) {
+  constexpr uint32_t T = 256 / ROWS;
+  const uint32_t t = threadIdx.x % T;
   if (n % 4 == 0) {
-    for (uint32_t i = threadIdx.x; i < n / 4; i += blockDim.x) {
-      const f32x4_t h = reinterpret_cast<const f32x4_t*>(hs)[i];
+    for (uint32_t i = t; i < n / 4; i += T) {
+      const f32x4_t h = *reinterpret_cast<const f32x4_t*>(hs + row_at<ROWS>(4 * i));
       f32x4_t y;
 #pragma unroll
       for (int j = 0; j < 4; ++j) y[j] = h[j] / rms;
@@ -104,14 +107,13 @@ CATENA_DEV void rms_finish_row(const float* hs, uint32_t n, uint64_t row, float 
       }
     }
   } else {
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-      const float y = hs[i] / rms;
+    for (uint32_t i = t; i < n; i += T) {
+      const float y = hs[row_at<ROWS>(i)] / rms;
       if (y_f32) y_f32[row * n + i] = y;
       if (y_bf16) y_bf16[row * n + i] = (uint16_t)f32_to_bf16_bits(y);
     }
   }
 }
-}  // namespace
 
 // With tokens given, the input row is the embedding gather
 // widen(table[tokens[src]]) (a token >= vocab gives NaN) instead of x[src];
@@ -121,37 +123,83 @@ CATENA_DEV void rms_finish_row(const float* hs, uint32_t n, uint64_t row, float 
 // (resid_parts > 1, part s at resid + s * resid_stride): resid[src] is then
 // ((P0 + P1) + ...) + P(parts-1), the adds that GEMM's own reduction makes.
 // resid[src] (the sum) is written to resid_out[src] when resid_out is given.
-extern "C" __global__ __launch_bounds__(256) void catena_rmsnorm_rows(
-    const float* __restrict__ x, const float* __restrict__ resid,
-    const uint32_t* __restrict__ row_index, float* __restrict__ h_out,
-    float* __restrict__ y_f32, uint16_t* __restrict__ y_bf16, uint32_t n,
-    const uint32_t* __restrict__ tokens, const uint16_t* __restrict__ table, uint32_t vocab,
-    uint32_t resid_parts, uint64_t resid_stride, float* __restrict__ resid_out) {
+// ROWS == 4: one wave per row, the four sums folded by wave 0.
+template <int ROWS>
+CATENA_DEV void rmsnorm_rows_body(const float* __restrict__ x, const float* __restrict__ resid,
+                                  const uint32_t* __restrict__ row_index, float* __restrict__ h_out,
+                                  float* __restrict__ y_f32, uint16_t* __restrict__ y_bf16, uint32_t n,
+                                  const uint32_t* __restrict__ tokens, const uint16_t* __restrict__ table,
+                                  uint32_t vocab, uint32_t resid_parts, uint64_t resid_stride,
+                                  float* __restrict__ resid_out, uint32_t rows, uint32_t slot) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr uint32_t T = 256 / ROWS;
+  const uint32_t wave = ROWS == 4 ? threadIdx.x / 64 : 0, tid = threadIdx.x % T;
   const uint32_t n_pad = (n + 3u) & ~3u;
-  float* hs = reinterpret_cast<float*>(smem);  // [n_pad]
-  float* sq = hs + n_pad;                      // [n_pad]
-  __shared__ float rms_s;
-  const uint32_t row = blockIdx.x;
-  const uint64_t src = row_index ? row_index[row] : row;
+  float* hs = reinterpret_cast<float*>(smem) + wave * slot;  // [n_pad] (ROWS == 4: padded)
+  float* sq = hs + n_pad;                                    // [n_pad], ROWS == 1 only
+  __shared__ float rms_s[ROWS];
+  const uint32_t row = blockIdx.x * ROWS + wave;
+  const bool live = ROWS == 1 || row < rows;
+  const uint64_t src = row_index && live ? row_index[row] : row;
   uint32_t tok = 0;
   bool tok_ok = true;
   const bool gather = tokens || (!x && table);
-  if (gather) {
+  if (gather && live) {
     tok = tokens ? tokens[src] : (uint32_t)src;
     tok_ok = tok < vocab;
   }
   const float nan = __uint_as_float(kNaNBits);
-  if (n % 4 == 0) {
+  if (live && n % 4 == 0) {
     const f32x4_t* x4 = reinterpret_cast<const f32x4_t*>(x + src * n);
     const f32x4_t* r4 = resid ? reinterpret_cast<const f32x4_t*>(resid + src * n) : nullptr;
     const uint2* e4 = gather ? reinterpret_cast<const uint2*>(table + (uint64_t)tok * n) : nullptr;
-    for (uint32_t i = threadIdx.x; i < n / 4; i += 256) {
+    auto put = [&](uint32_t i, const f32x4_t& h) {
+      *reinterpret_cast<f32x4_t*>(hs + row_at<ROWS>(4 * i)) = h;
+      if (ROWS == 1) {
+        f32x4_t s;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] = h[j] * h[j];
+        reinterpret_cast<f32x4_t*>(sq)[i] = s;
+      }
+      if (h_out) reinterpret_cast<f32x4_t*>(h_out + (uint64_t)row * n)[i] = h;
+    };
+    auto widen = [](const uint2& w) { return f32x4_t{bf16lo(w.x), bf16hi(w.x), bf16lo(w.y), bf16hi(w.y)}; };
+    uint32_t i = tid;
+    if (ROWS == 4) {
+      // one wave per row: four loads in flight per lane (eight of the table's)
+      if (!r4 && gather && tok_ok) {
+        for (; i + T * 7 < n / 4; i += T * 8) {
+          uint2 w[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) w[u] = e4[i + T * u];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) put(i + T * u, widen(w[u]));
+        }
+      } else if (!gather && (!r4 || resid_parts == 1)) {
+        for (; i + T * 3 < n / 4; i += T * 4) {
+          f32x4_t h[4], rr[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) h[u] = x4[i + T * u];
+          if (r4) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) rr[u] = r4[i + T * u];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              if (resid_out) reinterpret_cast<f32x4_t*>(resid_out + src * n)[i + T * u] = rr[u];
+#pragma unroll
+              for (int j = 0; j < 4; ++j) h[u][j] = h[u][j] + rr[u][j];
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) put(i + T * u, h[u]);
+        }
+      }
+    }
+    for (; i < n / 4; i += T) {
       f32x4_t h;
       if (gather) {
         if (tok_ok) {
-          const uint2 w = e4[i];
-          h = f32x4_t{bf16lo(w.x), bf16hi(w.x), bf16lo(w.y), bf16hi(w.y)};
+          h = widen(e4[i]);
         } else {
           h = f32x4_t{nan, nan, nan, nan};
         }
@@ -181,15 +229,12 @@ extern "C" __global__ __launch_bounds__(256) void catena_rmsnorm_rows(
 #pragma unroll
         for (int j = 0; j < 4; ++j) h[j] = h[j] + rr[j];
       }
-      f32x4_t s;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] = h[j] * h[j];
-      reinterpret_cast<f32x4_t*>(hs)[i] = h;
-      reinterpret_cast<f32x4_t*>(sq)[i] = s;
-      if (h_out) reinterpret_cast<f32x4_t*>(h_out + (uint64_t)row * n)[i] = h;
+      put(i, h);
     }
-  } else {
-    for (uint32_t i = threadIdx.x; i < n; i += 256) {
+  } else if (ROWS == 4 && live && !gather && !resid && !h_out) {
+    row_to_lds<4, false>(x + src * n, hs, n, [](float) {});
+  } else if (live) {
+    for (uint32_t i = tid; i < n; i += T) {
       float h;
       if (gather)
         h = tok_ok ? bf16_to_f32(table[(uint64_t)tok * n + i]) : nan;
@@ -201,25 +246,49 @@ extern "C" __global__ __launch_bounds__(256) void catena_rmsnorm_rows(
         if (resid_out) resid_out[src * n + i] = rr;
         h = h + rr;
       }
-      hs[i] = h;
-      sq[i] = h * h;
+      hs[row_at<ROWS>(i)] = h;
+      if (ROWS == 1) sq[i] = h * h;
       if (h_out) h_out[(uint64_t)row * n + i] = h;
     }
   }
+  // the slots past the row: the square of +0
+  if (ROWS == 4 && tid < n_pad - n) hs[row_at<ROWS>(n + tid)] = 0.0f;
   __syncthreads();
   if (threadIdx.x < 64) {
-    const float sum_sq = serial_sum_wave_long(sq, n);
-    if (threadIdx.x == 0) {
+    float sum_sq;
+    if constexpr (ROWS == 4)
+      sum_sq = serial_sum_rows4<true>(reinterpret_cast<float*>(smem) + (threadIdx.x / 16) * slot, n_pad);
+    else
+      sum_sq = serial_sum_wave_long(sq, n);
+    if (threadIdx.x % (64 / ROWS) == 0) {
       const float len_f = (float)(uint64_t)n;
       const float mean_sq = sum_sq / len_f;
       const float eps = u32_as_f32(0x3727C5ACu);
       const float t = mean_sq + eps;
-      rms_s = sqrt_newton(t);
+      rms_s[threadIdx.x / (64 / ROWS)] = sqrt_newton(t);
     }
   }
   __syncthreads();
-  rms_finish_row(hs, n, row, rms_s, y_f32, y_bf16);
+  if (live) rms_finish_row<ROWS>(hs, n, row, rms_s[wave], y_f32, y_bf16);
 }
+}  // namespace
+
+#define CATENA_RMSNORM_ROWS(name, ROWS)                                                                       \
+  extern "C" __global__ __launch_bounds__(256) void name(                                                     \
+      const float* __restrict__ x, const float* __restrict__ resid, const uint32_t* __restrict__ row_index,   \
+      float* __restrict__ h_out, float* __restrict__ y_f32, uint16_t* __restrict__ y_bf16, uint32_t n,        \
+      const uint32_t* __restrict__ tokens, const uint16_t* __restrict__ table, uint32_t vocab,                \
+      uint32_t resid_parts, uint64_t resid_stride, float* __restrict__ resid_out, uint32_t rows,              \
+      uint32_t slot) {                                                                                        \
+    rmsnorm_rows_body<ROWS>(x, resid, row_index, h_out, y_f32, y_bf16, n, tokens, table, vocab, resid_parts,  \
+                            resid_stride, resid_out, rows, slot);                                             \
+  }
+// grid = rows, dynamic LDS = 2 * round_up(n, 4) floats
+CATENA_RMSNORM_ROWS(catena_rmsnorm_rows, 1)
+// grid = ceil(rows / 4), dynamic LDS = 4 slots of `slot` floats (slot % 4 == 0, at
+// least pad32 of n rounded up to 4)
+CATENA_RMSNORM_ROWS(catena_rmsnorm_rows4, 4)
+#undef CATENA_RMSNORM_ROWS
 
 // RoPE on the q and k parts of a fused projection, bf16 q out, and the
 // KV-cache append.  qkv[R][3*H*D] f32 with R = B * Tq rows (row b*Tq + tq,

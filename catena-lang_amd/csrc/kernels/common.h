@@ -351,6 +351,120 @@ CATENA_DEV float serial_sum_wave_long(const float* s, uint32_t n) {
   return acc;
 }
 
+// Rows of a four-row workgroup in LDS: four floats of padding after every 32,
+// so that the 32-value blocks that a row's 16 lanes fold start 36 floats apart
+// and their 16-byte reads cover the banks once.
+CATENA_DEV uint32_t pad32(uint32_t i) { return i + (i >> 5) * 4u; }
+
+// The sequential fold of serial_sum_wave_long for four rows at once, one per
+// 16-lane DPP row (all 64 lanes call it with their own row's s, rows padded as
+// pad32 places them; every lane gets its row's sum): the wave holds 512 values
+// of each row, lane j values 32j .. 32j + 31, and step L adds a lane's values to
+// the sum its left neighbour in the row held after step L - 1 (row_shr:1).  One
+// v_add_f32 advances four rows, where the one-row form spends a wave's 64 lanes
+// on one of them; the next 512 values are read during the chain.  n % 4 == 0,
+// slots past a row's data hold +0; SQUARE folds the rounded squares.
+template <bool SQUARE>
+CATENA_DEV float serial_sum_rows4(const float* s, uint32_t n) {
+  const uint32_t j = threadIdx.x & 15u;
+  float acc = __uint_as_float(0u);
+  float v[32];
+  auto load = [&](float (&w)[32], uint32_t base) {
+    const uint32_t lo = base + 32 * j;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t e = lo + 4 * i;
+      const bool in = e < n;
+      const f32x4_t q = *reinterpret_cast<const f32x4_t*>(s + pad32(in ? e : 0u));
+#pragma unroll
+      for (int c = 0; c < 4; ++c) w[4 * i + c] = in ? (SQUARE ? q[c] * q[c] : q[c]) : __uint_as_float(0u);
+    }
+  };
+  if (n == 0) return acc;
+  load(v, 0);
+  for (uint32_t base = 0; base < n; base += 512) {
+    const uint32_t left = n - base;
+    const uint32_t nl = left >= 512u ? 16u : (left + 31u) / 32u;
+    float nx[32];
+    if (left > 512u) load(nx, base + 512);
+    __builtin_amdgcn_sched_barrier(0);
+    float a = acc;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) a = a + v[k];
+    auto block = [&]() {
+      // two wait states between the write of a and its DPP read, also across
+      // the loop's back edge
+      asm volatile("s_nop 1");
+      a = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xF, 0xF, true)) + v[0];
+#pragma unroll
+      for (int k = 1; k < 32; ++k) a = a + v[k];
+    };
+    uint32_t L = 1;
+#pragma unroll 1
+    for (; L + 5 <= nl; L += 5) {
+#pragma unroll
+      for (int r = 0; r < 5; ++r) block();
+    }
+#pragma unroll 1
+    for (; L < nl; ++L) block();
+    acc = __shfl(a, (int)((threadIdx.x & 48u) + nl - 1u), 64);
+#pragma unroll
+    for (int k = 0; k < 32; ++k) v[k] = nx[k];
+  }
+  return acc;
+}
+
+// ROWS rows share a workgroup of 256 threads, T = 256 / ROWS to a row: four in
+// pad32's layout (serial_sum_rows4), or one as it is (serial_sum_wave_long).
+template <int ROWS>
+CATENA_DEV uint32_t row_at(uint32_t i) {
+  return ROWS == 4 ? pad32(i) : i;
+}
+template <int ROWS, bool SQUARE>
+CATENA_DEV float rows_fold(const float* s, uint32_t slot, uint32_t n4) {
+  static_assert(ROWS == 4 || (ROWS == 1 && !SQUARE), "");
+  if constexpr (ROWS == 4) return serial_sum_rows4<SQUARE>(s + ((threadIdx.x & 63u) >> 4) * slot, n4);
+  return serial_sum_wave_long(s, n4);
+}
+
+// T threads move a row of n values from memory to its place in LDS, up to eight
+// loads in flight per lane, handing each value to see().  VEC: n % 4 == 0 and x
+// 16-byte aligned.
+template <int ROWS, bool VEC, class See>
+CATENA_DEV void row_to_lds(const float* x, float* s, uint32_t n, See see) {
+  constexpr uint32_t T = 256 / ROWS;
+  uint32_t i = threadIdx.x % T;
+  if (VEC) {
+    const f32x4_t* x4 = reinterpret_cast<const f32x4_t*>(x);
+    auto put = [&](uint32_t at, const f32x4_t& q) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) see(q[c]);
+      *reinterpret_cast<f32x4_t*>(s + row_at<ROWS>(4 * at)) = q;
+    };
+    for (; i + T * 7 < n / 4; i += T * 8) {
+      f32x4_t q[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) q[u] = x4[i + T * u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) put(i + T * u, q[u]);
+    }
+    for (; i < n / 4; i += T) put(i, x4[i]);
+  } else {
+    auto put = [&](uint32_t at, float q) {
+      see(q);
+      s[row_at<ROWS>(at)] = q;
+    };
+    for (; i + T * 7 < n; i += T * 8) {
+      float q[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) q[u] = x[i + T * u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) put(i + T * u, q[u]);
+    }
+    for (; i < n; i += T) put(i, x[i]);
+  }
+}
+
 // Cross-workgroup partial results.  The XCDs' L2 caches are not coherent
 // with each other, so partials that another workgroup will read are stored
 // and loaded as agent-scope atomics (relaxed): those bypass the non-coherent

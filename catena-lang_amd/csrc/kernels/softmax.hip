@@ -88,6 +88,128 @@ extern "C" __global__ __launch_bounds__(256) void catena_softmax_rows_f32(
   for (uint64_t t = tid; t < n; t += 256) yr[t] = yr[t] / den;
 }
 
+// The same for rows that fit LDS: a row is read once and written once and kept
+// in LDS between, one row to a workgroup, or (ROWS == 4) a wave to a row and
+// wave 0 folds the four denominators together (serial_sum_rows4).
+// The maximum: when a row holds no NaN, the fold's result is the largest value,
+// and its bits are the value's own unless it is a zero (of which the first one's
+// sign counts); a row with a NaN or a zero maximum takes the exact parallel form
+// over LDS.  VEC: n % 4 == 0 and 16-byte aligned rows.
+// What bounds the four-row form: at 4096 x 2048 it is one round of workgroups,
+// so its phases follow one another: both passes over memory about 13 us, exp~
+// and the division (35 and 12 instructions per value) about 7, the chain of adds
+// 4.3 us of latency; 50 -> 27 us on one box against the form above, which reads
+// x three times and its exp~ values back from memory (16384 x 512 59 -> 24, 1000
+// x 8191 80 -> 54).  The one-row form has 256 threads for the row and the same
+// chain: 1 x 2048 14.5 -> 7.4 us, 1 x 8192 51 -> 23, 1024 x 2048 17.7 -> 11.6.
+namespace {
+template <int ROWS, bool VEC>
+CATENA_DEV void softmax_lds_body(const float* x, float* y, uint64_t rows, uint32_t n, uint32_t slot) {
+  constexpr uint32_t T = 256 / ROWS;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ float den_s[ROWS], top_s[4];
+  __shared__ int nan_s[4];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, tid = threadIdx.x % T;
+  float* s = reinterpret_cast<float*>(smem) + (ROWS == 4 ? wave * slot : 0);
+  const uint64_t row = (uint64_t)blockIdx.x * ROWS + (ROWS == 4 ? wave : 0);
+  const bool live = ROWS == 1 || row < rows;
+  const float* xr = x + row * n;
+  const float lowest = __uint_as_float(0xFF800000u);
+  float top = lowest;
+  bool isnan = false;
+  if (live)
+    row_to_lds<ROWS, VEC>(xr, s, n, [&](float v) {
+      isnan |= v != v;
+      top = __builtin_fmaxf(top, v);  // a NaN leaves it
+    });
+  // the wave's largest value: inclusive scans within rows of 16 lanes, rows
+  // joined through row_bcast 15 and 31, lane 63's result for all
+#define CATENA_DPP_FMAX(ctrl, lanes)                                                                              \
+  top = __builtin_fmaxf(top, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(top), __float_as_int(top), \
+                                                                        (ctrl), (lanes), 0xF, false)))
+  CATENA_DPP_FMAX(0x111, 0xF);
+  CATENA_DPP_FMAX(0x112, 0xF);
+  CATENA_DPP_FMAX(0x114, 0xF);
+  CATENA_DPP_FMAX(0x118, 0xF);
+  CATENA_DPP_FMAX(0x142, 0xA);
+  CATENA_DPP_FMAX(0x143, 0xC);
+#undef CATENA_DPP_FMAX
+  float mx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(top), 63));
+  bool anynan = __builtin_amdgcn_ballot_w64(isnan) != 0;
+  if (ROWS == 1) {
+    if (lane == 0) {
+      top_s[wave] = mx;
+      nan_s[wave] = anynan;
+    }
+    __syncthreads();
+    mx = __builtin_fmaxf(__builtin_fmaxf(top_s[0], top_s[1]), __builtin_fmaxf(top_s[2], top_s[3]));
+    anynan = (nan_s[0] | nan_s[1] | nan_s[2] | nan_s[3]) != 0;
+  }
+  if (anynan || mx == 0.0f) {  // the same for every thread of the row; each wave for itself
+    int lastnan = -1;
+    for (uint32_t t = lane; t < n; t += 64)
+      if (s[row_at<ROWS>(t)] != s[row_at<ROWS>(t)]) lastnan = (int)t;
+    lastnan = wave_max_i32(lastnan);
+    if (lastnan == (int)n - 1) {
+      mx = s[row_at<ROWS>(n - 1)];
+    } else {
+      FirstMax fm{lowest, 0xFFFFFFFFu};
+      for (uint32_t t = lastnan + 1 + lane; t < n; t += 64)
+        fm = first_max_combine(fm, FirstMax{s[row_at<ROWS>(t)], t});
+      fm = wave_first_max(fm);
+      mx = fm.i == 0xFFFFFFFFu ? lowest : fm.v;
+    }
+    if (ROWS == 1) __syncthreads();  // every wave has read the row
+  }
+  if (live) {
+    for (uint32_t i = tid; i < (n + 3) / 4; i += T) {
+      f32x4_t* p = reinterpret_cast<f32x4_t*>(s + row_at<ROWS>(4 * i));
+      f32x4_t q = *p;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float shifted = q[c] - mx;
+        const float e = exp_approx(shifted);
+        q[c] = VEC || 4 * i + c < n ? e : 0.0f;  // the slots past the row: +0
+      }
+      *p = q;
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const float den = rows_fold<ROWS, false>(reinterpret_cast<float*>(smem), slot, (n + 3u) & ~3u);
+    if (lane % (64 / ROWS) == 0) den_s[lane / (64 / ROWS)] = den;
+  }
+  __syncthreads();
+  if (!live) return;
+  const float den = den_s[ROWS == 4 ? wave : 0];
+  float* yr = y + row * n;
+  if (VEC) {
+    for (uint32_t i = tid; i < n / 4; i += T) {
+      f32x4_t q = *reinterpret_cast<const f32x4_t*>(s + row_at<ROWS>(4 * i));
+#pragma unroll
+      for (int c = 0; c < 4; ++c) q[c] = q[c] / den;
+      reinterpret_cast<f32x4_t*>(yr)[i] = q;
+    }
+  } else {
+    for (uint32_t i = tid; i < n; i += T) yr[i] = s[row_at<ROWS>(i)] / den;
+  }
+}
+}  // namespace
+
+#define CATENA_SOFTMAX_LDS(name, ROWS, VEC)                                                                      \
+  extern "C" __global__ __launch_bounds__(256) void name(const float* x, float* y, uint64_t rows, uint32_t n,   \
+                                                         uint32_t slot) {                                       \
+    softmax_lds_body<ROWS, VEC>(x, y, rows, n, slot);                                                            \
+  }
+// grid = rows, block = 256, dynamic LDS = slot floats (n rounded up to 4)
+CATENA_SOFTMAX_LDS(catena_softmax_row_vec_f32, 1, true)
+CATENA_SOFTMAX_LDS(catena_softmax_row_f32, 1, false)
+// grid = ceil(rows / 4), block = 256, dynamic LDS = 4 slots of `slot` floats
+// (slot % 4 == 0, at least pad32 of n rounded up to 4)
+CATENA_SOFTMAX_LDS(catena_softmax_rows4_vec_f32, 4, true)
+CATENA_SOFTMAX_LDS(catena_softmax_rows4_f32, 4, false)
+#undef CATENA_SOFTMAX_LDS
+
 // math.exp-approx applied elementwise (catena-lang/stdlib/math.hex:185-199).
 extern "C" __global__ __launch_bounds__(256) void catena_exp_approx_f32(
     const float* __restrict__ x, float* __restrict__ y, uint64_t n) {

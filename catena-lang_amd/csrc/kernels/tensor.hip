@@ -83,6 +83,38 @@ extern "C" __global__ __launch_bounds__(64) void catena_sum_rows_f32(
   }
 }
 
+// The same for rows that fit LDS four to a workgroup: each wave brings a row in,
+// then wave 0 folds the four (serial_sum_rows4).  grid = ceil(rows / 4), block =
+// 256, dynamic LDS = 4 slots of `slot` floats (slot % 4 == 0, at least pad32 of n
+// rounded up to 4).
+namespace {
+template <bool VEC>
+CATENA_DEV void sum_rows4_body(const float* x, float* out, uint64_t rows, uint32_t n, uint32_t mean, uint32_t slot) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  float* s = reinterpret_cast<float*>(smem) + wave * slot;
+  const uint64_t row0 = (uint64_t)blockIdx.x * 4;
+  if (row0 + wave < rows) row_to_lds<4, VEC>(x + (row0 + wave) * n, s, n, [](float) {});
+  const uint32_t n4 = (n + 3u) & ~3u;
+  if (lane < n4 - n) s[pad32(n + lane)] = 0.0f;
+  __syncthreads();
+  if (wave != 0) return;
+  const float sum = serial_sum_rows4<false>(reinterpret_cast<float*>(smem) + (lane >> 4) * slot, n4);
+  if ((lane & 15u) == 0 && row0 + (lane >> 4) < rows) {
+    const float len_f = (float)(uint64_t)n;
+    out[row0 + (lane >> 4)] = mean ? sum / len_f : sum;
+  }
+}
+}  // namespace
+extern "C" __global__ __launch_bounds__(256) void catena_sum_rows4_vec_f32(const float* x, float* out, uint64_t rows,
+                                                                           uint32_t n, uint32_t mean, uint32_t slot) {
+  sum_rows4_body<true>(x, out, rows, n, mean, slot);
+}
+extern "C" __global__ __launch_bounds__(256) void catena_sum_rows4_f32(const float* x, float* out, uint64_t rows,
+                                                                       uint32_t n, uint32_t mean, uint32_t slot) {
+  sum_rows4_body<false>(x, out, rows, n, mean, slot);
+}
+
 // max-f32 of each row: the f32.max-env fold from -inf.  A NaN replaces the
 // accumulator and the next element replaces the NaN, so the result is the
 // last NaN when it is the final element, else the first maximum of the
