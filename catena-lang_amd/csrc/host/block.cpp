@@ -88,6 +88,16 @@ int residual_parts_rmsnorm_bf16(const float* x, const float* resid, uint32_t res
 
 int embed_norm_table_bf16(const uint16_t* table, uint32_t vocab, uint16_t* y, uint64_t n) {
   if (!table || !y) return fail(CATENA_ERR_INVALID_ARGUMENT, "null operand");
+  // bf16 rows in LDS while at least four of the kernel's waves fit a CU (n up to
+  // 5120); below that, or off 16 bytes, the general form
+  int st = ensure_init();
+  if (st) return st;
+  const uint64_t lds = ceil_div(n, 512) * 4096;
+  if (n > 0 && n % 8 == 0 && aligned16(table) && aligned16(y) && lds * 4 <= device().max_lds) {
+    uint32_t n32 = (uint32_t)n;
+    void* args[] = {&table, &y, &vocab, &n32};
+    return launch(KernelId::EmbedNormTable, dim3((unsigned)(((uint64_t)vocab + 4) / 4)), dim3(64), lds, args);
+  }
   return rmsnorm_launch(nullptr, nullptr, nullptr, nullptr, nullptr, y, (uint64_t)vocab + 1, n, nullptr,
                         table, vocab);
 }

@@ -104,6 +104,7 @@ const KernelSpec kKernels[] = {
     {KernelId::EmbedRowsBf16, "block", "catena_embed_rows_bf16"},
     {KernelId::RmsnormRows, "block", "catena_rmsnorm_rows"},
     {KernelId::RmsnormRows4, "block", "catena_rmsnorm_rows4"},
+    {KernelId::EmbedNormTable, "block", "catena_embed_norm_table"},
     {KernelId::RopeQkvStore, "block", "catena_rope_qkv_store"},
     {KernelId::RopeTable, "block", "catena_rope_table"},
     {KernelId::SiluMulBf16, "block", "catena_silu_mul_bf16"},

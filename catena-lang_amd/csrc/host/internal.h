@@ -66,6 +66,7 @@ enum class KernelId : int {
   EmbedRowsBf16,
   RmsnormRows,
   RmsnormRows4,  // four rows a workgroup
+  EmbedNormTable,
   RopeQkvStore,
   RopeTable,
   SiluMulBf16,

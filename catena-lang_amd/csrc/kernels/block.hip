@@ -15,6 +15,9 @@
 
 namespace {
 constexpr uint32_t kNaNBits = 0x7FC00000u;
+constexpr uint32_t kNaNPair = 0x7FC07FC0u;  // as two bf16 values
+// s_waitcnt on vmcnt only (vmcnt[3:0], vmcnt[5:4] at 15:14)
+#define CATENA_WAIT_VM(n) __builtin_amdgcn_s_waitcnt((((n) & 15) | (((n) >> 4) << 14)) | 0x0070 | 0x0F00)
 
 CATENA_DEV int block_max_i32(int v, int* red) {
 #pragma unroll
@@ -92,12 +95,13 @@ CATENA_DEV void rms_finish_row(const float* hs, uint32_t n, uint64_t row, float 
                                float* __restrict__ y_f32, uint16_t* __restrict__ y_bf16) {
   constexpr uint32_t T = 256 / ROWS;
   const uint32_t t = threadIdx.x % T;
+  const SharedDivisor d = shared_divisor(rms);
   if (n % 4 == 0) {
     for (uint32_t i = t; i < n / 4; i += T) {
       const f32x4_t h = *reinterpret_cast<const f32x4_t*>(hs + row_at<ROWS>(4 * i));
-      f32x4_t y;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = h[j] / rms;
+      float q[4] = {h[0], h[1], h[2], h[3]};
+      divide_shared(q, d);
+      const f32x4_t y = {q[0], q[1], q[2], q[3]};
       if (y_f32) reinterpret_cast<f32x4_t*>(y_f32 + row * n)[i] = y;
       if (y_bf16) {
         uint2 p;
@@ -289,6 +293,95 @@ CATENA_RMSNORM_ROWS(catena_rmsnorm_rows, 1)
 // least pad32 of n rounded up to 4)
 CATENA_RMSNORM_ROWS(catena_rmsnorm_rows4, 4)
 #undef CATENA_RMSNORM_ROWS
+
+// The table of every embedding row's norm, y[r] = bf16(nn.rmsnorm(widen(table[r])))
+// for r < vocab and of a row of NaN for r == vocab: the four-row form of
+// catena_rmsnorm_rows for bf16 rows.  One wave folds four rows and shares
+// nothing: the rows go straight to LDS as bf16, all of them in flight at once,
+// then 16 lanes fold a row 32 values at a time, then all 64 divide row by row.
+// Nothing is kept widened, so nine waves fit a CU at 2048 values, all of them
+// folding, where the general form has four of 16.  16-byte units are placed so
+// that the lanes' 64-byte reads spread over the banks.  Loads and stores are
+// nontemporal: the step's weights stay in the Infinity Cache.
+// What bounds it: the two streams (55 us for 32001 x 2048 at the copy rate) with
+// the folds' adds beside them; 106 us in the general form -> 66.
+// grid = ceil((vocab + 1) / 4), block = 64, n % 8 == 0, table and y 16-byte
+// aligned, dynamic LDS = 4 KiB per 512 values of n (rounded up)
+extern "C" __global__ __launch_bounds__(64) void catena_embed_norm_table(const uint16_t* __restrict__ table,
+                                                                         uint16_t* __restrict__ y, uint32_t vocab,
+                                                                         uint32_t n) {
+  typedef __attribute__((address_space(3))) void lds_void;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const uint32_t lane = threadIdx.x, j = lane & 15u, r = lane >> 4;
+  const uint32_t chunks = (n + 511u) / 512u;
+  u32x4_t* units = reinterpret_cast<u32x4_t*>(smem);  // [chunks][4 rows][64]
+  const uint64_t row0 = (uint64_t)blockIdx.x * 4;
+  // unit u of a chunk holds the row's unit (u & ~3) | ((u & 3) ^ ((u >> 4) & 3)),
+  // which is its own inverse
+  const uint32_t mine = (lane & ~3u) | ((lane & 3u) ^ ((lane >> 4) & 3u));
+  for (uint32_t c = 0; c < chunks; ++c) {
+    const uint32_t e = 512 * c + 8 * mine;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      const uint64_t row = row0 + i < vocab ? row0 + i : 0;
+      __builtin_amdgcn_global_load_lds(table + row * n + (e < n ? e : 0u), (lds_void*)(units + (4 * c + i) * 64), 16, 0,
+                                       2);
+    }
+  }
+  const bool real = row0 + r < vocab;  // else a row of NaN
+  float acc = __uint_as_float(0u);
+  for (uint32_t c = 0; c < chunks; ++c) {
+    // chunk c's four loads have landed; those of three more need not have
+    switch (chunks - 1 - c) {
+      case 0: CATENA_WAIT_VM(0); break;
+      case 1: CATENA_WAIT_VM(4); break;
+      case 2: CATENA_WAIT_VM(8); break;
+      default: CATENA_WAIT_VM(12);
+    }
+    asm volatile("" ::: "memory");
+    float v[32];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t e = 512 * c + 32 * j + 8 * p;
+      u32x4_t q = units[(4 * c + r) * 64 + 4 * j + (p ^ ((j >> 2) & 3u))];
+      if (!real) q = u32x4_t{kNaNPair, kNaNPair, kNaNPair, kNaNPair};
+      if (e >= n) q = u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[8 * p + 2 * k] = bf16lo(q[k]) * bf16lo(q[k]);
+        v[8 * p + 2 * k + 1] = bf16hi(q[k]) * bf16hi(q[k]);
+      }
+    }
+    const uint32_t left = n - 512 * c, nl = left >= 512u ? 16u : (left + 31u) / 32u;
+    acc = rows4_chain(v, acc, nl);
+  }
+  const float len_f = (float)(uint64_t)n;
+  const float mean_sq = acc / len_f;
+  const float eps = u32_as_f32(0x3727C5ACu);
+  const float rms = sqrt_newton(mean_sq + eps);
+#pragma unroll 1
+  for (uint32_t i = 0; i < 4 && row0 + i <= vocab; ++i) {
+    const SharedDivisor d =
+        shared_divisor(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(rms), (int)(16 * i))));
+    uint16_t* dst = y + (row0 + i) * n;
+    for (uint32_t c = 0; c < chunks; ++c) {
+      const uint32_t e = 512 * c + 8 * lane;
+      u32x4_t q = units[(4 * c + i) * 64 + mine];
+      if (row0 + i == vocab) q = u32x4_t{kNaNPair, kNaNPair, kNaNPair, kNaNPair};
+      float h[8];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        h[2 * k] = bf16lo(q[k]);
+        h[2 * k + 1] = bf16hi(q[k]);
+      }
+      divide_shared(h, d);
+      u32x4_t o;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = pack_bf16x2(h[2 * k], h[2 * k + 1]);
+      if (e < n) __builtin_nontemporal_store(o, reinterpret_cast<u32x4_t*>(dst + e));
+    }
+  }
+}
 
 // RoPE on the q and k parts of a fused projection, bf16 q out, and the
 // KV-cache append.  qkv[R][3*H*D] f32 with R = B * Tq rows (row b*Tq + tq,

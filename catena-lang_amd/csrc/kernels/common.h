@@ -27,17 +27,18 @@ CATENA_DEV float bf16hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
 CATENA_DEV float bf16_to_f32(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
 // f32 -> bf16 round-to-nearest-even; NaN keeps sign and top payload and is
-// made quiet.  Integer formulation so the CPU oracle (or_f32_to_bf16) and the
-// device agree bit for bit.
+// made quiet.  v_cvt_pk_bf16_f32 gives the bits of the CPU oracle's integer
+// form (or_f32_to_bf16) for each of the 2^32 inputs, in one instruction for two
+// values against eight each.
 CATENA_DEV uint32_t f32_to_bf16_bits(float x) {
-  uint32_t u = __float_as_uint(x);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (u >> 16) | 0x0040u;
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return u >> 16;
+  return __builtin_bit_cast(uint16_t, (__bf16)x);
 }
 
 CATENA_DEV uint32_t pack_bf16x2(float lo, float hi) {
-  return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  const f2 v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
 }
 
 // f32.round-to-u32 = (uint32_t)nearbyintf(x) (catena-lang/src/codegen/
@@ -351,10 +352,82 @@ CATENA_DEV float serial_sum_wave_long(const float* s, uint32_t n) {
   return acc;
 }
 
+// Correctly rounded quotients by one divisor that many elements share, in four
+// fused steps an element (the compiler's division takes about twelve, one of
+// them a quarter-rate reciprocal).  hi = RN(1/b), lo = RN((1 - b hi) hi), the
+// first remainder exact, so hi + lo = 1/b (1 + 2^-47); q0 = fma(a, hi, a lo) is
+// then within one ulp of a / b, its remainder fma(-b, q0, a) is exact and
+// fma(remainder, hi, q0) is the correctly rounded quotient (P. Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000 processor",
+// 1990: a faithful quotient and a correctly rounded reciprocal give it).  The
+// bounds keep every step in the normal range: b in [2^-20, 2^20] and the |a| of
+// a group in [2^-98, 2^100] give |a / b| >= 2^-118 and remainders that are
+// multiples of 2^-146.  Groups outside them, zeros (whose sign the steps would
+// lose), infinities and NaN take the plain division.
+struct SharedDivisor {
+  float b, hi, lo;
+  bool fast;
+};
+CATENA_DEV SharedDivisor shared_divisor(float b) {
+  SharedDivisor d;
+  d.b = b;
+  d.hi = 1.0f / b;
+  d.lo = __builtin_fmaf(-b, d.hi, 1.0f) * d.hi;
+  d.fast = b >= 0x1p-20f && b <= 0x1p20f;
+  return d;
+}
+template <int N>
+CATENA_DEV void divide_shared(float (&a)[N], const SharedDivisor& d) {
+  bool fast = d.fast;
+  float lo = __builtin_fabsf(a[0]), hi = lo;
+#pragma unroll
+  for (int i = 1; i < N; ++i) {
+    lo = __builtin_fminf(lo, __builtin_fabsf(a[i]));
+    hi = __builtin_fmaxf(hi, __builtin_fabsf(a[i]));
+  }
+  fast = fast && lo >= 0x1p-98f && hi <= 0x1p100f;
+  if (__builtin_amdgcn_ballot_w64(!fast) == 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float q = __builtin_fmaf(a[i], d.hi, a[i] * d.lo);
+      a[i] = __builtin_fmaf(__builtin_fmaf(-d.b, q, a[i]), d.hi, q);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) a[i] = a[i] / d.b;
+  }
+}
+
 // Rows of a four-row workgroup in LDS: four floats of padding after every 32,
 // so that the 32-value blocks that a row's 16 lanes fold start 36 floats apart
 // and their 16-byte reads cover the banks once.
 CATENA_DEV uint32_t pad32(uint32_t i) { return i + (i >> 5) * 4u; }
+
+// One 512-value chunk of a four-row fold: lane j of a 16-lane row holds values
+// 32 j .. 32 j + 31 of its row's chunk, nl of the lanes hold any; acc is the
+// row's sum so far, and so is what every lane of the row gets back.
+CATENA_DEV float rows4_chain(const float (&v)[32], float acc, uint32_t nl) {
+  float a = acc;
+#pragma unroll
+  for (int k = 0; k < 32; ++k) a = a + v[k];
+  auto block = [&]() {
+    // two wait states between the write of a and its DPP read, also across
+    // the loop's back edge
+    asm volatile("s_nop 1");
+    a = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xF, 0xF, true)) + v[0];
+#pragma unroll
+    for (int k = 1; k < 32; ++k) a = a + v[k];
+  };
+  uint32_t L = 1;
+#pragma unroll 1
+  for (; L + 5 <= nl; L += 5) {
+#pragma unroll
+    for (int r = 0; r < 5; ++r) block();
+  }
+#pragma unroll 1
+  for (; L < nl; ++L) block();
+  return __shfl(a, (int)((threadIdx.x & 48u) + nl - 1u), 64);
+}
 
 // The sequential fold of serial_sum_wave_long for four rows at once, one per
 // 16-lane DPP row (all 64 lanes call it with their own row's s, rows padded as
@@ -388,26 +461,7 @@ CATENA_DEV float serial_sum_rows4(const float* s, uint32_t n) {
     float nx[32];
     if (left > 512u) load(nx, base + 512);
     __builtin_amdgcn_sched_barrier(0);
-    float a = acc;
-#pragma unroll
-    for (int k = 0; k < 32; ++k) a = a + v[k];
-    auto block = [&]() {
-      // two wait states between the write of a and its DPP read, also across
-      // the loop's back edge
-      asm volatile("s_nop 1");
-      a = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xF, 0xF, true)) + v[0];
-#pragma unroll
-      for (int k = 1; k < 32; ++k) a = a + v[k];
-    };
-    uint32_t L = 1;
-#pragma unroll 1
-    for (; L + 5 <= nl; L += 5) {
-#pragma unroll
-      for (int r = 0; r < 5; ++r) block();
-    }
-#pragma unroll 1
-    for (; L < nl; ++L) block();
-    acc = __shfl(a, (int)((threadIdx.x & 48u) + nl - 1u), 64);
+    acc = rows4_chain(v, acc, nl);
 #pragma unroll
     for (int k = 0; k < 32; ++k) v[k] = nx[k];
   }

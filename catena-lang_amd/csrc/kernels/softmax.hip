@@ -181,17 +181,21 @@ CATENA_DEV void softmax_lds_body(const float* x, float* y, uint64_t rows, uint32
   }
   __syncthreads();
   if (!live) return;
-  const float den = den_s[ROWS == 4 ? wave : 0];
+  const SharedDivisor den = shared_divisor(den_s[ROWS == 4 ? wave : 0]);
   float* yr = y + row * n;
   if (VEC) {
     for (uint32_t i = tid; i < n / 4; i += T) {
-      f32x4_t q = *reinterpret_cast<const f32x4_t*>(s + row_at<ROWS>(4 * i));
-#pragma unroll
-      for (int c = 0; c < 4; ++c) q[c] = q[c] / den;
-      reinterpret_cast<f32x4_t*>(yr)[i] = q;
+      const f32x4_t e = *reinterpret_cast<const f32x4_t*>(s + row_at<ROWS>(4 * i));
+      float q[4] = {e[0], e[1], e[2], e[3]};
+      divide_shared(q, den);
+      reinterpret_cast<f32x4_t*>(yr)[i] = f32x4_t{q[0], q[1], q[2], q[3]};
     }
   } else {
-    for (uint32_t i = tid; i < n; i += T) yr[i] = s[row_at<ROWS>(i)] / den;
+    for (uint32_t i = tid; i < n; i += T) {
+      float q[1] = {s[row_at<ROWS>(i)]};
+      divide_shared(q, den);
+      yr[i] = q[0];
+    }
   }
 }
 }  // namespace

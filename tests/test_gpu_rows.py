@@ -7,6 +7,7 @@ import pytest
 
 import catena_amd as ca
 import oracle
+from oracle import decoder as od
 from gpu_util import say
 
 pytestmark = pytest.mark.gpu
@@ -33,10 +34,15 @@ def _rows(rows, n, seed):
         lambda r: np.where(np.arange(n) == n // 3, INF, r),
         lambda r: np.full_like(r, 1e-42),
         lambda r: np.minimum(r, np.float32(0.0)),
+        # quotients outside the bounds of the shared-divisor division
+        lambda r: r * np.float32(1e-33),
+        lambda r: r * np.float32(10.0) ** (-(np.arange(n) % 44)).astype(np.float32),
+        lambda r: r * np.float32(1e12),
+        lambda r: np.where(np.arange(n) % 5 == 0, np.float32(-0.0), r),
     ]
     at = rng.permutation(rows)[:len(special)]
     for i, f in zip(at, special):
-        x[i] = f(x[i])
+        x[i] = f(x[i]).astype(np.float32)
     return x, sorted(set(at.tolist()) | {0, rows - 1} | set(rng.integers(0, rows, 6).tolist()))
 
 
@@ -132,3 +138,23 @@ def test_residual_rmsnorm_bf16(n, parts):
     for a in range(0, rows, 1024):
         hs, ys = run(index[a:a + 1024])
         assert np.array_equal(h[a:a + 1024], hs) and np.array_equal(y[a:a + 1024], ys)
+
+
+# whole and partial 512-value chunks, the longest rows of the bf16 form and the
+# next ones (general form)
+@pytest.mark.parametrize("heads,vocab", [(1, 8), (1, 2056), (5, 1032), (16, 2104), (40, 1032), (41, 8)])
+def test_embed_norm_table(heads, vocab):
+    d = 128 * heads
+    say(f"normalized embedding table {vocab} x {d}")
+    x, _ = _rows(vocab, d, vocab + d)
+    bits = oracle.f32_to_bf16_bits_np(x).reshape(vocab, d)
+    dec = ca.Decoder(d, heads, 128, 1, vocab, 1, 16)
+    dec.init_weights(seed=1, std=0.02)
+    ca.mem_write(dec.tensor(ca.DEC_EMBED), bits)
+    dec.prefill(ca.Buffer.from_array(np.zeros((1, 1), np.uint32)), 1, 1, ca.Buffer(4))
+    tab = dec.read(ca.DEC_EMBED_NORM, np.uint16).reshape(vocab + 1, d)
+    dec.close()
+    want = od.residual_rmsnorm_bf16((bits.astype(np.uint32) << 16).view(np.float32))[1]
+    as_f32 = lambda u: (u.astype(np.uint32) << 16).view(np.float32)  # noqa: E731
+    _same(as_f32(tab[:vocab]), as_f32(want.reshape(vocab, d)))
+    assert np.isnan(as_f32(tab[vocab])).all()
