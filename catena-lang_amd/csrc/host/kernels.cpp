@@ -532,17 +532,20 @@ int catena_mi355x_gemm_f32_exact(const float* a, const float* b, float* c, uint6
     return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
   const uint64_t t16 = ceil_div(m, 16) * ceil_div(n, 16);
   const bool words = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 3u) == 0;
-  // One cell per thread on 16 x 16 tiles: A by DPP row broadcast and B through
-  // LDS (k % 16 == 0, 16-byte rows of B, 31-bit buffer offsets) up to four
-  // tiles for each CU (512^3: 13.0 us against 13.9), else A and B both through
-  // LDS while each CU gets one tile (255^3: 6.9 us against 8.6; 300 x 300 x 301,
-  // 361 tiles: 10.2 against 9.5) or operands are not word-aligned or too wide
-  // for the offsets below.
-  if (t16 <= 4 * kDecodeSpread && k > 0 && k % 16 == 0 && m % 4 == 0 && aligned16(b) && words &&
+  // One cell per thread on 16 x 16 tiles, A by DPP row broadcast and B through
+  // LDS (k % 16 == 0, 16-byte rows of B, 31-bit buffer offsets): up to 6.5 tiles
+  // for each CU (1792 x 192 x 1728, 1344 tiles: 54 us against 65 with 2 x 1; 576 x
+  // 1088 x 896, 2448: 47 against 42 with 4 x 1).  Else A and B both through LDS up
+  // to two tiles for each CU, to three where the operands outgrow an XCD's L2,
+  // which the row forms feel first (192 x 960 x 1103, 720 tiles: 36 us against 42
+  // with 2 x 1; 192 x 734 x 681, 552 tiles: 24 against 19), or when operands are
+  // not word-aligned or too wide for the offsets below.
+  if (t16 <= 13 * kDecodeSpread / 2 && k > 0 && k % 16 == 0 && m % 4 == 0 && aligned16(b) && words &&
       (n + 16) * k * 4 < (1ull << 31) && (k + 256) * m * 4 < (1ull << 31) && ceil_div(n, 16) <= 65535)
     return launch(KernelId::GemmF32ExactQ16, dim3((unsigned)ceil_div(m, 16), (unsigned)ceil_div(n, 16)), dim3(256),
                   256 * 16 * 4, args);
-  if (t16 <= kDecodeSpread || !words || k >= (1ull << 26) || m >= (1ull << 25)) {
+  const bool past_l2 = n + m > (3ull << 20) / 4 / (k > 0 ? k : 1);
+  if (t16 <= (past_l2 ? 3 : 2) * kDecodeSpread || !words || k >= (1ull << 26) || m >= (1ull << 25)) {
     if (t16 > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
     return launch(KernelId::GemmF32ExactT16, dim3((unsigned)t16), dim3(256), 0, args);
   }

@@ -48,7 +48,9 @@ def _check(n, m, k, shift=0, special=False):
     (257, 257, 1), (272, 257, 7), (273, 259, 16), (300, 301, 17), (1000, 70, 33), (70, 1000, 47), (5, 20000, 31),
     (385, 1537, 15), (400, 1600, 16), (401, 1601, 48), (9600, 63, 19), (9601, 65, 16),
     (1089, 2561, 8), (1120, 2560, 9), (33, 90000, 7), (1121, 2562, 24),
-    (512, 512, 16), (512, 516, 16), (516, 512, 32)])
+    (512, 512, 16), (512, 516, 16), (516, 512, 32),
+    # two tiles for each of 256 CUs (three past 3 MiB of operands), 6.5 of the DPP form
+    (512, 256, 17), (513, 255, 17), (522, 256, 1011), (522, 256, 1010), (769, 250, 801), (1664, 256, 16), (1665, 256, 16)])
 def test_row_forms(n, m, k):
     _check(n, m, k)
 
