@@ -58,6 +58,10 @@ const KernelSpec kKernels[] = {
     {KernelId::GemmF32ExactQ16, "gemm_f32_exact", "catena_gemm_f32_exact_q16"},
     {KernelId::GemmBf16EdgeBf16, "gemm_bf16", "catena_gemm_bf16_edge_bf16out"},
     {KernelId::GemmBf16EdgeF32, "gemm_bf16", "catena_gemm_bf16_edge_f32out"},
+    {KernelId::GemmBf16Any192x128F32, "gemm_bf16_any", "catena_gemm_bf16_any_192x128_f32out"},
+    {KernelId::GemmBf16Any192x128Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_192x128_bf16out"},
+    {KernelId::GemmBf16Any128x192F32, "gemm_bf16_any", "catena_gemm_bf16_any_128x192_f32out"},
+    {KernelId::GemmBf16Any128x192Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_128x192_bf16out"},
     {KernelId::GemmBf16Any128x128F32, "gemm_bf16_any", "catena_gemm_bf16_any_128x128_f32out"},
     {KernelId::GemmBf16Any128x128Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_128x128_bf16out"},
     {KernelId::GemmBf16Any64x128F32, "gemm_bf16_any", "catena_gemm_bf16_any_64x128_f32out"},

@@ -20,6 +20,10 @@ enum class KernelId : int {
   GemmF32ExactQ16,  // 16x16 tiles, A by DPP row broadcast: k % 16 == 0, m % 4 == 0
   GemmBf16EdgeBf16,  // no alignment, no scratch, any size (gemm_bf16.hip)
   GemmBf16EdgeF32,
+  GemmBf16Any192x128F32,
+  GemmBf16Any192x128Bf16,
+  GemmBf16Any128x192F32,
+  GemmBf16Any128x192Bf16,
   GemmBf16Any128x128F32,  // ragged and small shapes (gemm_bf16_any.hip), f32 / bf16 per tile
   GemmBf16Any128x128Bf16,
   GemmBf16Any64x128F32,

@@ -68,16 +68,20 @@ uint32_t decode_kw(uint64_t n_cols, uint64_t k, bool regs_path) {
 // `alone` and `shared`: microseconds per 32-k slab of one workgroup that has
 // its CU to itself, and of each of the `fit` workgroups that share a CU;
 // `stream`: GB/s at which one CU brings a weight in from HBM (the narrower
-// the tile's rows, the less).  Fitted to 2,900 timings of the five general
+// the tile's rows, the less).  Fitted to 2,900 timings of five general
 // kernels and the ragged 256 x 256 one over n = 17 .. 4000, widths 256 ..
 // 11264 and depths 512 .. 11008, 1 to 16 k groups: the tile it picks is on
 // average 2.4 % from the fastest (1.22x at worst, 0.5 % without k groups).
+// The 192 x 128 and 128 x 192 rows come from 150 more; where the choice moved to
+// them, 13 of 400 drawn products, those take 10 % less on average, none longer.
 struct GemmTile {
   KernelId f32, bf16;
   uint32_t bm, bn, waves, stages, stage_k, fit;
   double alone, shared, stream;
 };
 constexpr GemmTile kGemmTiles[] = {
+    {KernelId::GemmBf16Any192x128F32, KernelId::GemmBf16Any192x128Bf16, 192, 128, 4, 2, 64, 2, 0.44, 0.27, 36.3},
+    {KernelId::GemmBf16Any128x192F32, KernelId::GemmBf16Any128x192Bf16, 128, 192, 4, 2, 64, 2, 0.46, 0.29, 36.3},
     {KernelId::GemmBf16Any128x128F32, KernelId::GemmBf16Any128x128Bf16, 128, 128, 4, 2, 64, 2, 0.358, 0.211, 36.3},
     {KernelId::GemmBf16Any64x128F32, KernelId::GemmBf16Any64x128Bf16, 64, 128, 4, 3, 64, 2, 0.217, 0.158, 36.3},
     {KernelId::GemmBf16Any64x64F32, KernelId::GemmBf16Any64x64Bf16, 64, 64, 4, 2, 128, 2, 0.169, 0.105, 33.5},
@@ -85,7 +89,7 @@ constexpr GemmTile kGemmTiles[] = {
     {KernelId::GemmBf16Any32x32F32, KernelId::GemmBf16Any32x32Bf16, 32, 32, 4, 4, 128, 2, 0.075, 0.067, 24.8},
     {KernelId::GemmBf16K32EdgeF32, KernelId::GemmBf16K32EdgeBf16, 256, 256, 8, 4, 32, 1, 0.705, 0.705, 36.3},
 };
-constexpr int kTileRagged256 = 5;
+constexpr int kTileRagged256 = 7;
 // k groups a product may be split into (with 1: whole)
 constexpr uint32_t kGemmSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
 // row strides up to which the general kernels' 32-bit offsets reach (a stage

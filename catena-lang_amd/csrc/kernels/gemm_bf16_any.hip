@@ -34,6 +34,12 @@
 // (4.1 TB/s; 38 us whole), 999 x 2048 x 5632 1300 -> 40 us.  Tried for the 128
 // x 128 tile at 1000 x 6144 x 2048: stages of one slab, 4 deep 40 us, 3 deep
 // 38; eight waves 37; the 256 x 128 kernel 36.
+// The 192 x 128 and 128 x 192 tiles (also two workgroups to a CU, exactly its
+// LDS) read 20 % less LDS per MFMA and fill rounds that 128 x 128 leaves half
+// empty: 1340 x 6400 x 1408 46.3 -> 36.7 us, 1119 x 8320 x 4096 107 -> 88, 2816 x
+// 10368 x 1920 149 -> 120, 999 x 11264 x 2048 60.9 -> 52.9.  Tried beside them
+// and no better over 150 shapes: 128 x 192 in eight waves, three or four stages
+// (one workgroup to a CU), 256 x 192, fragments double-buffered in registers.
 // One barrier per stage: it follows the wait for the stage's loads and frees
 // the buffer read one stage earlier, which the loads of stage t + S - 1 then
 // fill, so S - 1 stages are in flight while one is multiplied.
@@ -48,8 +54,8 @@ typedef __attribute__((address_space(3))) i16x4_t lds_i16x4;
 
 template <int BN>
 CATENA_DEV uint32_t hB(uint32_t k) {
-  if (BN >= 128) return 2u * ((k & 3u) | (((k >> 3) & 1u) << 2));  // 256-byte rows: all alias
-  if (BN == 64) return 2u * (((k >> 1) & 1u) | (((k >> 3) & 1u) << 1));  // row parity picks the half
+  if (BN == 128) return 2u * ((k & 3u) | (((k >> 3) & 1u) << 2));  // 256-byte rows: all alias
+  if (BN == 64 || BN == 192) return 2u * (((k >> 1) & 1u) | (((k >> 3) & 1u) << 1));  // 128- and 384-byte rows: row parity picks the half
   return 2u * ((k >> 3) & 1u);                                     // 64-byte rows: k & 3 picks the quarter
 }
 
@@ -91,7 +97,7 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
   constexpr int A_INS = BM / 16, B_INS = BN / 16;      // 1-KiB loads per slab
   static_assert(KS * A_INS % WAVES == 0 && KS * B_INS % WAVES == 0, "whole loads per wave");
   constexpr int LA = KS * A_INS / WAVES, LB = KS * B_INS / WAVES, LOADS = LA + LB;  // per wave and stage
-  constexpr int BL = BN / 8, BR = 64 / BL;             // lanes per B row, B rows in one load
+  constexpr int BL = BN / 8;                           // 16-byte chunks per B row
   extern __shared__ __attribute__((aligned(1024))) uint16_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -118,8 +124,8 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
 #pragma unroll
   for (int l = 0; l < LB; ++l) {
     const int x = wave * LB + l;
-    const uint32_t kr = BR * (x % B_INS) + (uint32_t)lane / BL;  // row in the slab
-    const uint32_t q = (uint32_t)(lane % BL) ^ hB<BN>(kr);
+    const uint32_t ch = 64 * (x % B_INS) + (uint32_t)lane;  // 16-byte chunk of the slab
+    const uint32_t kr = ch / BL, q = ch % BL ^ hB<BN>(kr);  // its row, the global chunk it holds
     boff[l] = (uint32_t)(((x / B_INS * BK + kr) * ldb + 8 * q) * 2);
   }
   auto a_dst = [&](int buf, int l) {
@@ -128,7 +134,7 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
   };
   auto b_dst = [&](int buf, int l) {
     const int x = wave * LB + l;
-    return (lds_void*)(smem + buf * ST + x / B_INS * (A_ST + B_ST) + A_ST + x % B_INS * BR * BN);
+    return (lds_void*)(smem + buf * ST + x / B_INS * (A_ST + B_ST) + A_ST + x % B_INS * 512);
   };
   auto issue = [&](int64_t k0, int buf) {  // the stage at k0 into buffer buf
     const int64_t left = kend - k0;        // k rows left (<= 0: every load brings zeros)
@@ -250,6 +256,8 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
     gemm_any_body<BM, BN, WM, WN, KS, S, true>(A, B, C, M, N, K, lda, ldb, k_len, vec);                  \
   }
 
+CATENA_GEMM_ANY(192x128, 192, 128, 2, 2, 2, 2)
+CATENA_GEMM_ANY(128x192, 128, 192, 2, 2, 2, 2)
 CATENA_GEMM_ANY(128x128, 128, 128, 2, 2, 2, 2)
 CATENA_GEMM_ANY(64x128, 64, 128, 2, 2, 2, 3)
 CATENA_GEMM_ANY(64x64, 64, 64, 2, 2, 4, 2)

@@ -59,7 +59,8 @@ def _check(n, m, k, shifts=(0, 0, 0)):
     (17, 8, 8), (31, 40, 32), (32, 32, 40), (33, 64, 120), (63, 72, 136), (64, 128, 96), (65, 136, 264),
     (127, 248, 512), (129, 264, 1032), (255, 520, 96), (257, 256, 160), (513, 1032, 1000), (1000, 2056, 72),
     (700, 3000, 232), (1, 1, 1), (3, 7, 1000), (16, 9, 64), (5, 64, 9), (40, 33, 31), (100, 127, 129),
-    (257, 511, 255), (300, 1000, 2), (20, 4096, 3), (256, 256, 128), (256, 384, 256), (512, 512, 640)])
+    (257, 511, 255), (300, 1000, 2), (643, 10944, 136), (766, 11050, 137), (965, 10944, 136), (967, 10947, 129),
+    (20, 4096, 3), (256, 256, 128), (256, 384, 256), (512, 512, 640)])
 def test_general_shapes(n, m, k):
     _check(n, m, k)
 
