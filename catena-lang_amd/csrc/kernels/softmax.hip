@@ -6,11 +6,12 @@
 //   denom = f32.add-env fold from +0 of exp~(x_i - max)   (nn.hex:59-72)
 //   out_i = exp~(x_i - max) / denom                        (nn.hex:75-90)
 // The reference runs both folds serially on the host (the entry is host-only
-// because it contains a materialize).  Here one workgroup per row computes
-// the max with the exact parallel form of the fold (FirstMax, common.h),
-// writes exp~ values to the output, folds the denominator in ascending order
-// as one lane-to-lane chain in wave 0 (serial_sum_wave), and divides in
-// place -- bitwise the sequential result.
+// because it contains a materialize).  Rows that fit LDS: softmax_lds_body below.
+// Longer ones: one workgroup per row computes the max with the exact parallel
+// form of the fold (FirstMax, common.h), writes exp~ values to the output, folds
+// the denominator in ascending order as one lane-to-lane chain in wave 0
+// (serial_sum_wave), and divides in place.  Both are bitwise the sequential
+// result.
 #include "common.h"
 
 namespace {

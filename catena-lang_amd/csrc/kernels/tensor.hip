@@ -9,7 +9,8 @@
 //   max-f32                f32.max-env fold from -inf (acc >= x ? acc : x)
 //   sum-u64 / dot-u64      wrapping u64 sums (order-independent), the
 //                          reference's test programs tests/cases/reducec/basic.hex
-// The f32 sum stays one serial chain (serial_sum_wave); the max uses the
+// The f32 sum stays one serial chain (serial_sum_wave, or four rows' chains in
+// one wave, serial_sum_rows4); the max uses the
 // exact parallel form of its fold (FirstMax in common.h).
 #include "common.h"
 
