@@ -353,17 +353,18 @@ CATENA_DEV float serial_sum_wave_long(const float* s, uint32_t n) {
 }
 
 // Correctly rounded quotients by one divisor that many elements share, in four
-// fused steps an element (the compiler's division takes about twelve, one of
-// them a quarter-rate reciprocal).  hi = RN(1/b), lo = RN((1 - b hi) hi), the
-// first remainder exact, so hi + lo = 1/b (1 + 2^-47); q0 = fma(a, hi, a lo) is
-// then within one ulp of a / b, its remainder fma(-b, q0, a) is exact and
-// fma(remainder, hi, q0) is the correctly rounded quotient (P. Markstein,
-// "Computation of elementary functions on the IBM RISC System/6000 processor",
-// 1990: a faithful quotient and a correctly rounded reciprocal give it).  The
-// bounds keep every step in the normal range: b in [2^-20, 2^20] and the |a| of
-// a group in [2^-98, 2^100] give |a / b| >= 2^-118 and remainders that are
-// multiples of 2^-146.  Groups outside them, zeros (whose sign the steps would
-// lose), infinities and NaN take the plain division.
+// fused steps an element and the fixup that ends every division here (the
+// compiler's takes about twelve, one of them a quarter-rate reciprocal).  hi =
+// RN(1/b), lo = RN((1 - b hi) hi), the first remainder exact, so hi + lo = 1/b (1
+// + 2^-47); q0 = fma(a, hi, a lo) is then within one ulp of a / b, its remainder
+// fma(-b, q0, a) is exact and fma(remainder, hi, q0) is the correctly rounded
+// quotient (P. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", 1990: a faithful quotient and a correctly rounded
+// reciprocal give it).  The bounds keep every step in the normal range: b in
+// [2^-20, 2^20] and the |a| of a group in [2^-98, 2^100] give |a / b| >= 2^-118
+// and remainders that are multiples of 2^-146.  Groups outside them, zeros
+// included, take the plain division; 4.3e9 pairs, near ties and with extreme
+// mantissas among them, gave its bits.
 struct SharedDivisor {
   float b, hi, lo;
   bool fast;
@@ -390,7 +391,7 @@ CATENA_DEV void divide_shared(float (&a)[N], const SharedDivisor& d) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const float q = __builtin_fmaf(a[i], d.hi, a[i] * d.lo);
-      a[i] = __builtin_fmaf(__builtin_fmaf(-d.b, q, a[i]), d.hi, q);
+      a[i] = __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d.b, q, a[i]), d.hi, q), d.b, a[i]);
     }
   } else {
 #pragma unroll
