@@ -304,7 +304,7 @@ CATENA_RMSNORM_ROWS(catena_rmsnorm_rows4, 4)
 // that the lanes' 64-byte reads spread over the banks.  Loads and stores are
 // nontemporal: the step's weights stay in the Infinity Cache.
 // What bounds it: the two streams (55 us for 32001 x 2048 at the copy rate) with
-// the folds' adds beside them; 106 us in the general form -> 66.
+// the folds' adds beside them; 106 us in the general form -> 69.
 // grid = ceil((vocab + 1) / 4), block = 64, n % 8 == 0, table and y 16-byte
 // aligned, dynamic LDS = 4 KiB per 512 values of n (rounded up)
 extern "C" __global__ __launch_bounds__(64) void catena_embed_norm_table(const uint16_t* __restrict__ table,
