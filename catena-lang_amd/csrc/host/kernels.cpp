@@ -125,6 +125,7 @@ struct GemmPlan {
   uint32_t splits = 1;
   double us = 0;
 };
+// k > 0 when may_split (an empty fold has no groups)
 GemmPlan gemm_plan(uint64_t n, uint64_t m, uint64_t k, bool ragged256, bool may_split) {
   GemmPlan best;
   best.us = -1;
@@ -462,7 +463,7 @@ int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_
     const uint64_t a_bytes = pack_a ? ceil_div(n * lda * 2, 256) * 256 : 0;
     const uint64_t b_bytes = pack_b ? ceil_div(k * ldb * 2, 256) * 256 : 0;
     const bool ragged256 = k > 0 && (k % 32 == 0 || pack_a);
-    const bool splittable = may_split && !tile_ok && !n128_ok && n * m % 4 == 0;
+    const bool splittable = may_split && k > 0 && !tile_ok && !n128_ok && n * m % 4 == 0;
     GemmPlan p = gemm_plan(n, m, k, ragged256, splittable);
     uint64_t need = a_bytes + b_bytes + (p.splits > 1 ? p.splits * n * m * 4 : 0);
     std::unique_lock<std::mutex> ws_guard(d.ws_mu, std::defer_lock);

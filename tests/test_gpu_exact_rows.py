@@ -59,3 +59,15 @@ def test_row_forms(n, m, k):
 @pytest.mark.parametrize("shift,special", [(4, False), (12, True), (0, True), (2, False)])
 def test_addresses_and_special_values(n, m, k, shift, special):
     _check(n, m, k, shift, special)
+
+
+# the forms' ranges: 16 x 16 tiles, 2 x 1, 4 x 1, 8 x 2
+@pytest.mark.parametrize("n,m", [(1, 1), (33, 31), (300, 301), (401, 1601), (1121, 2562)])
+def test_empty_fold(n, m):
+    """k == 0: every cell is the fold's start, +0; the operands may be null."""
+    say(f"gemm f32 exact empty fold {n}x{m}")
+    cb = ca.Buffer.from_array(np.full(n * m * 4 + 512, 0xA5, np.uint8))
+    ca.gemm_f32_exact(0, 0, cb.ptr + 256, n, m, 0)
+    raw = cb.read(np.uint8)
+    assert not raw[256:-256].any()
+    assert np.all(raw[:256] == 0xA5) and np.all(raw[-256:] == 0xA5)

@@ -116,3 +116,16 @@ def test_strides_past_the_32_bit_offsets():
     say(f"bf16 gemm {n}x{m}x{k}")
     got = _product(a16, b16, True)
     assert np.array_equal(got, as_f32(a16) @ as_f32(b16).astype(np.float64))
+
+
+@pytest.mark.parametrize("n,m", [(1, 1), (3, 7), (8, 128), (16, 9), (17, 8), (32, 32), (33, 31), (256, 256), (1000, 2056)])
+@pytest.mark.parametrize("out_f32", [True, False])
+def test_empty_fold(n, m, out_f32):
+    """k == 0: every element is the fold's start, +0; the operands may be null."""
+    es = 4 if out_f32 else 2
+    say(f"bf16 gemm empty fold {n}x{m} f32 {out_f32}")
+    cb = ca.Buffer.from_array(np.full(n * m * es + 512, 0xA5, np.uint8))
+    ca.gemm_bf16(0, 0, cb.ptr + 256, n, m, 0, out_f32=out_f32)
+    raw = cb.read(np.uint8)
+    assert not raw[256:-256].any()
+    assert np.all(raw[:256] == 0xA5) and np.all(raw[-256:] == 0xA5)
