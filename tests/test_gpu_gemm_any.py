@@ -65,6 +65,25 @@ def test_general_shapes(n, m, k):
     _check(n, m, k)
 
 
+# the 256 x 256 tile with ragged edges (the tile the host's estimate takes for
+# these): 1, 15, 16, 17 rows in the last tile; 1, 15, 17 k rows in the last slab
+# and slabs past k; B packed, A packed, both, none
+@pytest.mark.parametrize("n,m,k", [(257, 13567, 1), (271, 14976, 1), (272, 14720, 1), (273, 14593, 1), (1025, 11648, 33),
+                                   (1040, 10990, 33), (1537, 7681, 47), (1537, 7552, 49), (1281, 6138, 81),
+                                   (1025, 11007, 64), (1025, 7432, 96)])
+def test_ragged_256_tile(n, m, k):
+    # what the packed operands of a longer product leave in the scratch memory:
+    # a row read past one of this product's shows as a NaN
+    nan = np.full((n, k + 39), NAN16, np.uint16), np.full((k + 39, m), NAN16, np.uint16)
+    _product(*nan, True)
+    _check(n, m, k)
+
+
+@pytest.mark.parametrize("shifts", [(1, 0, 0), (0, 1, 0), (0, 0, 1)])
+def test_ragged_256_tile_unaligned(shifts):
+    _check(1025, 7432, 96, shifts)
+
+
 # few tiles and a deep k: folded as 2 .. 16 k groups, the last one shorter
 @pytest.mark.parametrize("n,m,k", [(17, 256, 8192), (24, 96, 4104), (48, 4096, 2888), (64, 512, 8200), (100, 1024, 5000),
                                    (33, 64, 16384), (20, 60, 4099)])
