@@ -159,19 +159,19 @@ CATENA_DEV void gemm_k32_body(const uint16_t* __restrict__ A, const uint16_t* __
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           (void*)(A + m0 * LDA + (live ? k0 : 0)), (short)0,
           !live ? 0 : EDGE ? records((M - m0 < BM ? M - m0 : BM) * LDA - k0) : (int)(BM * LDA * 2), kRsrcWord3);
-      const uint32_t step = idx ? (uint32_t)(16 * LDA * 2) : 0;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rs, (lds_void*)(smem + stage * A_ST + (32 * wave + 16 * idx) * BK), 16,
-          (int)(EDGE ? aoff + step : aoff), EDGE ? 0 : (int)step, 0, 0);
+          EDGE && idx ? (int)(aoff + (uint32_t)(16 * LDA * 2)) : (int)aoff,
+          !EDGE && idx ? (int)(16 * LDA * 2) : 0, 0, 0);
     } else {
       const int b = idx - 2;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           (void*)(B + (live ? k0 : 0) * LDB + n0), (short)0,
           !live ? 0 : EDGE ? records((K - k0 < BK ? K - k0 : BK) * LDB - n0) : (int)(BK * N * 2), kRsrcWord3);
-      const uint32_t step = b ? (uint32_t)(16 * LDB * 2) : 0;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rs, (lds_void*)(smem + S * A_ST + stage * B_ST + ((64 / B_LANES) * wave + 16 * b) * BN), 16,
-          (int)(EDGE ? boff + step : boff), EDGE ? 0 : (int)step, 0, 0);
+          EDGE && b ? (int)(boff + (uint32_t)(16 * LDB * 2)) : (int)boff,
+          !EDGE && b ? (int)(16 * LDB * 2) : 0, 0, 0);
     }
   };
 
