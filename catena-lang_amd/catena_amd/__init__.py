@@ -123,6 +123,8 @@ SIGNATURES = {
     "catena_pool_trim": (_int, []),
     "catena_mi355x_gemm_f32_exact": (_int, [_vp, _vp, _vp, _u64, _u64, _u64]),
     "catena_mi355x_gemm_bf16": (_int, [_vp, _vp, _vp, _u64, _u64, _u64, _int]),
+    "catena_mi355x_gemm_bf16_plan": (_int, [_u64, _u64, _u64, ctypes.POINTER(_u32), ctypes.POINTER(_u64),
+                                            ctypes.POINTER(_u32), ctypes.POINTER(_u32)]),
     "catena_mi355x_gemm_bf16_argmax": (_int, [_vp, _vp, _vp, _vp, _u64, _u64, _u64]),
     "catena_mi355x_gemm_bf16_decode_plan": (_int, [_u64, _u64, _u64, ctypes.POINTER(_u32),
                                                    ctypes.POINTER(_u64)]),
@@ -319,6 +321,15 @@ def gemm_f32_exact(a, b, c, n: int, m: int, k: int) -> None:
 
 def gemm_bf16(a, b, c, n: int, m: int, k: int, out_f32: bool = False) -> None:
     check(lib().catena_mi355x_gemm_bf16(_p(a), _p(b), _p(c), n, m, k, 1 if out_f32 else 0))
+
+
+def gemm_bf16_plan(n: int, m: int, k: int):
+    """(k groups, k of a group, tile rows, tile columns) of gemm_bf16 for this
+    shape; needs no device."""
+    groups, group_k, rows, cols = _u32(), _u64(), _u32(), _u32()
+    check(lib().catena_mi355x_gemm_bf16_plan(n, m, k, ctypes.byref(groups), ctypes.byref(group_k),
+                                             ctypes.byref(rows), ctypes.byref(cols)))
+    return groups.value, group_k.value, rows.value, cols.value
 
 
 def gemm_bf16_argmax(a, b, c, idx, n: int, m: int, k: int) -> None:

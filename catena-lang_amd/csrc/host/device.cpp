@@ -58,6 +58,8 @@ const KernelSpec kKernels[] = {
     {KernelId::GemmF32ExactQ16, "gemm_f32_exact", "catena_gemm_f32_exact_q16"},
     {KernelId::GemmBf16EdgeBf16, "gemm_bf16", "catena_gemm_bf16_edge_bf16out"},
     {KernelId::GemmBf16EdgeF32, "gemm_bf16", "catena_gemm_bf16_edge_f32out"},
+    {KernelId::GemmBf16EdgeGroupsBf16, "gemm_bf16", "catena_gemm_bf16_edge_groups_bf16out"},
+    {KernelId::GemmBf16EdgeGroupsF32, "gemm_bf16", "catena_gemm_bf16_edge_groups_f32out"},
     {KernelId::GemmBf16Any192x128F32, "gemm_bf16_any", "catena_gemm_bf16_any_192x128_f32out"},
     {KernelId::GemmBf16Any192x128Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_192x128_bf16out"},
     {KernelId::GemmBf16Any128x192F32, "gemm_bf16_any", "catena_gemm_bf16_any_128x192_f32out"},
@@ -72,6 +74,10 @@ const KernelSpec kKernels[] = {
     {KernelId::GemmBf16Any32x64Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_32x64_bf16out"},
     {KernelId::GemmBf16Any32x32F32, "gemm_bf16_any", "catena_gemm_bf16_any_32x32_f32out"},
     {KernelId::GemmBf16Any32x32Bf16, "gemm_bf16_any", "catena_gemm_bf16_any_32x32_bf16out"},
+    {KernelId::GemmBf16Any64x64SeqF32, "gemm_bf16_any", "catena_gemm_bf16_any_64x64_seq_f32out"},
+    {KernelId::GemmBf16Any64x64SeqBf16, "gemm_bf16_any", "catena_gemm_bf16_any_64x64_seq_bf16out"},
+    {KernelId::GemmBf16Any32x32SeqF32, "gemm_bf16_any", "catena_gemm_bf16_any_32x32_seq_f32out"},
+    {KernelId::GemmBf16Any32x32SeqBf16, "gemm_bf16_any", "catena_gemm_bf16_any_32x32_seq_bf16out"},
     {KernelId::PackRowsBf16, "gemm_bf16_any", "catena_pack_rows_bf16"},
     {KernelId::GemmBf16K32EdgeF32, "gemm_bf16_k32", "catena_gemm_bf16_k32_edge_f32out"},
     {KernelId::GemmBf16K32EdgeBf16, "gemm_bf16_k32", "catena_gemm_bf16_k32_edge_bf16out"},

@@ -20,6 +20,8 @@ enum class KernelId : int {
   GemmF32ExactQ16,  // 16x16 tiles, A by DPP row broadcast: k % 16 == 0, m % 4 == 0
   GemmBf16EdgeBf16,  // no alignment, no scratch, any size (gemm_bf16.hip)
   GemmBf16EdgeF32,
+  GemmBf16EdgeGroupsBf16,  // the same, k groups in sequence
+  GemmBf16EdgeGroupsF32,
   GemmBf16Any192x128F32,
   GemmBf16Any192x128Bf16,
   GemmBf16Any128x192F32,
@@ -34,6 +36,10 @@ enum class KernelId : int {
   GemmBf16Any32x64Bf16,
   GemmBf16Any32x32F32,
   GemmBf16Any32x32Bf16,
+  GemmBf16Any64x64SeqF32,  // k groups in sequence
+  GemmBf16Any64x64SeqBf16,
+  GemmBf16Any32x32SeqF32,
+  GemmBf16Any32x32SeqBf16,
   PackRowsBf16,  // an operand copied to 16-byte rows (gemm_bf16_any.hip)
   GemmBf16K32EdgeF32,  // the 256 x 256 tile kernel on ragged shapes
   GemmBf16K32EdgeBf16,

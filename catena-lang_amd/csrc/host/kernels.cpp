@@ -90,6 +90,8 @@ constexpr GemmTile kGemmTiles[] = {
     {KernelId::GemmBf16K32EdgeF32, KernelId::GemmBf16K32EdgeBf16, 256, 256, 8, 4, 32, 1, 0.705, 0.705, 36.3},
 };
 constexpr int kTileRagged256 = 7;
+// the two of them that fold groups in sequence, and that form's kernels
+constexpr int kTileSeq64 = 4, kTileSeq32 = 6;
 // k groups a product may be split into (with 1: whole)
 constexpr uint32_t kGemmSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
 // row strides up to which the general kernels' 32-bit offsets reach (a stage
@@ -125,7 +127,9 @@ struct GemmPlan {
   uint32_t splits = 1;
   double us = 0;
 };
-// k > 0 when may_split (an empty fold has no groups)
+// ragged256: the 256 x 256 kernel may run (A's rows hold whole 32-k slabs, as
+// they do when k % 32 == 0 or when k % 8 != 0, which packs them).  k > 0
+// when may_split (an empty fold has no groups).
 GemmPlan gemm_plan(uint64_t n, uint64_t m, uint64_t k, bool ragged256, bool may_split) {
   GemmPlan best;
   best.us = -1;
@@ -142,6 +146,35 @@ GemmPlan gemm_plan(uint64_t n, uint64_t m, uint64_t k, bool ragged256, bool may_
     }
   }
   return best;
+}
+
+// The 32-k stage kernels need K % 128 == 0 (whole groups of 4 stages); they
+// address A's 256-row tile and B's 32-row slab with 32-bit buffer offsets.
+bool k32_stages(uint64_t m, uint64_t k) {
+  return k % 128 == 0 && k > 0 && k <= (1ull << 22) && m <= (1ull << 24);
+}
+// Shapes of whole 256-row tiles.  They are never split into k groups: their
+// order is the one the decoder's fused projections share.
+bool whole_tiles(uint64_t n, uint64_t m, uint64_t k) {
+  return k > 0 && n % 256 == 0 && ((m % 256 == 0 && k % 64 == 0) || (m % 128 == 0 && k32_stages(m, k)));
+}
+// The general kernels' 32-bit offsets reach these row strides
+bool strides_fit(uint64_t m, uint64_t k) { return k <= kGemmMaxStride && m <= kGemmMaxStride; }
+// Whole tiles that the 256-row tile kernels take when the pointers are aligned.
+// With fewer than 160 of the narrow tiles most CUs would be idle: then the
+// general kernels' smaller tiles are faster (256 x 2048 x 2048: 16 narrow tiles
+// take 38 us, 256 tiles of 32 x 64 10 us; 1024 x 6144 x 2048: 192 narrow tiles
+// and 128 x 128 tiles both 35 us).
+bool tile_kernels(uint64_t n, uint64_t m, uint64_t k) {
+  return whole_tiles(n, m, k) && !((n / 256) * ceil_div(m, 128) < 160 && strides_fit(m, k));
+}
+
+// The k groups of a general product and the tile they are folded on: what
+// fixes the order of its sums, so a function of (n, m, k) alone, never of
+// addresses, of scratch memory or of stream capture.
+GemmPlan gemm_order(uint64_t n, uint64_t m, uint64_t k, bool may_split) {
+  const bool splittable = may_split && k > 0 && n * m % 4 == 0 && strides_fit(m, k) && !whole_tiles(n, m, k);
+  return gemm_plan(n, m, k, k > 0 && (k % 32 == 0 || k % 8 != 0), splittable);
 }
 
 // Y = P[0] + P[1] + ... + P[S-1] in ascending order, f32 or bf16
@@ -389,10 +422,9 @@ int gemm_bf16_rope_qkv(const uint16_t* a, const uint16_t* w, const float* tab, c
 
 // bf16 product of any shape.  Every kernel below adds the same 32-k MFMA
 // steps in the same ascending order per output element, so which one runs
-// never changes the bits, except where a product is split into k groups
-// (f32 partials added in ascending order): ragged shapes with few tiles
-// only, never the aligned shapes, whose bits the fused projections share.
-// may_split = false keeps the one order throughout (the decoder).
+// never changes the bits.  Ragged shapes with few tiles are folded as k groups
+// whose f32 sums are added in ascending order (gemm_order); may_split = false
+// keeps the one order throughout (the decoder).
 int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_t m, uint64_t k,
               int out_f32, bool may_split) {
   int st = ensure_init();
@@ -409,33 +441,23 @@ int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_
                             DecodeEpiArgs{}, nullptr, 0);
 
   const bool ptr_ok = aligned16(a) && aligned16(b) && aligned16(c);
-  const bool tile_ok = n % 256 == 0 && m % 256 == 0 && k % 64 == 0 && k > 0 && ptr_ok;
-  // the 32-k stage kernels need K % 128 == 0 (whole groups of 4 stages);
-  // they address A's 256-row tile and B's 32-row slab with
-  // 32-bit buffer offsets
-  const bool k32_ok = k % 128 == 0 && k > 0 && k <= (1ull << 22) && m <= (1ull << 24);
-  const bool n128_ok = n % 256 == 0 && m % 128 == 0 && k32_ok && ptr_ok;
   const uint64_t tiles = ceil_div(n, 256) * ceil_div(m, 256);
   if (ceil_div(n, 256) * ceil_div(m, 128) > 0x7FFFFFFFu)
     return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
-  const bool strides_ok = k <= kGemmMaxStride && m <= kGemmMaxStride;
   // Aligned shapes: direct-to-LDS kernels (8 waves): the four-stage 32-k
   // kernel on 256 x 256 tiles, or on 256 x 128 tiles when N % 256 == 128 or
   // when that takes fewer rounds of the chip; the two-stage 64-k kernel when
-  // K % 128 != 0.  With fewer than 160 of the narrow tiles most CUs would be
-  // idle: then the general kernels' smaller tiles are faster (256 x 2048 x
-  // 2048: 16 narrow tiles take 38 us, 256 tiles of 32 x 64 10 us; 1024 x
-  // 6144 x 2048: 192 narrow tiles and 128 x 128 tiles both 35 us).
-  if ((tile_ok || n128_ok) && !((n / 256) * ceil_div(m, 128) < 160 && strides_ok)) {
+  // K % 128 != 0.
+  if (ptr_ok && tile_kernels(n, m, k)) {
     void* args[] = {&a, &b, &c, &n, &m, &k};
     KernelId id;
     size_t lds;
     uint64_t grid;
-    if (k32_ok && (!tile_ok || prefer_n128(n, m, d.cu_count))) {
+    if (k32_stages(m, k) && (m % 256 != 0 || prefer_n128(n, m, d.cu_count))) {
       id = out_f32 ? KernelId::GemmBf16K32N128F32 : KernelId::GemmBf16K32N128Bf16;
       lds = 4ull * (256 + 128) * 32 * sizeof(uint16_t);  // 98304 B
       grid = (n / 256) * (m / 128);
-    } else if (k32_ok) {
+    } else if (k32_stages(m, k)) {
       id = out_f32 ? KernelId::GemmBf16K32F32 : KernelId::GemmBf16K32Bf16;
       lds = 4ull * (256 + 256) * 32 * sizeof(uint16_t);  // 131072 B
       grid = tiles;
@@ -453,32 +475,36 @@ int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_
   // partials of k groups go there too.  Where there is no scratch -- the
   // stream is being captured (a graph would keep the address, and growing the
   // block is not allowed), the product would need too much, or the device has
-  // none left -- a product runs unsplit, or, if it needs packing, on the
-  // bounds-checked kernel of gemm_bf16.hip, which also takes strides past the
-  // 32-bit offsets here.
+  // none left -- the groups are folded in sequence, and a product that needs
+  // packing runs on the bounds-checked kernel of gemm_bf16.hip, which also
+  // takes strides past the 32-bit offsets here.  None of that changes the bits.
   const bool pack_a = k > 0 && (k % 8 != 0 || !aligned16(a));
   const bool pack_b = k > 0 && (m % 8 != 0 || !aligned16(b));
-  if (strides_ok) {
+  const GemmPlan order = gemm_order(n, m, k, may_split);
+  uint64_t k_len = order.splits > 1 ? gemm_k_len(k, order.splits, kGemmTiles[order.tile].stage_k) : k;
+  if (strides_fit(m, k)) {
     const uint64_t lda = pack_a ? ceil_div(k, 32) * 32 : k, ldb = pack_b ? ceil_div(m, 8) * 8 : m;
     const uint64_t a_bytes = pack_a ? ceil_div(n * lda * 2, 256) * 256 : 0;
     const uint64_t b_bytes = pack_b ? ceil_div(k * ldb * 2, 256) * 256 : 0;
-    const bool ragged256 = k > 0 && (k % 32 == 0 || pack_a);
-    const bool splittable = may_split && k > 0 && !tile_ok && !n128_ok && n * m % 4 == 0;
-    GemmPlan p = gemm_plan(n, m, k, ragged256, splittable);
-    uint64_t need = a_bytes + b_bytes + (p.splits > 1 ? p.splits * n * m * 4 : 0);
+    const uint64_t part_bytes = order.splits > 1 ? order.splits * n * m * 4 : 0;
     std::unique_lock<std::mutex> ws_guard(d.ws_mu, std::defer_lock);
     char* ws = nullptr;
-    if (need > 0) {
+    bool with_parts = part_bytes > 0;
+    if (a_bytes + b_bytes + part_bytes > 0) {
       hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-      const bool scratch_ok = need <= kGemmScratchMax &&
-                              hipStreamIsCapturing(d.stream, &cap) == hipSuccess &&
-                              cap == hipStreamCaptureStatusNone;
+      const bool live = hipStreamIsCapturing(d.stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
       ws_guard.lock();  // the block stays ours until everything is launched
-      void* w = nullptr;
-      if (scratch_ok && workspace(need, &w) == CATENA_OK) {
-        ws = static_cast<char*>(w);
-      } else {
-        p = gemm_plan(n, m, k, ragged256, false);
+      // with the partials, or the packed operands alone
+      for (const uint64_t need : {a_bytes + b_bytes + part_bytes, a_bytes + b_bytes}) {
+        if (live && need > 0 && need <= kGemmScratchMax) {
+          void* w = nullptr;
+          if (workspace(need, &w) == CATENA_OK) {
+            ws = static_cast<char*>(w);
+            break;
+          }
+          clear_error();  // no scratch is no failure
+        }
+        with_parts = false;
       }
     }
     if (ws || !(pack_a || pack_b)) {
@@ -493,24 +519,37 @@ int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_
         if (st) return st;
         pb = reinterpret_cast<uint16_t*>(ws + a_bytes);
       }
-      const GemmTile& t = kGemmTiles[p.tile];
+      const bool seq = order.splits > 1 && !with_parts;
+      int tile = order.tile;
+      if (seq)
+        tile = gemm_cost(kGemmTiles[kTileSeq32], n, m, k, 1) < gemm_cost(kGemmTiles[kTileSeq64], n, m, k, 1) ? kTileSeq32
+                                                                                                           : kTileSeq64;
+      const GemmTile& t = kGemmTiles[tile];
       const size_t lds = (size_t)t.stages * t.stage_k * (t.bm + t.bn) * sizeof(uint16_t);
       if (lds > d.max_lds) return fail(CATENA_ERR_UNSUPPORTED, "device LDS %zu < %zu", d.max_lds, lds);
-      const dim3 grid((unsigned)(ceil_div(n, t.bm) * ceil_div(m, t.bn)), p.splits);
-      float* parts = p.splits > 1 ? reinterpret_cast<float*>(ws + a_bytes + b_bytes) : nullptr;
+      const dim3 grid((unsigned)(ceil_div(n, t.bm) * ceil_div(m, t.bn)), with_parts ? order.splits : 1);
+      float* parts = with_parts ? reinterpret_cast<float*>(ws + a_bytes + b_bytes) : nullptr;
       void* out = parts ? parts : c;
       const bool store_f32 = out_f32 || parts;
+      KernelId id = store_f32 ? t.f32 : t.bf16;
+      if (seq && tile == kTileSeq64) id = out_f32 ? KernelId::GemmBf16Any64x64SeqF32 : KernelId::GemmBf16Any64x64SeqBf16;
+      if (seq && tile == kTileSeq32) id = out_f32 ? KernelId::GemmBf16Any32x32SeqF32 : KernelId::GemmBf16Any32x32SeqBf16;
       // four columns to a store of the general kernels, eight bf16 ones to one of the 256 x 256 kernel's
-      uint32_t vec = (parts || aligned16(c)) && m % (p.tile == kTileRagged256 && !store_f32 ? 8 : 4) == 0;
-      uint64_t k_len = p.splits > 1 ? gemm_k_len(k, p.splits, t.stage_k) : k;
+      uint32_t vec = (parts || aligned16(c)) && m % (tile == kTileRagged256 && !store_f32 ? 8 : 4) == 0;
       uint64_t sa = lda, sb = ldb;
       void* any_args[] = {&pa, &pb, &out, &n, &m, &k, &sa, &sb, &k_len, &vec};
       void* edge_args[] = {&pa, &pb, &out, &n, &m, &k, &sa, &sb, &vec};
-      st = launch(store_f32 ? t.f32 : t.bf16, grid, dim3(64 * t.waves), lds,
-                  p.tile == kTileRagged256 ? edge_args : any_args);
+      st = launch(id, grid, dim3(64 * t.waves), lds, tile == kTileRagged256 ? edge_args : any_args);
       if (st || !parts) return st;
-      return reduce_parts(parts, p.splits, n * m, c, !out_f32);
+      return reduce_parts(parts, order.splits, n * m, c, !out_f32);
     }
+  }
+  if (order.splits > 1) {
+    void* args[] = {&a, &b, &c, &n, &m, &k, &k_len};
+    const size_t lds = 2ull * (256 + 128) * 72 * sizeof(uint16_t);  // 110592 B
+    if (lds > d.max_lds) return fail(CATENA_ERR_UNSUPPORTED, "device LDS %zu < %zu", d.max_lds, lds);
+    return launch(out_f32 ? KernelId::GemmBf16EdgeGroupsF32 : KernelId::GemmBf16EdgeGroupsBf16,
+                  dim3((unsigned)(ceil_div(n, 256) * ceil_div(m, 128))), dim3(256), lds, args);
   }
   void* args[] = {&a, &b, &c, &n, &m, &k};
   const size_t lds = 2ull * 2 * 256 * 72 * sizeof(uint16_t);  // 147456 B
@@ -746,6 +785,24 @@ int catena_mi355x_gemm_bf16_decode_plan(uint64_t n, uint64_t m, uint64_t k, uint
     return fail(CATENA_ERR_INVALID_ARGUMENT,
                 "not a decode-GEMM shape (1 <= n <= 16, m %% 8 == 0, k %% 8 == 0, k > 0)");
   *partials_bytes = decode_partials_bytes(n, m, k, k_groups);
+  return CATENA_OK;
+}
+
+int catena_mi355x_gemm_bf16_plan(uint64_t n, uint64_t m, uint64_t k, uint32_t* k_groups,
+                                 uint64_t* group_k, uint32_t* tile_rows, uint32_t* tile_cols) {
+  if (!k_groups || !group_k || !tile_rows || !tile_cols)
+    return fail(CATENA_ERR_INVALID_ARGUMENT, "null output");
+  *k_groups = 1;
+  *group_k = k;
+  *tile_rows = *tile_cols = 0;
+  if (n == 0 || m == 0 || tile_kernels(n, m, k) || !strides_fit(m, k)) return CATENA_OK;
+  const GemmPlan p = gemm_order(n, m, k, true);
+  if (p.splits > 1) {
+    *k_groups = p.splits;
+    *group_k = gemm_k_len(k, p.splits, kGemmTiles[p.tile].stage_k);
+  }
+  *tile_rows = kGemmTiles[p.tile].bm;
+  *tile_cols = kGemmTiles[p.tile].bn;
   return CATENA_OK;
 }
 

@@ -27,10 +27,14 @@
 // slab's MFMAs.  B arrives N-contiguous, but the MFMA B operand wants 8
 // consecutive k per lane, so each thread transposes an 8x8 bf16 block in
 // registers before writing it to LDS k-contiguous.
+//
+// Groups form: products that gemm_bf16_any.hip folds as k groups take the
+// same groups here, on 256 x 128 tiles, one after the other, each added to the
+// sum of those before it: the same bits.
 #include "common.h"
 
 namespace {
-constexpr int BM = 256, BN = 256, BK = 64;
+constexpr int BM = 256, BK = 64;
 constexpr int LDK = BK + 8;  // padded row (in bf16): 144 B, conflict-free b128 reads
 constexpr int TILE_ELEMS = BM * LDK;
 
@@ -56,26 +60,26 @@ CATENA_DEV void tile_of(uint32_t bid, uint32_t tiles_m, uint32_t tiles_n, uint32
 }
 
 CATENA_DEV u32x4_t load_a_chunk(const uint16_t* __restrict__ A, uint64_t M, uint64_t K,
-                                uint64_t row, uint64_t col) {
+                                uint64_t kend, uint64_t row, uint64_t col) {
   uint32_t w[4];
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
     uint32_t lo = 0, hi = 0;
-    if (row < M && col + 2 * h < K) lo = A[row * K + col + 2 * h];
-    if (row < M && col + 2 * h + 1 < K) hi = A[row * K + col + 2 * h + 1];
+    if (row < M && col + 2 * h < kend) lo = A[row * K + col + 2 * h];
+    if (row < M && col + 2 * h + 1 < kend) hi = A[row * K + col + 2 * h + 1];
     w[h] = lo | (hi << 16);
   }
   return u32x4_t{w[0], w[1], w[2], w[3]};
 }
 
-CATENA_DEV u32x4_t load_b_chunk(const uint16_t* __restrict__ B, uint64_t K, uint64_t N,
+CATENA_DEV u32x4_t load_b_chunk(const uint16_t* __restrict__ B, uint64_t kend, uint64_t N,
                                 uint64_t row, uint64_t col) {
   uint32_t w[4];
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
     uint32_t lo = 0, hi = 0;
-    if (row < K && col + 2 * h < N) lo = B[row * N + col + 2 * h];
-    if (row < K && col + 2 * h + 1 < N) hi = B[row * N + col + 2 * h + 1];
+    if (row < kend && col + 2 * h < N) lo = B[row * N + col + 2 * h];
+    if (row < kend && col + 2 * h + 1 < N) hi = B[row * N + col + 2 * h + 1];
     w[h] = lo | (hi << 16);
   }
   return u32x4_t{w[0], w[1], w[2], w[3]};
@@ -96,9 +100,12 @@ CATENA_DEV void transpose8x8(const u32x4_t in[8], u32x4_t out[8]) {
   }
 }
 
-template <bool OUT_BF16>
+// k_len: k per group (GROUPS)
+template <bool OUT_BF16, bool GROUPS>
 CATENA_DEV void gemm_bf16_body(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                               void* __restrict__ C, uint64_t M, uint64_t N, uint64_t K) {
+                               void* __restrict__ C, uint64_t M, uint64_t N, uint64_t K, uint64_t k_len) {
+  constexpr int BN = GROUPS ? 128 : 256;
+  constexpr int WJ = BN / 32;  // 16-column blocks of a wave
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   uint16_t* As = smem;                  // [2][BM][LDK]
   uint16_t* Bs = smem + 2 * TILE_ELEMS;  // [2][BN][LDK], k-contiguous per column
@@ -115,27 +122,31 @@ CATENA_DEV void gemm_bf16_body(const uint16_t* __restrict__ A, const uint16_t* _
   const uint64_t m0 = (uint64_t)tm * BM, n0 = (uint64_t)tn * BN;
 
   // A loader: chunk idx = tid + 256*e -> row idx/8, 8-col chunk idx%8
-  // B loader: thread owns the 8x8 block (k-block kb, n-block nb)
+  // B loader: thread owns the 8x8 block (k-block kb, n-block nb), if there is one
   const int kb = tid & 7, nb = tid >> 3;
 
+  const bool has_b = !GROUPS || nb < BN / 8;
+  uint64_t kend = GROUPS && k_len < K ? k_len : K;
   u32x4_t ra[8], rb[8];
   auto gload = [&](uint64_t k0) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       int idx = tid + 256 * e;
-      ra[e] = load_a_chunk(A, M, K, m0 + (idx >> 3), k0 + (idx & 7) * 8);
+      ra[e] = load_a_chunk(A, M, K, kend, m0 + (idx >> 3), k0 + (idx & 7) * 8);
     }
 #pragma unroll
-    for (int r = 0; r < 8; ++r) rb[r] = load_b_chunk(B, K, N, k0 + kb * 8 + r, n0 + nb * 8);
+    for (int r = 0; r < 8; ++r)
+      rb[r] = load_b_chunk(B, has_b ? kend : 0, N, k0 + kb * 8 + r, n0 + nb * 8);
   };
   auto lstore = [&](int buf) {
     uint16_t* as = As + buf * TILE_ELEMS;
-    uint16_t* bs = Bs + buf * TILE_ELEMS;
+    uint16_t* bs = Bs + buf * BN * LDK;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       int idx = tid + 256 * e;
       *reinterpret_cast<u32x4_t*>(as + (idx >> 3) * LDK + (idx & 7) * 8) = ra[e];
     }
+    if (!has_b) return;
     u32x4_t t[8];
     transpose8x8(rb, t);
 #pragma unroll
@@ -143,40 +154,64 @@ CATENA_DEV void gemm_bf16_body(const uint16_t* __restrict__ A, const uint16_t* _
       *reinterpret_cast<u32x4_t*>(bs + (nb * 8 + j) * LDK + kb * 8) = t[j];
   };
 
-  f32x4_t acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const uint64_t nk = (K + BK - 1) / BK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-
   const int frag_row = lane & 15;
   const int frag_k = (lane >> 4) * 8;
-  for (uint64_t it = 0; it < nk; ++it) {
-    const int cur = (int)(it & 1);
-    if (it + 1 < nk) gload((it + 1) * BK);
-    const uint16_t* as = As + cur * TILE_ELEMS + (wm * 128 + frag_row) * LDK + frag_k;
-    const uint16_t* bs = Bs + cur * TILE_ELEMS + (wn * 128 + frag_row) * LDK + frag_k;
+  f32x4_t acc[8][WJ];
+  auto fold = [&](uint64_t kbeg) {  // k in [kbeg, kend)
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      bf16x8_t af[8];
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        af[i] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(as + i * 16 * LDK + s * 32));
+      for (int j = 0; j < WJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    const uint64_t nk = (kend - kbeg + BK - 1) / BK;
+    gload(kbeg);
+    lstore(0);
+    __syncthreads();
+
+    for (uint64_t it = 0; it < nk; ++it) {
+      const int cur = (int)(it & 1);
+      if (it + 1 < nk) gload(kbeg + (it + 1) * BK);
+      const uint16_t* as = As + cur * TILE_ELEMS + (wm * 128 + frag_row) * LDK + frag_k;
+      const uint16_t* bs = Bs + cur * BN * LDK + (wn * BN / 2 + frag_row) * LDK + frag_k;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        bf16x8_t bfr = as_bf16x8(*reinterpret_cast<const u32x4_t*>(bs + j * 16 * LDK + s * 32));
+      for (int s = 0; s < 2; ++s) {
+        bf16x8_t af[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr, acc[i][j], 0, 0, 0);
+          af[i] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(as + i * 16 * LDK + s * 32));
+#pragma unroll
+        for (int j = 0; j < WJ; ++j) {
+          bf16x8_t bfr = as_bf16x8(*reinterpret_cast<const u32x4_t*>(bs + j * 16 * LDK + s * 32));
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr, acc[i][j], 0, 0, 0);
+        }
       }
+      if (it + 1 < nk) lstore(cur ^ 1);
+      __syncthreads();
     }
-    if (it + 1 < nk) lstore(cur ^ 1);
-    __syncthreads();
+  };
+  fold(0);
+  if constexpr (GROUPS) {
+    f32x4_t sum[8][WJ];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < WJ; ++j) sum[i][j] = acc[i][j];
+    for (uint64_t kbeg = k_len; kbeg < K; kbeg += k_len) {
+      kend = kbeg + k_len < K ? kbeg + k_len : K;
+      fold(kbeg);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < WJ; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sum[i][j][q] = sum[i][j][q] + acc[i][j][q];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < WJ; ++j) acc[i][j] = sum[i][j];
   }
 
   // Epilogue: lane holds rows 4*(lane/16)+q, column lane%16 of each block.
@@ -185,8 +220,8 @@ CATENA_DEV void gemm_bf16_body(const uint16_t* __restrict__ A, const uint16_t* _
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint64_t gc = n0 + wn * 128 + j * 16 + ccol;
+    for (int j = 0; j < WJ; ++j) {
+      const uint64_t gc = n0 + wn * BN / 2 + j * 16 + ccol;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const uint64_t gr = m0 + wm * 128 + i * 16 + crow + q;
@@ -201,12 +236,24 @@ CATENA_DEV void gemm_bf16_body(const uint16_t* __restrict__ A, const uint16_t* _
 }
 }  // namespace
 
+// grid = ceil(M / 256) ceil(N / 256), dynamic LDS 147456 B
 #define CATENA_GEMM_BF16_KERNEL(NAME, OUTB)                                            \
   extern "C" __global__ __launch_bounds__(256) void NAME(                            \
       const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, void* __restrict__ C, \
       uint64_t M, uint64_t N, uint64_t K) {                                          \
-    gemm_bf16_body<OUTB>(A, B, C, M, N, K);                                          \
+    gemm_bf16_body<OUTB, false>(A, B, C, M, N, K, K);                                \
   }
 
 CATENA_GEMM_BF16_KERNEL(catena_gemm_bf16_edge_bf16out, true)
 CATENA_GEMM_BF16_KERNEL(catena_gemm_bf16_edge_f32out, false)
+
+// grid = ceil(M / 256) ceil(N / 128), dynamic LDS 110592 B
+#define CATENA_GEMM_BF16_GROUPS_KERNEL(NAME, OUTB)                                     \
+  extern "C" __global__ __launch_bounds__(256) void NAME(                            \
+      const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, void* __restrict__ C, \
+      uint64_t M, uint64_t N, uint64_t K, uint64_t k_len) {                          \
+    gemm_bf16_body<OUTB, true>(A, B, C, M, N, K, k_len);                             \
+  }
+
+CATENA_GEMM_BF16_GROUPS_KERNEL(catena_gemm_bf16_edge_groups_bf16out, true)
+CATENA_GEMM_BF16_GROUPS_KERNEL(catena_gemm_bf16_edge_groups_f32out, false)

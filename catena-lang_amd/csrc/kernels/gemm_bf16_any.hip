@@ -9,7 +9,10 @@
 // tile kernels' bits, whatever tile computes it.  With splits > 1 (grid.y)
 // split z folds k in [z k_len, (z + 1) k_len) in that order into its own f32
 // partial P[z] = [M][N], and a second launch adds them in ascending z; the
-// split is a function of the shape alone.  No atomics.
+// split is a function of the shape alone.  No atomics.  The seq kernels fold
+// the same groups one after the other in one workgroup and add each to the
+// sum of those before it: the same bits where no memory for partials may be
+// taken.
 //
 // Operands: A [M] rows of stride lda, B [K] rows of stride ldb, both strides
 // multiples of 8 elements and both pointers 16-byte aligned (the host packs an
@@ -87,7 +90,7 @@ CATENA_DEV int records(int64_t n) {
   return b <= 0 ? 0 : b > 0x7FFFFFF0ll ? 0x7FFFFFF0 : (int)b;
 }
 
-template <int BM, int BN, int WM, int WN, int KS, int S, bool OUT_BF16>
+template <int BM, int BN, int WM, int WN, int KS, int S, bool OUT_BF16, bool SEQ = false>
 CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                               void* __restrict__ C, uint64_t M, uint64_t N, uint64_t K_all,
                               uint64_t lda, uint64_t ldb, uint64_t k_len, uint32_t vec) {
@@ -105,8 +108,8 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
   uint32_t tm, tn;
   tile_of(blockIdx.x, (uint32_t)((M + BM - 1) / BM), (uint32_t)((N + BN - 1) / BN), tm, tn);
   const uint64_t m0 = (uint64_t)tm * BM, n0 = (uint64_t)tn * BN;
-  const uint64_t kbeg = (uint64_t)blockIdx.y * k_len;
-  const int64_t kend = (int64_t)(kbeg + k_len < K_all ? kbeg + k_len : K_all);
+  uint64_t kbeg = SEQ ? 0 : (uint64_t)blockIdx.y * k_len;
+  int64_t kend = (int64_t)(kbeg + k_len < K_all ? kbeg + k_len : K_all);
 
   // Load l of a wave: A load x = wave LA + l is rows 16 (x % A_INS) .. +15 of
   // slab x / A_INS; B load x = wave LB + l rows BR (x % B_INS) .. of slab
@@ -169,45 +172,64 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
   }
 
   f32x4_t acc[WI][WJ];
+  f32x4_t sum[SEQ ? WI : 1][SEQ ? WJ : 1];  // of the groups before this one
+  for (;;) {
 #pragma unroll
-  for (int i = 0; i < WI; ++i)
+    for (int i = 0; i < WI; ++i)
 #pragma unroll
-    for (int j = 0; j < WJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < WJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int64_t kspan = kend - (int64_t)kbeg;
-  const uint64_t nt = kspan > 0 ? (uint64_t)(kspan + KS * BK - 1) / (KS * BK) : 0;
+    const int64_t kspan = kend - (int64_t)kbeg;
+    const uint64_t nt = kspan > 0 ? (uint64_t)(kspan + KS * BK - 1) / (KS * BK) : 0;
 #pragma unroll
-  for (int t = 0; t < S - 1; ++t) issue((int64_t)kbeg + t * KS * BK, t);
-  int buf = 0;
-  for (uint64_t t = 0; t < nt; ++t) {
-    CATENA_WAIT_VMCNT(LOADS * (S - 2));  // this wave's loads of stage t have landed
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();        // every wave's have, and stage t - 1 is read
-    asm volatile("" ::: "memory");
-    issue((int64_t)kbeg + (int64_t)(t + S - 1) * KS * BK, buf == 0 ? S - 1 : buf - 1);
-    const char* st = reinterpret_cast<const char*>(smem + buf * ST);
+    for (int t = 0; t < S - 1; ++t) issue((int64_t)kbeg + t * KS * BK, t);
+    int buf = 0;
+    for (uint64_t t = 0; t < nt; ++t) {
+      CATENA_WAIT_VMCNT(LOADS * (S - 2));  // this wave's loads of stage t have landed
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();        // every wave's have, and stage t - 1 is read
+      asm volatile("" ::: "memory");
+      issue((int64_t)kbeg + (int64_t)(t + S - 1) * KS * BK, buf == 0 ? S - 1 : buf - 1);
+      const char* st = reinterpret_cast<const char*>(smem + buf * ST);
 #pragma unroll
-    for (int u = 0; u < KS; ++u) {
-      const char* sl = st + u * (A_ST + B_ST) * 2;
-      bf16x8_t fa[WI], fb[WJ];
-#pragma unroll
-      for (int i = 0; i < WI; ++i)
-        fa[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sl + a_lds + i * 16 * BK * 2));
-#pragma unroll
-      for (int j = 0; j < WJ; ++j)
-        fb[j] = cat_bf16(__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(sl + b_lds[j][0])),
-                         __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(sl + b_lds[j][1])));
-#pragma unroll
-      for (int j = 0; j < WJ; ++j)
+      for (int u = 0; u < KS; ++u) {
+        const char* sl = st + u * (A_ST + B_ST) * 2;
+        bf16x8_t fa[WI], fb[WJ];
 #pragma unroll
         for (int i = 0; i < WI; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+          fa[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(sl + a_lds + i * 16 * BK * 2));
+#pragma unroll
+        for (int j = 0; j < WJ; ++j)
+          fb[j] = cat_bf16(__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(sl + b_lds[j][0])),
+                           __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(sl + b_lds[j][1])));
+#pragma unroll
+        for (int j = 0; j < WJ; ++j)
+#pragma unroll
+          for (int i = 0; i < WI; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+      }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the buffer is read before the next barrier
+      buf = buf + 1 == S ? 0 : buf + 1;
     }
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the buffer is read before the next barrier
-    buf = buf + 1 == S ? 0 : buf + 1;
+    CATENA_WAIT_VMCNT(0);  // no LDS writes outstanding past this point
+    if constexpr (!SEQ) {
+      break;
+    } else {
+#pragma unroll
+      for (int i = 0; i < WI; ++i)
+#pragma unroll
+        for (int j = 0; j < WJ; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[i][j][q] = sum[i][j][q] = kbeg ? sum[i][j][q] + acc[i][j][q] : acc[i][j][q];
+      kbeg += k_len;
+      if (kbeg >= K_all) break;
+      kend = (int64_t)(kbeg + k_len < K_all ? kbeg + k_len : K_all);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();  // every wave has read this group's stages
+      asm volatile("" ::: "memory");
+    }
   }
-  CATENA_WAIT_VMCNT(0);  // no LDS writes outstanding past this point
 
   // acc[i][j] lane (G, s) holds C[row 16 i + s][cols 16 j + 4G .. +3]; vec: N
   // and C's address let four columns be stored at once
@@ -229,7 +251,7 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
             if (gc + q < N) c[q] = (uint16_t)f32_to_bf16_bits(v[q]);
         }
       } else {
-        float* c = static_cast<float*>(C) + ((uint64_t)blockIdx.y * M + gr) * N + gc;
+        float* c = static_cast<float*>(C) + ((SEQ ? 0 : (uint64_t)blockIdx.y * M) + gr) * N + gc;
         if (vec) {
           if (gc < N) *reinterpret_cast<f32x4_t*>(c) = v;
         } else {
@@ -243,26 +265,29 @@ CATENA_DEV void gemm_any_body(const uint16_t* __restrict__ A, const uint16_t* __
 }
 }  // namespace
 
-// grid (tiles, splits), block 64 WM WN, dynamic LDS S KS (BM + BN) 64 B
-#define CATENA_GEMM_ANY(NAME, BM, BN, WM, WN, KS, S)                                                     \
+// grid (tiles, splits), or tiles where SEQ; block 64 WM WN, dynamic LDS S KS (BM +
+// BN) 64 B
+#define CATENA_GEMM_ANY(NAME, SEQ, BM, BN, WM, WN, KS, S)                                                \
   extern "C" __global__ __launch_bounds__(64 * WM * WN) void catena_gemm_bf16_any_##NAME##_f32out(       \
       const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, void* __restrict__ C, uint64_t M,  \
       uint64_t N, uint64_t K, uint64_t lda, uint64_t ldb, uint64_t k_len, uint32_t vec) {                \
-    gemm_any_body<BM, BN, WM, WN, KS, S, false>(A, B, C, M, N, K, lda, ldb, k_len, vec);                 \
+    gemm_any_body<BM, BN, WM, WN, KS, S, false, SEQ>(A, B, C, M, N, K, lda, ldb, k_len, vec);            \
   }                                                                                                      \
   extern "C" __global__ __launch_bounds__(64 * WM * WN) void catena_gemm_bf16_any_##NAME##_bf16out(      \
       const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, void* __restrict__ C, uint64_t M,  \
       uint64_t N, uint64_t K, uint64_t lda, uint64_t ldb, uint64_t k_len, uint32_t vec) {                \
-    gemm_any_body<BM, BN, WM, WN, KS, S, true>(A, B, C, M, N, K, lda, ldb, k_len, vec);                  \
+    gemm_any_body<BM, BN, WM, WN, KS, S, true, SEQ>(A, B, C, M, N, K, lda, ldb, k_len, vec);             \
   }
 
-CATENA_GEMM_ANY(192x128, 192, 128, 2, 2, 2, 2)
-CATENA_GEMM_ANY(128x192, 128, 192, 2, 2, 2, 2)
-CATENA_GEMM_ANY(128x128, 128, 128, 2, 2, 2, 2)
-CATENA_GEMM_ANY(64x128, 64, 128, 2, 2, 2, 3)
-CATENA_GEMM_ANY(64x64, 64, 64, 2, 2, 4, 2)
-CATENA_GEMM_ANY(32x64, 32, 64, 1, 4, 4, 6)
-CATENA_GEMM_ANY(32x32, 32, 32, 2, 2, 4, 4)
+CATENA_GEMM_ANY(192x128, false, 192, 128, 2, 2, 2, 2)
+CATENA_GEMM_ANY(128x192, false, 128, 192, 2, 2, 2, 2)
+CATENA_GEMM_ANY(128x128, false, 128, 128, 2, 2, 2, 2)
+CATENA_GEMM_ANY(64x128, false, 64, 128, 2, 2, 2, 3)
+CATENA_GEMM_ANY(64x64, false, 64, 64, 2, 2, 4, 2)
+CATENA_GEMM_ANY(32x64, false, 32, 64, 1, 4, 4, 6)
+CATENA_GEMM_ANY(32x32, false, 32, 32, 2, 2, 4, 4)
+CATENA_GEMM_ANY(64x64_seq, true, 64, 64, 2, 2, 4, 2)
+CATENA_GEMM_ANY(32x32_seq, true, 32, 32, 2, 2, 4, 4)
 
 // An operand whose rows do not start on 16 bytes, copied to rows of ld
 // elements (a multiple of 8) with zeros past its columns: dst[r][0 .. ld).

@@ -114,9 +114,24 @@ int catena_mi355x_gemm_f32_exact(const float *a, const float *b, float *c, uint6
  * accumulation on MFMA in a fixed order, output bf16 (RNE) or f32 when
  * out_f32 != 0.  Same contraction as above, extended to bf16 (no reference
  * counterpart: catena has no bf16, catena-lang/src/codegen/lower_types.rs:13-22).
- * n <= 16 (decode shape) uses the weight-streaming kernel (both outputs). */
+ * n <= 16 (decode shape) uses the weight-streaming kernel (both outputs) when
+ * m % 8 == 0, k % 8 == 0 and the pointers are 16-byte aligned.  Any other
+ * product is one ascending fold of 32-k MFMA steps per element, or, where few
+ * output tiles meet a deep k, a few such folds over consecutive k ranges whose
+ * f32 sums are added in ascending order (catena_mi355x_gemm_bf16_plan); its
+ * bits do not depend on the pointers or on whether the call is captured into
+ * a graph. */
 int catena_mi355x_gemm_bf16(const uint16_t *a, const uint16_t *b, void *c, uint64_t n,
                             uint64_t m, uint64_t k, int out_f32);
+
+/* How catena_mi355x_gemm_bf16 folds a product that is not the weight-streaming
+ * kernel's: the number of k groups (1: one fold), the k of each group but the
+ * last, and the rows and columns of the output tile a workgroup owns (0 when
+ * the aligned 256-row tile kernels or, for m or k past 2^22, the kernel with
+ * 64-bit addressing takes it).  A function of (n, m, k) alone; needs no
+ * device.  No reference counterpart. */
+int catena_mi355x_gemm_bf16_plan(uint64_t n, uint64_t m, uint64_t k, uint32_t *k_groups,
+                                 uint64_t *group_k, uint32_t *tile_rows, uint32_t *tile_cols);
 
 /* The k split of the decode-shape GEMM (1 <= n <= 16, m % 8 == 0, k % 8 ==
  * 0): the number of k groups whose f32 partials are added in ascending

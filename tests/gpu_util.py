@@ -1,4 +1,6 @@
 """Helpers shared by the GPU parity tests (not collected by pytest)."""
+import ctypes
+import re
 import sys
 
 import numpy as np
@@ -57,3 +59,28 @@ def gemm_within_bound(a16: np.ndarray, b16: np.ndarray, got32: np.ndarray) -> fl
     ratio = float((err / np.maximum(bound, 1e-300)).max())
     assert np.all(err <= bound), ratio
     return ratio
+
+
+def _hip():
+    """The HIP runtime that the library has loaded."""
+    return ctypes.CDLL(re.search(r"\S+/libamdhip64\.so\S*", open("/proc/self/maps").read()).group())
+
+
+def captured(fn):
+    """`fn`'s launches as a graph of the library's stream: a function that
+    replays it."""
+    hip, vp = _hip(), ctypes.c_void_p
+    ca.synchronize()
+    stream, graph, run = vp(ca.stream()), vp(), vp()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # thread-local mode
+    try:
+        fn()
+    finally:
+        st = hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+    assert st == 0 and graph.value
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    hip.hipGraphDestroy(graph)
+
+    def replay():
+        assert hip.hipGraphLaunch(run, stream) == 0
+    return replay

@@ -159,6 +159,27 @@ def test_decode_split_depends_on_shape_only():
         ca.gemm_bf16_decode_plan(4, 100, 128)
 
 
+def test_product_order_depends_on_shape_only():
+    """The k groups of a bf16 product are a function of (n, m, k): no device is
+    initialised here.  Whole tiles are one fold, so is a product without k or
+    whose output does not fill groups of four."""
+    for n, m, k in [(32, 32, 0), (8, 128, 0), (256, 256, 0), (256, 256, 8192), (256, 384, 8192), (512, 768, 4160),
+                    (4096, 4096, 4096), (17, 255, 8192), (1000, 6144, 2048), (17, 8, (1 << 22) + 64)]:
+        assert ca.gemm_bf16_plan(n, m, k)[:2] == (1, k), (n, m, k)
+    cases = {(64, 4096, 11008): (8, 1408), (17, 256, 8192): (16, 512), (64, 64, 1 << 22): (16, 1 << 18)}
+    for (n, m, k), want in cases.items():
+        assert ca.gemm_bf16_plan(n, m, k)[:2] == want, (n, m, k)
+    # whole 32-k MFMA steps per group, and the last group is not empty
+    for n in (17, 24, 64, 100, 300):
+        for m in (60, 1024, 4096):
+            for k in (1, 7, 512, 4099, 11008, 20000):
+                groups, group_k, rows, cols = ca.gemm_bf16_plan(n, m, k)
+                assert (groups == 1 and group_k == k) or (group_k % 32 == 0 and (groups - 1) * group_k < k <= groups * group_k)
+                assert rows and cols
+    # the tile kernels' own shapes, and strides past 32-bit offsets, name no tile
+    assert ca.gemm_bf16_plan(4096, 4096, 4096)[2:] == (0, 0) == ca.gemm_bf16_plan(17, 8, (1 << 22) + 64)[2:]
+
+
 def test_sum_rows_longer_than_the_fold_bound_are_rejected():
     """sum-f32 / mean-f32 rows are folded in 32-bit chunks of 2048 values:
     rows past 0xFFFFF800 elements are refused before any device call (the

@@ -6,7 +6,7 @@ import pytest
 
 import catena_amd as ca
 import oracle
-from gpu_util import as_f32, gemm_within_bound, say
+from gpu_util import as_f32, captured, gemm_within_bound, say
 
 pytestmark = pytest.mark.gpu
 
@@ -60,7 +60,7 @@ def _check(n, m, k, shifts=(0, 0, 0)):
     (127, 248, 512), (129, 264, 1032), (255, 520, 96), (257, 256, 160), (513, 1032, 1000), (1000, 2056, 72),
     (700, 3000, 232), (1, 1, 1), (3, 7, 1000), (16, 9, 64), (5, 64, 9), (40, 33, 31), (100, 127, 129),
     (257, 511, 255), (300, 1000, 2), (643, 10944, 136), (766, 11050, 137), (965, 10944, 136), (967, 10947, 129),
-    (20, 4096, 3), (256, 256, 128), (256, 384, 256), (512, 512, 640)])
+    (20, 4096, 3), (256, 256, 128), (256, 384, 256), (512, 512, 640), (48, 4096, 2888)])
 def test_general_shapes(n, m, k):
     _check(n, m, k)
 
@@ -72,6 +72,7 @@ def test_general_shapes(n, m, k):
                                    (1040, 10990, 33), (1537, 7681, 47), (1537, 7552, 49), (1281, 6138, 81),
                                    (1025, 11007, 64), (1025, 7432, 96)])
 def test_ragged_256_tile(n, m, k):
+    assert ca.gemm_bf16_plan(n, m, k)[2:] == (256, 256)
     # what the packed operands of a longer product leave in the scratch memory:
     # a row read past one of this product's shows as a NaN
     nan = np.full((n, k + 39), NAN16, np.uint16), np.full((k + 39, m), NAN16, np.uint16)
@@ -81,14 +82,17 @@ def test_ragged_256_tile(n, m, k):
 
 @pytest.mark.parametrize("shifts", [(1, 0, 0), (0, 1, 0), (0, 0, 1)])
 def test_ragged_256_tile_unaligned(shifts):
+    assert ca.gemm_bf16_plan(1025, 7432, 96)[2:] == (256, 256)
     _check(1025, 7432, 96, shifts)
 
 
 # few tiles and a deep k: folded as 2 .. 16 k groups, the last one shorter
-@pytest.mark.parametrize("n,m,k", [(17, 256, 8192), (24, 96, 4104), (48, 4096, 2888), (64, 512, 8200), (100, 1024, 5000),
-                                   (33, 64, 16384), (20, 60, 4099)])
+@pytest.mark.parametrize("n,m,k", [(17, 256, 8192), (24, 96, 4104), (48, 2048, 2888), (64, 512, 8200), (100, 1024, 5000),
+                                   (33, 64, 16384), (20, 60, 4099), (48, 4096, 6024), (999, 2048, 5632)])
 def test_k_groups(n, m, k):
+    assert ca.gemm_bf16_plan(n, m, k)[0] > 1
     _check(n, m, k)
+    _check(n, m, k, (0, 0, 1))  # the groups' sum stored by the element
 
 
 # every address a caller may pass: 2, 4 and 8-byte aligned operands and outputs
@@ -148,3 +152,77 @@ def test_empty_fold(n, m, out_f32):
     raw = cb.read(np.uint8)
     assert not raw[256:-256].any()
     assert np.all(raw[:256] == 0xA5) and np.all(raw[-256:] == 0xA5)
+
+
+# whole tiles (one fold), k groups, the 256 x 256 tile, packed operands
+ORDERED = [(256, 256, 8192), (512, 768, 4160), (17, 256, 8192), (64, 512, 8200), (100, 1024, 5000), (20, 60, 4099),
+           (40, 777, 2072), (999, 2048, 5632), (1025, 7432, 96)]
+
+
+@pytest.mark.parametrize("n,m,k", ORDERED)
+def test_same_bits_at_any_address(n, m, k):
+    """The order of a sum is the shape's, not the pointers'."""
+    say(f"bf16 gemm at several addresses {n}x{m}x{k} plan {ca.gemm_bf16_plan(n, m, k)}")
+    a16, b16 = _inputs(n, m, k, n + m + k)
+    want = _product(a16, b16, True)
+    gemm_within_bound(a16, b16, want)
+    want16 = oracle.f32_to_bf16_bits_np(want)
+    for shifts in [(1, 0, 0), (0, 1, 0), (0, 0, 1), (4, 4, 1), (5, 3, 2)]:
+        assert np.array_equal(_product(a16, b16, True, shifts).view(np.uint32), want.view(np.uint32)), shifts
+        assert np.array_equal(_product(a16, b16, False, shifts), want16), shifts
+
+
+@pytest.mark.parametrize("n,m,k", ORDERED)
+@pytest.mark.parametrize("shifts", [(0, 0, 0), (1, 0, 0), (3, 5, 1)])
+@pytest.mark.parametrize("out_f32", [True, False])
+def test_captured_bits_equal_eager(n, m, k, shifts, out_f32):
+    """A graph takes no scratch memory: groups fold in sequence, unaligned
+    operands on the kernel that loads by the element; the bits are the same, on
+    every replay, whatever eager products do to the scratch in between."""
+    say(f"bf16 gemm captured {n}x{m}x{k} shifts {shifts} f32 {out_f32}")
+    a16, b16 = _inputs(n, m, k, n + m + k)
+    es = 4 if out_f32 else 2
+    (_ab, ap), (_bb, bp) = _placed(a16, shifts[0]), _placed(b16, shifts[1])
+    cb, eager = (ca.Buffer.from_array(np.full(n * m * es + 64, 0xA5, np.uint8)) for _ in range(2))
+    off = es * shifts[2]
+    replay = captured(lambda: ca.gemm_bf16(ap, bp, cb.ptr + off, n, m, k, out_f32=out_f32))
+    other = _inputs(33, 1024, 4099, 1)
+    for _ in range(3):
+        replay()
+        ca.gemm_bf16(ap, bp, eager.ptr + off, n, m, k, out_f32=out_f32)
+        assert np.array_equal(cb.read(np.uint8), eager.read(np.uint8))
+        cb.write(np.full(n * m * es + 64, 0xA5, np.uint8))
+        _product(*other, True)
+
+
+def test_same_bits_without_scratch():
+    """Operands whose packed copies pass the scratch limit: the groups on the
+    kernel that loads by the element.  64 x 64 x 2^22 from aligned operands, from
+    one unaligned (packed) and from both (1 GiB and more)."""
+    n = m = 64
+    k = 1 << 22
+    say(f"bf16 gemm {n}x{m}x{k} without scratch")
+    assert ca.gemm_bf16_plan(n, m, k)[0] > 1
+    size = n * k
+    rng = np.random.default_rng(4)
+    one = oracle.f32_to_bf16_bits_np(rng.normal(0, 1, 999983).astype(np.float32))  # a prime: no two rows alike
+    a16, b16 = np.resize(one, size), np.resize(one[::-1], size)
+    flat = np.full(size + 128, NAN16, np.uint16)
+
+    def place(x, shift):
+        flat[:] = NAN16
+        flat[64 + shift:64 + shift + size] = x
+        buf = ca.Buffer.from_array(flat)
+        return buf, buf.ptr + 2 * (64 + shift)
+    out = []
+    for sa, sb in [(0, 0), (0, 1), (1, 1)]:
+        (_a, ap), (_b, bp) = place(a16, sa), place(b16, sb)
+        for es in (4, 2):
+            cb = ca.Buffer(n * m * es)
+            ca.gemm_bf16(ap, bp, cb, n, m, k, out_f32=es == 4)
+            out.append(cb.read(np.uint32 if es == 4 else np.uint16, (n, m)))
+    assert np.isfinite(out[0].view(np.float32)).all() and np.any(out[0])
+    for got in out[2::2]:
+        assert np.array_equal(got, out[0])
+    for got in out[1::2]:
+        assert np.array_equal(got, oracle.f32_to_bf16_bits_np(out[0].view(np.float32)))
