@@ -205,6 +205,22 @@ uint64_t size_class(uint64_t len) {
 }
 }  // namespace
 
+// Cached blocks back to the device, once nothing queued uses them
+static int release_cached() {
+  int st = hip_check(hipStreamSynchronize(device().stream), "hipStreamSynchronize");
+  if (st) return st;
+  Pool& p = pool();
+  std::lock_guard<std::mutex> g(p.mu);
+  for (auto& kv : p.free_lists) {
+    for (void* ptr : kv.second) {
+      hipFree(ptr);
+      p.bytes_cached -= kv.first;
+    }
+    kv.second.clear();
+  }
+  return CATENA_OK;
+}
+
 int pool_alloc(uint64_t len, void** out) {
   *out = nullptr;
   if (len == 0) return CATENA_OK;
@@ -228,7 +244,7 @@ int pool_alloc(uint64_t len, void** out) {
   hipError_t e = hipMalloc(&ptr, cls);
   if (e != hipSuccess) {
     // one retry after releasing cached blocks
-    catena_pool_trim();
+    release_cached();
     e = hipMalloc(&ptr, cls);
     if (e != hipSuccess)
       return fail(CATENA_ERR_OUT_OF_MEMORY, "hipMalloc(%llu): %s", (unsigned long long)cls,
@@ -263,28 +279,25 @@ uint64_t pool_capacity(void* ptr) {
   return it == p.live.end() ? 0 : it->second;
 }
 
-// Library-held scratch (split-K partials): grown on demand, never shrunk
-// while the library is loaded.  The caller holds Device::ws_mu until it has
+// Library-held scratch, grown on demand.  The caller holds Device::ws_mu until it has
 // enqueued the launch that uses the block.
-int workspace(uint64_t bytes, void** out) {
-  Device& d = device();
-  if (bytes <= d.ws_bytes) {
-    *out = d.ws;
+int workspace(Device::Scratch& ws, uint64_t bytes, void** out) {
+  if (bytes <= ws.bytes) {
+    *out = ws.p;
     return CATENA_OK;
   }
-  if (d.ws) {
+  if (ws.p) {
     // queued kernels may still read the old block: wait before releasing it
-    int st = hip_check(hipStreamSynchronize(d.stream), "hipStreamSynchronize");
+    int st = hip_check(hipStreamSynchronize(device().stream), "hipStreamSynchronize");
     if (st) return st;
-    pool_free(d.ws);
-    d.ws = nullptr;
-    d.ws_bytes = 0;
+    pool_free(ws.p);
+    ws = Device::Scratch{};
   }
   void* p = nullptr;
   int st = pool_alloc(bytes, &p);
   if (st) return st;
-  d.ws = p;
-  d.ws_bytes = size_class(bytes);
+  ws.p = p;
+  ws.bytes = size_class(bytes);
   *out = p;
   return CATENA_OK;
 }
@@ -383,9 +396,10 @@ int catena_mi355x_shutdown(void) {
   const int st = hip_check(hipStreamSynchronize(d.stream), "hipStreamSynchronize");
   {
     std::lock_guard<std::mutex> ws(d.ws_mu);
-    if (d.ws) pool_free(d.ws);
-    d.ws = nullptr;
-    d.ws_bytes = 0;
+    for (Device::Scratch* s : {&d.ws_decode, &d.ws_general}) {
+      if (s->p) pool_free(s->p);
+      *s = Device::Scratch{};
+    }
   }
   catena_pool_trim();  // cached blocks go back to the device
   d.ready.store(false, std::memory_order_release);
@@ -470,18 +484,12 @@ int catena_pool_stats(uint64_t* bytes_live, uint64_t* bytes_cached, uint64_t* de
 int catena_pool_trim(void) {
   Device& d = device();
   if (!d.ready.load(std::memory_order_acquire)) return CATENA_OK;
-  int st = hip_check(hipStreamSynchronize(d.stream), "hipStreamSynchronize");
-  if (st) return st;
-  Pool& p = pool();
-  std::lock_guard<std::mutex> g(p.mu);
-  for (auto& kv : p.free_lists) {
-    for (void* ptr : kv.second) {
-      hipFree(ptr);
-      p.bytes_cached -= kv.first;
-    }
-    kv.second.clear();
+  {
+    std::lock_guard<std::mutex> ws(d.ws_mu);  // no call is between taking the block and its launch
+    if (d.ws_general.p) pool_free(d.ws_general.p);
+    d.ws_general = Device::Scratch{};
   }
-  return CATENA_OK;
+  return release_cached();
 }
 
 }  // extern "C"

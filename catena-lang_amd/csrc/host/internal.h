@@ -117,8 +117,15 @@ struct Device {
   static constexpr int kMaxModules = 32;
   hipModule_t modules[kMaxModules] = {};
   int n_modules = 0;
-  void* ws = nullptr;  // split-K partials
-  uint64_t ws_bytes = 0;
+  // Library-held blocks, each grown on demand.  Decode: the decode GEMM's split-K
+  // partials, whose address a captured graph may hold, so it moves only for a
+  // larger decode GEMM.  General: packed operands and partials of the other
+  // bf16 products, at most 1 GiB; no graph holds it, and catena_pool_trim gives
+  // it back.
+  struct Scratch {
+    void* p = nullptr;
+    uint64_t bytes = 0;
+  } ws_decode, ws_general;
   // Zeroed once at init; kernels that take completion tickets return their
   // counters to zero.  Layout: kTicketsGemm column-block counters,
   // kTicketsRows row counters, kTicketsMisc single counters, then
@@ -218,7 +225,7 @@ int launch(KernelId id, dim3 grid, dim3 block, size_t lds, void** args);
 int pool_alloc(uint64_t len, void** out);
 int pool_free(void* ptr);
 uint64_t pool_capacity(void* ptr);
-int workspace(uint64_t bytes, void** out);
+int workspace(Device::Scratch& ws, uint64_t bytes, void** out);
 
 // catena_mi355x_gemm_bf16 (kernels.cpp); may_split: the product may be folded
 // as k groups whose partials are added (another order of the same sum).

@@ -276,7 +276,7 @@ int gemm_bf16_decode(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, 
       P = static_cast<float*>(scratch);
     } else {
       void* ws = nullptr;
-      st = workspace(pbytes, &ws);
+      st = workspace(d.ws_decode, pbytes, &ws);
       if (st) return st;
       P = static_cast<float*>(ws);
     }
@@ -498,7 +498,7 @@ int gemm_bf16(const uint16_t* a, const uint16_t* b, void* c, uint64_t n, uint64_
       for (const uint64_t need : {a_bytes + b_bytes + part_bytes, a_bytes + b_bytes}) {
         if (live && need > 0 && need <= kGemmScratchMax) {
           void* w = nullptr;
-          if (workspace(need, &w) == CATENA_OK) {
+          if (workspace(d.ws_general, need, &w) == CATENA_OK) {
             ws = static_cast<char*>(w);
             break;
           }

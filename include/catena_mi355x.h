@@ -95,7 +95,8 @@ int catena_mem_free(catena_mem_t *mem);
 int catena_mem_write(catena_mem_t mem, uint64_t offset, const void *src, uint64_t len);
 int catena_mem_read(catena_mem_t mem, uint64_t offset, void *dst, uint64_t len);
 int catena_pool_stats(uint64_t *bytes_live, uint64_t *bytes_cached, uint64_t *device_allocs);
-/* Release every cached (free) block back to the device. */
+/* Release every cached (free) block, and the scratch memory that bf16 products
+ * of ragged or unaligned operands have taken, back to the device. */
 int catena_pool_trim(void);
 
 /* ------------------------------------------------------------------ */

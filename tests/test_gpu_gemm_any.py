@@ -226,3 +226,41 @@ def test_same_bits_without_scratch():
         assert np.array_equal(got, out[0])
     for got in out[1::2]:
         assert np.array_equal(got, oracle.f32_to_bf16_bits_np(out[0].view(np.float32)))
+
+
+def test_scratch_is_given_back():
+    """Packed operands sit in a block of their own, which catena_pool_trim
+    returns; the next product takes a new one."""
+    n, m, k = 70, 2049, 4099
+    a16, b16 = _inputs(n, m, k, 11)
+    want = _product(a16, b16, True)
+    say("scratch given back")
+    live = ca.pool_stats()["bytes_live"]
+    ca.lib().catena_pool_trim()
+    assert ca.pool_stats()["bytes_live"] <= live - k * m * 2
+    assert ca.pool_stats()["bytes_cached"] == 0
+    assert np.array_equal(_product(a16, b16, True).view(np.uint32), want.view(np.uint32))
+
+
+def test_captured_decode_product_outlives_larger_products():
+    """A graph of the decode GEMM holds the address of its partials: products
+    that need more scratch, and a trim, leave that block where it is."""
+    n, m, k = 8, 4096, 11008
+    assert ca.gemm_bf16_decode_plan(n, m, k)[0] > 1
+    a16, b16 = _inputs(n, m, k, 12)
+    ab, bb, cb = ca.Buffer.from_array(a16), ca.Buffer.from_array(b16), ca.Buffer(n * m * 4)
+    ca.gemm_bf16(ab, bb, cb, n, m, k, out_f32=True)  # sizes the block
+    want = cb.read(np.uint32)
+    say("decode gemm captured, larger products between replays")
+    replay = captured(lambda: ca.gemm_bf16(ab, bb, cb, n, m, k, out_f32=True))
+    big = _inputs(65, 8193, 4099, 13)
+    for _ in range(3):
+        _product(*big, True)
+        ca.lib().catena_pool_trim()
+        # what would now sit where the block was
+        held = [ca.Buffer.from_array(np.full(1 << s, 0xA5, np.uint8)) for s in range(18, 25)]
+        cb.write(np.zeros(n * m, np.float32))
+        replay()
+        assert np.array_equal(cb.read(np.uint32), want)
+        for h in held:
+            assert np.all(h.read(np.uint8) == 0xA5)
