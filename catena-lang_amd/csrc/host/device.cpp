@@ -54,6 +54,7 @@ const KernelSpec kKernels[] = {
     {KernelId::GemmF32Exact8x2, "gemm_f32_exact", "catena_gemm_f32_exact_8x2"},
     {KernelId::GemmF32Exact4x1, "gemm_f32_exact", "catena_gemm_f32_exact_4x1"},
     {KernelId::GemmF32Exact2x1, "gemm_f32_exact", "catena_gemm_f32_exact_2x1"},
+    {KernelId::GemmF32ExactT64, "gemm_f32_exact", "catena_gemm_f32_exact_t64"},
     {KernelId::GemmF32ExactT16, "gemm_f32_exact", "catena_gemm_f32_exact_t16"},
     {KernelId::GemmF32ExactQ16, "gemm_f32_exact", "catena_gemm_f32_exact_q16"},
     {KernelId::GemmBf16EdgeBf16, "gemm_bf16", "catena_gemm_bf16_edge_bf16out"},

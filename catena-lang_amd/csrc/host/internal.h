@@ -16,6 +16,7 @@ enum class KernelId : int {
   GemmF32Exact8x2 = 0,  // 8 rows x 2 columns per lane, A by scalar loads (gemm_f32_exact.hip)
   GemmF32Exact4x1,
   GemmF32Exact2x1,
+  GemmF32ExactT64,  // 64x64 tiles through LDS, any alignment and size
   GemmF32ExactT16,  // 16x16 tiles for small outputs
   GemmF32ExactQ16,  // 16x16 tiles, A by DPP row broadcast: k % 16 == 0, m % 4 == 0
   GemmBf16EdgeBf16,  // no alignment, no scratch, any size (gemm_bf16.hip)

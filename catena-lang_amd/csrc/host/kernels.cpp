@@ -571,35 +571,58 @@ int catena_mi355x_gemm_f32_exact(const float* a, const float* b, float* c, uint6
   void* args[] = {&a, &b, &c, &n, &m, &k};
   // Every cell is the same k-ascending chain in every form, so the choice
   // never changes the bits.
-  const uint64_t gx = ceil_div(m, 64), gy = ceil_div(n, 64);
-  if (gx * gy >= kDecodeSpread && (gx > 0x7FFFFFFFu || gy > 65535u))
-    return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
+  const uint64_t gx = ceil_div(m, 64), gy = ceil_div(n, 64), t64 = gx * gy, S = kDecodeSpread;
+  if (t64 >= S && (gx > 0x7FFFFFFFu || gy > 65535u)) return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
   const uint64_t t16 = ceil_div(m, 16) * ceil_div(n, 16);
   const bool words = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 3u) == 0;
+  // 16 columns or fewer: a 16 x 16 tile idles none of a wave's lanes that a form
+  // 64 or 128 columns wide does not idle too (65536 x 4 x 64: 7 us by DPP, 12 through
+  // LDS, 15 with 4 x 1, 26 with 8 x 2, 16 with 64 x 64 tiles)
+  const bool narrow = m <= 16 && k >= 32;
   // One cell per thread on 16 x 16 tiles, A by DPP row broadcast and B through
   // LDS (k % 16 == 0, 16-byte rows of B, 31-bit buffer offsets): up to 6.5 tiles
   // for each CU (1792 x 192 x 1728, 1344 tiles: 54 us against 65 with 2 x 1; 576 x
   // 1088 x 896, 2448: 47 against 42 with 4 x 1).  Else A and B both through LDS up
   // to two tiles for each CU, to three where the operands outgrow an XCD's L2,
   // which the row forms feel first (192 x 960 x 1103, 720 tiles: 36 us against 42
-  // with 2 x 1; 192 x 734 x 681, 552 tiles: 24 against 19), or when operands are
-  // not word-aligned or too wide for the offsets below.
-  if (t16 <= 13 * kDecodeSpread / 2 && k > 0 && k % 16 == 0 && m % 4 == 0 && aligned16(b) && words &&
+  // with 2 x 1; 192 x 734 x 681, 552 tiles: 24 against 19).
+  if ((t16 <= 13 * S / 2 || narrow) && k > 0 && k % 16 == 0 && m % 4 == 0 && aligned16(b) && words &&
       (n + 16) * k * 4 < (1ull << 31) && (k + 256) * m * 4 < (1ull << 31) && ceil_div(n, 16) <= 65535)
     return launch(KernelId::GemmF32ExactQ16, dim3((unsigned)ceil_div(m, 16), (unsigned)ceil_div(n, 16)), dim3(256),
                   256 * 16 * 4, args);
   const bool past_l2 = n + m > (3ull << 20) / 4 / (k > 0 ? k : 1);
-  if (t16 <= (past_l2 ? 3 : 2) * kDecodeSpread || !words || k >= (1ull << 26) || m >= (1ull << 25)) {
+  const bool small = t16 <= (past_l2 ? 3 : 2) * S || narrow;
+  // The row forms take word-aligned operands within the offsets below.
+  const bool reach = words && k < (1ull << 26) && m < (1ull << 25);
+  // 64 x 64 tiles through LDS: what the row forms cannot take, from 320 tiles on
+  // (operands off by 2 bytes, 1280 x 1280 x 512, 400 tiles: 94 us against 119 on 16 x
+  // 16; 1024^3, 256: 228 against 153; 1024 x 1024 x 64: 13 against 15), and where
+  // those are slower:
+  //   * few k, whose remainder they fold one by one behind its loads (2560 x 2560 x
+  //     15: 10.5 us against 13.0 with 8 x 2; x 24, no remainder: 13.4 against 13.5;
+  //     1280 x 1280 x 12: 5.3 against 6.3 with 4 x 1; x 16: 5.8 against 4.6), but not
+  //     below half a tile of rows (16 x 2^22 x 8: 162 against 117);
+  //   * an operand past the 256 MiB cache that the narrow side makes them read again
+  //     (131072 x 64 x 1000: 423 us against 610 with 4 x 1; 64 x 2^22 x 64: 968 against
+  //     1028), from eight tiles for each CU (20000 x 128 x 8000, 626: 1997 against 1001).
+  const bool few_k = (k < 16 && t64 >= 5 * S / 4) || (k < 32 && (k < 24 || k % 8 != 0) && t64 >= 3 * S);
+  const bool reread = t64 >= 8 * S && ((m <= 128 && n * k > (64ull << 20)) || (n <= 64 && k * m > (64ull << 20)));
+  if (reach ? !small && n > 32 && (few_k || reread) : t64 > 5 * S / 4 || (t64 >= S && k < 128))
+    return launch(KernelId::GemmF32ExactT64, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, args);
+  if (small || !reach) {
     if (t16 > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
     return launch(KernelId::GemmF32ExactT16, dim3((unsigned)t16), dim3(256), 0, args);
   }
   // Rows and columns per lane: 8 x 2 from 700 workgroups on (2.7 waves per
   // SIMD: 1800 x 1700 x 1500, 798 of them, 233 us against 243 with 4 x 1; 1500^3,
-  // 564, 197 against 172), 4 x 1 from 600 on (300 x 2000 x 500, 608: 21.6 us
-  // against 26.9 with 2 x 1; 1024 x 512 x 1024, 512: 48 against 42), else 2 x 1.
+  // 564, 197 against 172) and past 64 columns, where its second ones are not idle
+  // (65536 x 64 x 256: 88 us against 49 with 4 x 1), 4 x 1 from 600 on (300 x 2000 x
+  // 500, 608: 21.6 us against 26.9 with 2 x 1; 1024 x 512 x 1024, 512: 48 against 42),
+  // else 2 x 1.
   const uint64_t g82 = ceil_div(m, 128) * ceil_div(n, 32), g41 = gx * ceil_div(n, 16), g21 = gx * ceil_div(n, 8);
-  const KernelId id = g82 >= 700 ? KernelId::GemmF32Exact8x2 : g41 >= 600 ? KernelId::GemmF32Exact4x1
-                                                                          : KernelId::GemmF32Exact2x1;
+  const KernelId id = g82 >= 700 && m > 64 ? KernelId::GemmF32Exact8x2
+                      : g41 >= 600         ? KernelId::GemmF32Exact4x1
+                                           : KernelId::GemmF32Exact2x1;
   const uint64_t grid = id == KernelId::GemmF32Exact8x2 ? g82 : id == KernelId::GemmF32Exact4x1 ? g41 : g21;
   if (grid > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "matrix too large");
   uint32_t m32 = (uint32_t)m, k32 = (uint32_t)k;

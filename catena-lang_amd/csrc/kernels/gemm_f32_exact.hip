@@ -202,6 +202,88 @@ CATENA_GEMM_F32_ROWS(catena_gemm_f32_exact_8x2, 8, 2, 8)
 CATENA_GEMM_F32_ROWS(catena_gemm_f32_exact_4x1, 4, 1, 16)
 CATENA_GEMM_F32_ROWS(catena_gemm_f32_exact_2x1, 2, 1, 16)
 
+// The same contraction with nothing asked of the operands: any alignment, any
+// size.  A 64 x 64 output tile is staged through LDS 16 k values at a time and
+// every thread owns 4 x 4 cells.  Bound by its LDS reads, eight to 16
+// multiply-adds; with few k by the store of the output, which it makes sooner
+// than the row forms (4096 x 4096 x 7: 16.2 us, 4.2 TB/s, against 18.5), and it
+// reads each operand once per 64 rows or columns.
+namespace {
+constexpr int L_T = 64, L_K = 16;
+}
+
+extern "C" __global__ __launch_bounds__(256) void catena_gemm_f32_exact_t64(
+    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
+    uint64_t n, uint64_t m, uint64_t k) {
+  __shared__ float As[L_K][L_T + 1];
+  __shared__ float Bs[L_K][L_T];
+
+  const int tid = threadIdx.x;
+  const int tx = tid % 16;  // column group: cols tx + 16*jj
+  const int ty = tid / 16;  // row group: rows ty + 16*ii
+  const uint64_t row0 = (uint64_t)blockIdx.y * L_T;
+  const uint64_t col0 = (uint64_t)blockIdx.x * L_T;
+
+  float acc[4][4];
+#pragma unroll
+  for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) acc[ii][jj] = __uint_as_float(0u);
+
+  for (uint64_t k0 = 0; k0 < k; k0 += L_K) {
+    const int kt = (k - k0) < (uint64_t)L_K ? (int)(k - k0) : L_K;
+    // A tile: 64 rows x 16 k (row-major in A) -> As[kk][row]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      int idx = tid + 256 * e;  // 0..1023
+      int r = idx / L_K, kk = idx % L_K;
+      uint64_t gi = row0 + r;
+      float v = 0.0f;
+      if (gi < n && kk < kt) v = A[gi * k + k0 + kk];
+      As[kk][r] = v;
+    }
+    // B tile: 16 k x 64 cols -> Bs[kk][col]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      int idx = tid + 256 * e;
+      int kk = idx / L_T, c = idx % L_T;
+      uint64_t gj = col0 + c;
+      float v = 0.0f;
+      if (gj < m && kk < kt) v = B[(k0 + kk) * m + gj];
+      Bs[kk][c] = v;
+    }
+    __syncthreads();
+    // Only the kt live k-values are folded: the chain sees exactly
+    // k = 0 .. k-1 in ascending order.
+    for (int kk = 0; kk < kt; ++kk) {
+      float a[4], b[4];
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) a[ii] = As[kk][ty + 16 * ii];
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) b[jj] = Bs[kk][tx + 16 * jj];
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          float prod = a[ii] * b[jj];
+          acc[ii][jj] = acc[ii][jj] + prod;
+        }
+    }
+    __syncthreads();
+  }
+
+#pragma unroll
+  for (int ii = 0; ii < 4; ++ii) {
+    uint64_t gi = row0 + ty + 16 * ii;
+    if (gi >= n) continue;
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      uint64_t gj = col0 + tx + 16 * jj;
+      if (gj < m) C[gi * m + gj] = acc[ii][jj];
+    }
+  }
+}
+
 // The same contraction for small outputs, where whole waves of columns would
 // leave most CUs idle (256^3 is 128 workgroups of the smallest form above): a 16x16 output
 // tile per workgroup of 256 threads, one cell per thread, so 256^3 launches
