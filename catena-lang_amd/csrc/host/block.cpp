@@ -146,7 +146,13 @@ int attn_causal(const uint16_t* q, const uint16_t* k, const uint16_t* v, const u
   // kernel, give the same bits.
   //   * at most 64 blocks: one query per workgroup, since 16 times as many
   //     workgroups then still find CUs (128 queries x 8 heads over 1028 keys:
-  //     56 us against 64 in 64 blocks; 200 queries, 104 blocks: 98 against 67);
+  //     56 us against 64 in 64 blocks; 200 queries, 104 blocks: 98 against 67).
+  //     Past 1088 rows a CU holds one block, whose time falls less than in half
+  //     from 16 queries to 8, and the one-query form's grows with the queries
+  //     alone: the two meet at 1984 queries in blocks of 8 and 2560 in blocks of
+  //     16 (2048 rows, one query / blocks: 128 pairs x 8 queries 96 / 184 us, x 16
+  //     188 / 238, x 20 235 / 237, x 24 275 / 236; 256 pairs x 8 203 / 193), as long as
+  //     its scores of max_len leave a CU four workgroups;
   //   * four waves while at least three workgroups share a CU (up to 704
   //     rows) and there are more than two for each CU; eight otherwise, which
   //     finish a block sooner and keep a CU busier where two blocks or one
@@ -161,9 +167,11 @@ int attn_causal(const uint16_t* q, const uint16_t* k, const uint16_t* v, const u
     return 16 * 136 * 2 + 3 * 16 * 4 + (size_t)3 * waves * 16 * 4 + (size_t)ceil_div(rows, 64) * 64 * 17 * 4;
   };
   const uint64_t bh = (uint64_t)batch * heads, grid = bh * ceil_div(tq, 16);
-  if (tq >= 8 && grid > 64 && aligned16(q) && pf_lds(8, rows_bound) <= device().max_lds) {
+  const uint32_t nqb = (uint32_t)ceil_div(tq, 16);
+  const bool few = grid <= 64 || (rows_bound > 1088 && 4 * attn_lds_bytes(max_len) <= device().max_lds &&
+                                  bh * tq <= 1408 + 72ull * std::min(tq, 16u));
+  if (tq >= 8 && !few && aligned16(q) && pf_lds(8, rows_bound) <= device().max_lds) {
     if (grid > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "too many query blocks");
-    const uint32_t nqb = (uint32_t)ceil_div(tq, 16);
     // keys the queries before block qb may see: the last of them is followed
     // by tq - 16 qb others
     auto rows_before = [&](uint32_t qb) {

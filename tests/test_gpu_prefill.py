@@ -47,7 +47,10 @@ def _inputs(B, Tq, H, L, seed, special):
 @pytest.mark.parametrize("B,Tq,H,L,pfx", [
     (1, 257, 4, 300, 0), (2, 129, 4, 640, 400), (1, 520, 16, 704, 100), (1, 520, 16, 705, 100),
     (2, 270, 16, 704, 434), (1, 100, 10, 1088, 900), (1, 100, 10, 1089, 900), (1, 600, 16, 1100, 500),
-    (1, 300, 4, 2304, 2000), (1, 300, 4, 2305, 2000), (1, 64, 16, 90, 0), (1, 65, 16, 90, 0), (1, 1100, 8, 1150, 40)])
+    (1, 300, 4, 2304, 2000), (1, 300, 4, 2305, 2000), (1, 64, 16, 90, 0), (1, 65, 16, 90, 0), (1, 1100, 8, 1150, 40),
+    # past 1088 rows: at and past the fewest queries that take blocks
+    (1, 300, 10, 1089, 700), (1, 300, 10, 2304, 2000), (1, 64, 40, 1100, 1000), (1, 64, 41, 1100, 1000),
+    (8, 8, 31, 1200, 1100), (8, 8, 32, 1200, 1100), (4, 9, 60, 1190, 1100), (3, 33, 25, 1300, 1200), (3, 33, 26, 1300, 1200)])
 @pytest.mark.parametrize("special", [False, True])
 def test_every_form_equals_the_one_query_kernel(B, Tq, H, L, pfx, special):
     q16, k16, v16 = _inputs(B, Tq, H, L, B + Tq + H + L + pfx, special)
@@ -62,7 +65,8 @@ def test_every_form_equals_the_one_query_kernel(B, Tq, H, L, pfx, special):
     starts = sorted({0, 7, Tq // 3, Tq // 2, max(0, Tq - 23), Tq - 7})
     for t0 in starts:
         sub = np.ascontiguousarray(q16[:, t0:t0 + 7])
-        want = _causal(sub, kb, vb, [max(0, n - (Tq - 7 - t0)) for n in lens], L, True)
+        after = Tq - t0 - sub.shape[1]
+        want = _causal(sub, kb, vb, [max(0, n - after) for n in lens], L, True)
         a, b = got[:, t0:t0 + 7], want
         an, bn = np.isnan(a.view(np.float32)), np.isnan(b.view(np.float32))
         assert np.array_equal(an, bn), t0
