@@ -151,8 +151,11 @@ int attn_causal(const uint16_t* q, const uint16_t* k, const uint16_t* v, const u
   //     from 16 queries to 8, and the one-query form's grows with the queries
   //     alone: the two meet at 1984 queries in blocks of 8 and 2560 in blocks of
   //     16 (2048 rows, one query / blocks: 128 pairs x 8 queries 96 / 184 us, x 16
-  //     188 / 238, x 20 235 / 237, x 24 275 / 236; 256 pairs x 8 203 / 193), as long as
-  //     its scores of max_len leave a CU four workgroups;
+  //     188 / 238, x 20 235 / 237, x 24 275 / 236; 256 pairs x 8 203 / 193).
+  //     Both as long as the one-query workgroups, whose LDS holds max_len scores,
+  //     take two rounds of the chip at most (a one-layer prompt of 64 tokens x 16
+  //     heads in a cache of 32768 rows, one to a CU: 99 us against 91; of 33: 91 /
+  //     88; of 16: 88 / 95; of 64 in 8192 rows, three to a CU: 88 / 91);
   //   * four waves while at least three workgroups share a CU (up to 704
   //     rows) and there are more than two for each CU; eight otherwise, which
   //     finish a block sooner and keep a CU busier where two blocks or one
@@ -168,8 +171,8 @@ int attn_causal(const uint16_t* q, const uint16_t* k, const uint16_t* v, const u
   };
   const uint64_t bh = (uint64_t)batch * heads, grid = bh * ceil_div(tq, 16);
   const uint32_t nqb = (uint32_t)ceil_div(tq, 16);
-  const bool few = grid <= 64 || (rows_bound > 1088 && 4 * attn_lds_bytes(max_len) <= device().max_lds &&
-                                  bh * tq <= 1408 + 72ull * std::min(tq, 16u));
+  const bool few = bh * tq <= 2ull * (unsigned)device().cu_count * (device().max_lds / attn_lds_bytes(max_len)) &&
+                   (grid <= 64 || (rows_bound > 1088 && bh * tq <= 1408 + 72ull * std::min(tq, 16u)));
   if (tq >= 8 && !few && aligned16(q) && pf_lds(8, rows_bound) <= device().max_lds) {
     if (grid > 0x7FFFFFFFu) return fail(CATENA_ERR_UNSUPPORTED, "too many query blocks");
     // keys the queries before block qb may see: the last of them is followed

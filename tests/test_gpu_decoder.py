@@ -646,3 +646,21 @@ def test_decoder_c5_full_workload_stagewise():
     assert np.array_equal(dec.read(ca.DEC_LOGITS, np.float32).view(np.uint32),
                           final_logits.view(np.uint32))
     dec.close()
+
+
+@pytest.mark.parametrize("batch,t", [(1, 64), (3, 33), (1, 8)])
+def test_decoder_prompt_bits_do_not_depend_on_the_cache(batch, t):
+    """A short prompt takes one query per workgroup in a short cache and blocks
+    of queries in a long one, whose scores would leave a CU one workgroup."""
+    heads, vocab = 16, 1024
+    say(f"decoder prompt of {batch} x {t} tokens in caches of 128 and 20000 positions")
+    tok = np.random.default_rng(t).integers(0, vocab, (batch, t)).astype(np.uint32)
+    logits = []
+    for max_len in (128, 20000):
+        dec = ca.Decoder(128 * heads, heads, 256, 1, vocab, batch, max_len)
+        dec.init_weights(seed=3, std=0.02)
+        dec.prefill(ca.Buffer.from_array(tok), batch, t, ca.Buffer(batch * 4))
+        logits.append(dec.read(ca.DEC_LOGITS, np.uint32)[:batch * vocab])
+        dec.close()
+    assert np.array_equal(*logits)
+    assert np.isfinite(logits[0].view(np.float32)).all()
