@@ -738,17 +738,23 @@ int catena_mi355x_softmax_f32(const float* x, float* y, uint64_t rows, uint64_t 
   // six rows a CU, where three such workgroups fit one.  Measured, one against
   // four: 1024 x 2048 11.6 / 12.7 us, 2048 x 2048 21.0 / 18.7, 16384 x 512 36.1 /
   // 24.2, 4096 x 4096 58.9 / 59.4, 8192 x 6000 173 / 302.  Longer rows: one row
-  // per workgroup through memory.
+  // per workgroup through memory.  So too when LDS holds one or two rows a CU and
+  // that takes more than three rounds, since the form through memory folds eight
+  // rows a CU at a time (LDS against memory: 768 x 30000 252 / 274 us, 800 331 / 276,
+  // 4096 1439 / 950 at 32768; 1536 x 16384 152 / 164, 2048 201 / 178); two rows a CU
+  // and more than eight are its streams' time again, and LDS reads x once (8192 x
+  // 16384 792 / 870).
   const bool vec = n % 4 == 0 && aligned16(x) && aligned16(y);
   uint32_t n32 = (uint32_t)n, slot = rows4_slot(n);
   void* lds_args[] = {&x, &y, &rows, &n32, &slot};
   if (slot && rows4_per_cu(slot) >= 3 && rows >= 6ull * (unsigned)device().cu_count)
     return launch(vec ? KernelId::SoftmaxRows4Vec : KernelId::SoftmaxRows4, dim3((unsigned)ceil_div(rows, 4)),
                   dim3(256), 4 * (size_t)slot * sizeof(float), lds_args);
-  if (n <= (device().max_lds - 64) / sizeof(float)) {
+  const uint64_t row_lds = ceil_div(n, 4) * 4 * sizeof(float), cus = (unsigned)device().cu_count;
+  const uint64_t fit = device().max_lds / (row_lds + 64);
+  if (fit >= 3 || (fit > 0 && rows <= 3 * fit * cus) || (fit == 2 && rows > 8 * cus))
     return launch(vec ? KernelId::SoftmaxRowVec : KernelId::SoftmaxRow, dim3((unsigned)rows), dim3(256),
-                  ceil_div(n, 4) * 4 * sizeof(float), lds_args);
-  }
+                  row_lds, lds_args);
   void* args[] = {&x, &y, &n};
   return launch(KernelId::SoftmaxRows, dim3((unsigned)rows), dim3(256), 0, args);
 }

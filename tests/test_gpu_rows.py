@@ -58,7 +58,9 @@ def _placed(x, shift):
 # forms (40944) and the next ones
 @pytest.mark.parametrize("rows,n", [(1, 1), (3, 2), (5, 33), (9, 511), (1535, 64), (1536, 64), (1537, 65), (1541, 512),
                                     (1539, 516), (1537, 1028), (1537, 2047), (2, 9088), (3, 9089), (2, 40944),
-                                    (2, 40945)])
+                                    (2, 40945),
+                                    # one row a CU: LDS up to three rounds; two: up to three and past eight rows a CU
+                                    (768, 20448), (769, 20449), (1536, 13652), (1537, 13653), (2049, 13652)])
 @pytest.mark.parametrize("shift", [0, 4])
 def test_softmax(rows, n, shift):
     say(f"softmax rows {rows} n {n} shift {shift}")
