@@ -161,12 +161,15 @@ bool whole_tiles(uint64_t n, uint64_t m, uint64_t k) {
 // The general kernels' 32-bit offsets reach these row strides
 bool strides_fit(uint64_t m, uint64_t k) { return k <= kGemmMaxStride && m <= kGemmMaxStride; }
 // Whole tiles that the 256-row tile kernels take when the pointers are aligned.
-// With fewer than 160 of the narrow tiles most CUs would be idle: then the
-// general kernels' smaller tiles are faster (256 x 2048 x 2048: 16 narrow tiles
-// take 38 us, 256 tiles of 32 x 64 10 us; 1024 x 6144 x 2048: 192 narrow tiles
-// and 128 x 128 tiles both 35 us).
+// Up to 128 of the narrow tiles half the CUs would be idle: then the general
+// kernels' smaller tiles are faster (256 x 2048 x 2048: 16 narrow tiles take 38
+// us, 256 tiles of 32 x 64 10 us; 512 x 8192 x 4096, 128: 48 / 45; past it they are
+// not: 3328 x 1280 x 1408, 130: 22.3 / 23.3; 512 x 9728 x 768, 152: 14.0 / 16.8; 768
+// x 6272 x 128, 147: 7.9 / 9.0).  The 64-k stage kernel, on wide tiles alone, is
+// passed up to 159 (1536 x 2816 x 1600, 132: 39.5 / 25.4).
 bool tile_kernels(uint64_t n, uint64_t m, uint64_t k) {
-  return whole_tiles(n, m, k) && !((n / 256) * ceil_div(m, 128) < 160 && strides_fit(m, k));
+  const uint64_t few = k32_stages(m, k) ? 128 : 159;
+  return whole_tiles(n, m, k) && !((n / 256) * ceil_div(m, 128) <= few && strides_fit(m, k));
 }
 
 // The k groups of a general product and the tile they are folded on: what
