@@ -21,7 +21,7 @@ import pytest
 
 import catena_amd as ca
 import oracle
-from gpu_util import U, as_f32, bf16_ulp_diff, bf16_ulp_of, dev_normal_bf16, gemm_within_bound, hash_bits, say
+from gpu_util import U, as_f32, bf16_ulp_diff, bf16_ulp_of, captured, dev_normal_bf16, gemm_within_bound, hash_bits, say
 
 pytestmark = pytest.mark.gpu
 
@@ -68,8 +68,11 @@ def _check(a16, b16, got32, got16, rows=None):
     return stats
 
 
-@pytest.mark.parametrize("n,m,k", [(256, 256, 64), (512, 256, 1024), (256, 768, 320)])
-def test_tile_kernel_full_compare(n, m, k):
+# few tiles (general kernels); 256 x 256 tiles with 32-k stages; with 64-k stages
+@pytest.mark.parametrize("n,m,k,tiled", [(256, 256, 64, False), (512, 256, 1024, False), (256, 768, 320, False),
+                                         (4096, 2304, 128, True), (2560, 2048, 64, True), (2560, 2048, 192, True)])
+def test_tile_kernel_full_compare(n, m, k, tiled):
+    assert (ca.gemm_bf16_plan(n, m, k)[2:] == (0, 0)) == tiled
     say(f"bf16 gemm tile {n}x{m}x{k}")
     a, b, a16, b16 = _inputs(n, m, k, seed=100 + n + m + k)
     c32, c16 = ca.Buffer(n * m * 4), ca.Buffer(n * m * 2)
@@ -81,27 +84,34 @@ def test_tile_kernel_full_compare(n, m, k):
 
 
 def test_tile_widths_give_identical_bits():
-    """The 256 x 256 and 256 x 128 tile kernels keep the same per-accumulator
-    k32 order, so a cell's bits do not depend on which one computed it: the
-    first 512 rows of a 4096-row product (256 x 256 tiles, one per CU) equal
-    the 512-row product of the same rows (256 x 128 tiles: fewer rounds)."""
-    n, m, k = 4096, 2048, 1024
-    say(f"bf16 gemm tile widths {n}x{m}x{k} vs 512x{m}x{k}")
+    """The 256 x 256 and 256 x 128 tile kernels and the general ones keep the
+    same per-accumulator k32 order, so a cell's bits do not depend on which one
+    computed it: of 2304 columns, 4096 rows take 256 x 256 tiles (144 of them;
+    the 288 narrow ones would be two rounds of the chip), their first 2304 rows
+    alone 256 x 128 tiles (one round), their first 512 the general kernels."""
+    n, m, k = 4096, 2304, 1024
+    say(f"bf16 gemm tile widths {n}x{m}x{k} vs 2304 and 512 rows")
+    assert [ca.gemm_bf16_plan(r, m, k)[2:] == (0, 0) for r in (n, 2304, 512)] == [True, True, False]
     a, b, _, _ = _inputs(n, m, k, seed=901)
     for out_f32, dt, es in ((False, np.uint16, 2), (True, np.uint32, 4)):
-        full, part = ca.Buffer(n * m * es), ca.Buffer(512 * m * es)
+        full = ca.Buffer(n * m * es)
         ca.gemm_bf16(a, b, full, n, m, k, out_f32=out_f32)
-        ca.gemm_bf16(a, b, part, 512, m, k, out_f32=out_f32)
-        assert np.array_equal(full.read(dt, (n, m))[:512], part.read(dt, (512, m)))
+        for rows in (2304, 512):
+            part = ca.Buffer(rows * m * es)
+            ca.gemm_bf16(a, b, part, rows, m, k, out_f32=out_f32)
+            assert np.array_equal(full.read(dt, (n, m))[:rows], part.read(dt, (rows, m)))
 
 
-def test_k64_kernel_equals_k32_kernel_on_zero_padded_k():
+# 12 narrow tiles: general kernels on both sides; 160 and 320: the 64-k kernel
+# against 256 x 128 and 256 x 256 tiles
+@pytest.mark.parametrize("n,m,k", [(512, 768, 4160), (2560, 2048, 448), (5120, 2048, 192)])
+def test_k64_kernel_equals_k32_kernel_on_zero_padded_k(n, m, k):
     """K % 128 != 0 takes the two-stage 64-k kernel, K % 128 == 0 the
     four-stage 32-k kernel; both add k32 MFMA steps in ascending order, so
-    padding K = 4160 with 64 zero columns of A (and zero rows of B) to 4224
-    gives the same bits: the extra steps add exact zeros to nonzero sums."""
-    n, m, k = 512, 768, 4160
+    padding K with 64 zero columns of A (and zero rows of B) gives the same
+    bits: the extra steps add exact zeros to nonzero sums."""
     kp = k + 64
+    assert (ca.gemm_bf16_plan(n, m, k)[2:] == (0, 0)) == (n >= 2560) == (ca.gemm_bf16_plan(n, m, kp)[2:] == (0, 0))
     rng = np.random.default_rng(902)
     a32 = rng.normal(0, 1, (n, k)).astype(np.float32)
     b32 = rng.normal(0, 1, (k, m)).astype(np.float32)
@@ -119,9 +129,11 @@ def test_k64_kernel_equals_k32_kernel_on_zero_padded_k():
     assert np.array_equal(outs[0], outs[1])
 
 
-@pytest.mark.parametrize("n,m,k", [(256, 384, 256), (512, 128, 1152)])
-def test_narrow_tile_kernel_full_compare(n, m, k):
-    """N % 256 == 128: only the 256 x 128 tile kernel applies."""
+@pytest.mark.parametrize("n,m,k,tiled", [(256, 384, 256, False), (512, 128, 1152, False), (2560, 1664, 256, True)])
+def test_narrow_tile_kernel_full_compare(n, m, k, tiled):
+    """N % 256 == 128: of the tile kernels only the 256 x 128 one applies (few
+    tiles go to the general kernels)."""
+    assert (ca.gemm_bf16_plan(n, m, k)[2:] == (0, 0)) == tiled
     say(f"bf16 gemm 256x128 tiles {n}x{m}x{k}")
     a, b, a16, b16 = _inputs(n, m, k, seed=400 + n + m + k)
     c32, c16 = ca.Buffer(n * m * 4), ca.Buffer(n * m * 2)
@@ -134,12 +146,19 @@ def test_narrow_tile_kernel_full_compare(n, m, k):
 
 @pytest.mark.parametrize("n,m,k", [(1, 1, 1), (17, 9, 5), (300, 200, 100), (257, 513, 72),
                                    (64, 64, 63)])
-def test_edge_kernel_full_compare(n, m, k):
-    say(f"bf16 gemm edge {n}x{m}x{k}")
+@pytest.mark.parametrize("graph", [False, True])
+def test_edge_kernel_full_compare(n, m, k, graph):
+    """Sizes no tile divides: the general kernels, and, captured into a graph,
+    where rows off 16 bytes cannot be packed, the bounds-checked kernel."""
+    say(f"bf16 gemm edge {n}x{m}x{k} graph {graph}")
     a, b, a16, b16 = _inputs(n, m, k, seed=200 + n + m + k)
+    if graph:  # one element off 16 bytes
+        a = ca.Buffer.from_array(np.concatenate([np.zeros(1, np.uint16), a16.reshape(-1)]))
+    ap = a.ptr + 2 if graph else a
     c32, c16 = ca.Buffer(n * m * 4), ca.Buffer(n * m * 2)
-    ca.gemm_bf16(a, b, c32, n, m, k, out_f32=True)
-    ca.gemm_bf16(a, b, c16, n, m, k, out_f32=False)
+    for c in (c32, c16):
+        run = lambda: ca.gemm_bf16(ap, b, c, n, m, k, out_f32=c is c32)  # noqa: E731,B023
+        (captured(run) if graph else run)()
     g32, g16 = c32.read(np.float32, (n, m)), c16.read(np.uint16, (n, m))
     assert np.array_equal(g16, oracle.f32_to_bf16_bits_np(g32))
     _check(a16, b16, g32, g16)
@@ -243,8 +262,7 @@ def test_decode_and_tile_kernels_random_shapes():
     """Seeded random shapes through gemm_bf16: 16 decode shapes (M <= 16; N
     and K multiples of 8, so both the streamed path (K % 32 == 0) and the
     register path, ragged column blocks and one to many k groups) and 12
-    wider ones (M > 16: tile, 64-k and bounds-checked edge kernels by
-    shape), each against the oracle under the stated bound, f32 and bf16
+    wider ones (M > 16: general kernels), each against the oracle under the stated bound, f32 and bf16
     outputs consistent and bitwise run to run."""
     rng = np.random.default_rng(777)
     shapes = []

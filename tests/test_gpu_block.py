@@ -292,6 +292,28 @@ def _attn_inputs(B, Tq, H, L, seed):
     return q, k, v
 
 
+def _causal_copies(q16, k16, v16, lens, B, Tq, H, L, scale, blocks):
+    """f32 and bf16 causal attention of the problem laid side by side often
+    enough that the call has at least `blocks` blocks of 16 queries (0: once), and
+    more queries than the one-query kernel takes past 1,088 rows: up to 64 blocks
+    run on that kernel, more on the block kernel with eight waves, more than 512
+    (up to 704 rows) with four.  Every copy has the first one's bits."""
+    D, c = 128, 1
+    if blocks:
+        c = max(-(-blocks // (B * H * -(-Tq // 16))), -(-2561 // (B * H * Tq)) if L > 1088 else 1)
+    tile = lambda x, shape: np.ascontiguousarray(np.broadcast_to(x.reshape(shape), (c,) + shape))  # noqa: E731
+    q, k, v = (ca.Buffer.from_array(tile(x, s)) for x, s in ((q16, (B, Tq, H, D)), (k16, (B, H, L, D)), (v16, (B, H, L, D))))
+    lb = ca.Buffer.from_array(np.tile(np.array(lens, np.uint32), c))
+    out = []
+    for f32, dt in ((True, np.uint32), (False, np.uint16)):
+        o = ca.Buffer(c * B * Tq * H * D * (4 if f32 else 2))
+        ca.attn_causal_bf16(q, k, v, lb, o, c * B, Tq, H, L, D, scale, out_f32=f32)
+        got = o.read(dt, (c, B * Tq, H * D))
+        assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+        out.append(got[0])
+    return out[0].view(np.float32), out[1]
+
+
 @pytest.mark.parametrize("B,Tq,H,L,lens", [(2, 4, 3, 64, [10, 4]), (1, 7, 2, 300, [300]),
                                            (2, 64, 4, 512, [512, 100]), (3, 2, 1, 16, [1, 0, 16])])
 def test_attention_causal_matches_prefix_decode(B, Tq, H, L, lens):
@@ -311,9 +333,10 @@ def test_attention_causal_matches_prefix_decode(B, Tq, H, L, lens):
     _bitwise(o16.read(np.uint16, (B * Tq, H * D)), oracle.f32_to_bf16_bits_np(want))
 
 
-def test_attention_causal_random_configs():
-    """Ten seeded random causal configurations (Tq from 2 to 80, so both the
-    16-query prefill kernel and the one-query kernel run; cached prefixes
+@pytest.mark.parametrize("blocks", [0, 65, 513])
+def test_attention_causal_random_configs(blocks):
+    """Ten seeded random causal configurations (Tq from 2 to 80) on the
+    one-query kernel and on both forms of the block kernel (cached prefixes
     with lens > Tq, sequences shorter than Tq, empty ones; random scales):
     f32 output bitwise the oracle's causal attention, bf16 output its RNE."""
     D = 128
@@ -327,20 +350,18 @@ def test_attention_causal_random_configs():
             lens[0] = L
         scale = float(np.float32(rng.uniform(0.05, 0.2)))
         q, k, v = _attn_inputs(B, Tq, H, L, 900 + i)
-        lb = ca.Buffer.from_array(np.array(lens, np.uint32))
-        o32 = ca.Buffer(B * Tq * H * D * 4)
-        o16 = ca.Buffer(B * Tq * H * D * 2)
-        say(f"causal attention random config B={B} Tq={Tq} H={H} L={L} lens={lens} scale={scale}")
-        ca.attn_causal_bf16(q, k, v, lb, o32, B, Tq, H, L, D, scale, out_f32=True)
-        ca.attn_causal_bf16(q, k, v, lb, o16, B, Tq, H, L, D, scale, out_f32=False)
-        want = od.attn_causal(q.read(np.uint16), k.read(np.uint16, (B, H, L, D)),
-                              v.read(np.uint16, (B, H, L, D)), lens, B, Tq, H, D, scale)
-        _bitwise(o32.read(np.float32, (B * Tq, H * D)), want)
-        _bitwise(o16.read(np.uint16, (B * Tq, H * D)), oracle.f32_to_bf16_bits_np(want))
+        say(f"causal attention random config B={B} Tq={Tq} H={H} L={L} lens={lens} scale={scale} blocks {blocks}")
+        q16, k16, v16 = q.read(np.uint16), k.read(np.uint16, (B, H, L, D)), v.read(np.uint16, (B, H, L, D))
+        g32, g16 = _causal_copies(q16, k16, v16, lens, B, Tq, H, L, scale, blocks)
+        want = od.attn_causal(q16, k16, v16, lens, B, Tq, H, D, scale)
+        _bitwise(g32, want)
+        _bitwise(g16, oracle.f32_to_bf16_bits_np(want))
 
 
-def test_attention_causal_prefill_nan_inf_tie_scores():
-    """The 16-query prefill kernel (Tq >= 8) on scores with a NaN inside the
+@pytest.mark.parametrize("blocks", [0, 65, 513])
+def test_attention_causal_prefill_nan_inf_tie_scores(blocks):
+    """Causal attention (one query per workgroup, and both forms of the block
+    kernel) on scores with a NaN inside the
     prefix (the max restarts after it), a NaN at exactly one query's last
     position (that query's max is the NaN), an overflowing score, all-equal
     (+0) scores, and a partial last block of queries (Tq = 20)."""
@@ -355,18 +376,15 @@ def test_attention_causal_prefill_nan_inf_tie_scores():
     k32[0, 3, :, :] = 0.0          # every score +0
     k16 = oracle.f32_to_bf16_bits_np(k32)
     v16 = oracle.f32_to_bf16_bits_np(rng.normal(0, 1, (B, H, L, D)).astype(np.float32))
-    q, k, v = ca.Buffer.from_array(q16), ca.Buffer.from_array(k16), ca.Buffer.from_array(v16)
-    lb = ca.Buffer.from_array(np.array(lens, np.uint32))
     scale = 1.0 / math.sqrt(D)
-    o32 = ca.Buffer(B * Tq * H * D * 4)
-    say("causal prefill attention NaN / inf / tie scores")
-    ca.attn_causal_bf16(q, k, v, lb, o32, B, Tq, H, L, D, scale, out_f32=True)
-    want = od.attn_causal(q16, k16, v16, lens, B, Tq, H, D, scale)
-    _bitwise(o32.read(np.float32, (B * Tq, H * D)), want)
+    say(f"causal prefill attention NaN / inf / tie scores, blocks {blocks}")
+    got, _ = _causal_copies(q16, k16, v16, lens, B, Tq, H, L, scale, blocks)
+    _bitwise(got, od.attn_causal(q16, k16, v16, lens, B, Tq, H, D, scale))
 
 
-def test_attention_prefill_mfma_fold_range_guard():
-    """The prefill kernel folds q.k on the matrix cores (one rounding per
+@pytest.mark.parametrize("blocks", [0, 65, 513])
+def test_attention_prefill_mfma_fold_range_guard(blocks):
+    """The block kernel folds q.k on the matrix cores (one rounding per
     step, exact products) only while every nonzero q / k magnitude is in
     [2^-63, 2^63); otherwise the workgroup refolds with v_mul_f32 +
     v_add_f32.  Heads scaled so that products fall in the denormal range
@@ -389,18 +407,15 @@ def test_attention_prefill_mfma_fold_range_guard():
     q16 = oracle.f32_to_bf16_bits_np(q32).reshape(-1)
     k16 = oracle.f32_to_bf16_bits_np(k32)
     v16 = oracle.f32_to_bf16_bits_np(rng.normal(0, 1, (B, H, L, D)).astype(np.float32))
-    q, k, v = ca.Buffer.from_array(q16), ca.Buffer.from_array(k16), ca.Buffer.from_array(v16)
-    lb = ca.Buffer.from_array(np.array(lens, np.uint32))
     scale = 1.0 / math.sqrt(D)
-    o32 = ca.Buffer(B * Tq * H * D * 4)
-    say("prefill attention: MFMA fold range guard (denormal / overflow / edge heads)")
-    ca.attn_causal_bf16(q, k, v, lb, o32, B, Tq, H, L, D, scale, out_f32=True)
-    want = od.attn_causal(q16, k16, v16, lens, B, Tq, H, D, scale)
-    _bitwise(o32.read(np.float32, (B * Tq, H * D)), want)
+    say(f"prefill attention: MFMA fold range guard (denormal / overflow / edge heads), blocks {blocks}")
+    got, _ = _causal_copies(q16, k16, v16, lens, B, Tq, H, L, scale, blocks)
+    _bitwise(got, od.attn_causal(q16, k16, v16, lens, B, Tq, H, D, scale))
 
 
-def test_attention_prefill_pv_products_specials():
-    """The prefill kernel forms the P·V products on the matrix cores with a
+@pytest.mark.parametrize("blocks", [0, 65, 513])
+def test_attention_prefill_pv_products_specials(blocks):
+    """The block kernel forms the P·V products on the matrix cores with a
     zero accumulator (fl(p * v), then the adds on the VALU).  Heads that
     push those products to the edges: head 0 spreads the scores over
     hundreds (exp~ of the shifted scores, wrapped powers of two included,
@@ -428,14 +443,10 @@ def test_attention_prefill_pv_products_specials():
     v16[:, 2] = (rng.integers(1, 0x80, (B, L, D)) | (rng.integers(0, 2, (B, L, D)) << 15)).astype(np.uint16)
     q16 = oracle.f32_to_bf16_bits_np(q32).reshape(-1)
     k16 = oracle.f32_to_bf16_bits_np(k32)
-    q, k, v = ca.Buffer.from_array(q16), ca.Buffer.from_array(k16), ca.Buffer.from_array(v16)
-    lb = ca.Buffer.from_array(np.array(lens, np.uint32))
     scale = 1.0 / math.sqrt(D)
-    o32 = ca.Buffer(B * Tq * H * D * 4)
-    say("prefill attention: P.V products at the edges (tiny p, V specials, denormal V)")
-    ca.attn_causal_bf16(q, k, v, lb, o32, B, Tq, H, L, D, scale, out_f32=True)
+    say(f"prefill attention: P.V products at the edges (tiny p, V specials, denormal V), blocks {blocks}")
+    got, _ = _causal_copies(q16, k16, v16, lens, B, Tq, H, L, scale, blocks)
     want = od.attn_causal(q16, k16, v16, lens, B, Tq, H, D, scale)
-    got = o32.read(np.float32, (B * Tq, H * D))
     _bitwise(got, want)
     # the heads reach the cases they are for
     w = want.reshape(B, Tq, H, D)
@@ -498,24 +509,21 @@ def test_argmax_chunked_nan_and_tie_patterns():
 @pytest.mark.parametrize("B,Tq,H,L,lens", [(2, 37, 3, 200, [200, 37]), (1, 512, 2, 640, [512]),
                                            (3, 8, 2, 96, [96, 8, 30]), (2, 100, 1, 700, [700, 120]),
                                            (1, 12, 2, 1000, [1000]), (1, 20, 2, 1200, [1200])])
-def test_attention_prefill_kernel_equals_per_query_kernel(B, Tq, H, L, lens):
-    """The causal attention (the 16-query-block kernel for Tq >= 8 while its
-    score buffer fits, L <= 1,088; the one-query kernel beyond, as in the
-    last case) against the decode kernel run once per query on that query's
-    prefix (same bits by construction), including cached prefixes
-    (lens > Tq), partial last blocks and sequences shorter than Tq."""
+@pytest.mark.parametrize("blocks", [0, 65, 513])
+def test_attention_prefill_kernel_equals_per_query_kernel(B, Tq, H, L, lens, blocks):
+    """The causal attention (the one-query kernel for few blocks of queries, the
+    block kernel with eight or four waves for more) against the decode kernel
+    run once per query on that query's prefix (same bits by construction),
+    including cached prefixes (lens > Tq), partial last blocks and sequences
+    shorter than Tq."""
     D = 128
     q, k, v = _attn_inputs(B, Tq, H, L, B * 7 + Tq)
-    lb = ca.Buffer.from_array(np.array(lens, np.uint32))
     scale = 1.0 / math.sqrt(D)
-    a32 = ca.Buffer(B * Tq * H * D * 4)
-    a16 = ca.Buffer(B * Tq * H * D * 2)
-    say(f"prefill attention B={B} Tq={Tq} H={H} L={L} lens={lens}")
-    ca.attn_causal_bf16(q, k, v, lb, a32, B, Tq, H, L, D, scale, out_f32=True)
-    ca.attn_causal_bf16(q, k, v, lb, a16, B, Tq, H, L, D, scale, out_f32=False)
-    got = a32.read(np.float32, (B, Tq, H, D))
-    assert np.array_equal(a16.read(np.uint16, (B, Tq, H, D)),
-                          oracle.f32_to_bf16_bits_np(got))
+    say(f"prefill attention B={B} Tq={Tq} H={H} L={L} lens={lens} blocks {blocks}")
+    g32, g16 = _causal_copies(q.read(np.uint16), k.read(np.uint16, (B, H, L, D)), v.read(np.uint16, (B, H, L, D)), lens,
+                              B, Tq, H, L, scale, blocks)
+    assert np.array_equal(g16, oracle.f32_to_bf16_bits_np(g32))
+    got = g32.reshape(B, Tq, H, D)
     q_host = q.read(np.uint16, (B, Tq, H, D))
     ob = ca.Buffer(B * H * D * 4)
     for t in range(Tq):
@@ -527,4 +535,4 @@ def test_attention_prefill_kernel_equals_per_query_kernel(B, Tq, H, L, lens):
     if B * Tq * H <= 4096:
         want = od.attn_causal(q.read(np.uint16), k.read(np.uint16, (B, H, L, D)),
                               v.read(np.uint16, (B, H, L, D)), lens, B, Tq, H, D, scale)
-        _bitwise(a32.read(np.float32, (B * Tq, H * D)), want)
+        _bitwise(g32, want)

@@ -102,16 +102,24 @@ def test_unaligned_operands(n, m, k, shifts):
     _check(n, m, k, shifts)
 
 
-@pytest.mark.parametrize("n,m,k", [(999, 768, 256), (200, 1024, 544), (333, 1536, 160), (1000, 2048, 96)])
-def test_unsplit_bits_equal_the_aligned_kernels(n, m, k):
+# the padded product's depth and narrow tiles: 32-k stages on narrow (129 .. 256)
+# and on wide tiles (257 .. 512), 64-k stages (160 and more)
+@pytest.mark.parametrize("n,m,k,pk,tiles", [
+    (999, 768, 256, 256, 129), (999, 768, 256, 256, 257), (200, 1024, 544, 640, 129), (200, 1024, 544, 576, 160),
+    (333, 1536, 160, 256, 257), (333, 1536, 160, 192, 160), (1000, 2048, 96, 128, 257), (1000, 1920, 96, 128, 129)])
+def test_unsplit_bits_equal_the_aligned_kernels(n, m, k, pk, tiles):
     """A product that is not split has the bits of the same product padded to
-    whole tiles: rows and k rows of zeros change no other cell's MFMA steps."""
+    whole tiles, and repeated until the tile kernels take it: rows and k rows of
+    zeros change no other cell's MFMA steps."""
     a16, b16, g32 = _check(n, m, k)
-    pn, pk = -(-n // 256) * 256, -(-k // 128) * 128
+    assert ca.gemm_bf16_plan(n, m, k)[0] == 1
+    pn = -(-n // 256) * 256
     ap, bp = np.zeros((pn, pk), np.uint16), np.zeros((pk, m), np.uint16)
     ap[:n, :k], bp[:k] = a16, b16
-    say(f"bf16 gemm padded {pn}x{m}x{pk}")
-    full = _product(np.concatenate([ap] * 5)[:5 * pn], bp, True)[:n]
+    copies = -(-tiles // (pn // 256 * -(-m // 128)))
+    say(f"bf16 gemm padded {copies} x {pn}x{m}x{pk}")
+    assert ca.gemm_bf16_plan(copies * pn, m, pk)[2:] == (0, 0)
+    full = _product(np.concatenate([ap] * copies), bp, True)[:n]
     assert np.array_equal(full.view(np.uint32), g32.view(np.uint32))
 
 
@@ -137,8 +145,9 @@ def test_strides_past_the_32_bit_offsets():
     a16 = oracle.f32_to_bf16_bits_np(rng.integers(-1, 2, (n, k)).astype(np.float32))
     b16 = oracle.f32_to_bf16_bits_np(rng.integers(-1, 2, (k, m)).astype(np.float32))
     say(f"bf16 gemm {n}x{m}x{k}")
-    got = _product(a16, b16, True)
-    assert np.array_equal(got, as_f32(a16) @ as_f32(b16).astype(np.float64))
+    want = as_f32(a16) @ as_f32(b16).astype(np.float64)
+    assert np.array_equal(_product(a16, b16, True), want)
+    assert np.array_equal(_product(a16, b16, False), oracle.f32_to_bf16_bits_np(want.astype(np.float32)))
 
 
 @pytest.mark.parametrize("n,m", [(1, 1), (3, 7), (8, 128), (16, 9), (17, 8), (32, 32), (33, 31), (256, 256), (1000, 2056)])

@@ -321,21 +321,26 @@ def test_runtime_programs_random():
 
 
 def test_tile_gemm_paths_random():
-    """Random shapes aimed at each tile path of gemm_bf16: M a multiple of
-    256 with N a multiple of 128 and K a multiple of 128 (32-k kernel, wide
-    or narrow tiles by the host's rule) or of 64 only (64-k kernel), and the
-    same with one dimension off the tile (bounds-checked kernel): the bf16
+    """Random shapes aimed at each path of gemm_bf16: M a multiple of 256
+    with N a multiple of 128 and K a multiple of 128 or of 64 only, of few
+    tiles (general kernels) and of enough for the tile kernels (32-k stages on
+    narrow and on wide tiles, 64-k stages), and the same with one dimension
+    off the tile (general kernels): the bf16
     output within the stated bound of the sequential oracle, bitwise the RNE
     of the f32 output, and bitwise run to run."""
     from gpu_util import as_f32, bf16_ulp_of, U
     rng = np.random.default_rng(83)
-    for i in range(12):
+    tiled = [(2304, 2048, 128), (4096, 2304, 128), (2560, 2048, 192)]
+    assert all(ca.gemm_bf16_plan(*s)[2:] == (0, 0) for s in tiled)
+    for i in range(12 + len(tiled)):
         n = 256 * int(rng.integers(1, 3))
         m = 128 * int(rng.integers(1, 9))
         k = 128 * int(rng.integers(1, 6)) if i % 3 != 1 else 64 * (2 * int(rng.integers(1, 5)) + 1)
         if i % 4 == 3:
             which = int(rng.integers(0, 3))
             n, m, k = (n + 3, m, k) if which == 0 else (n, m + 8, k) if which == 1 else (n, m, k + 8)
+        if i >= 12:
+            n, m, k = tiled[i - 12]
         a = dev_normal_bf16(n * k, 1100 + i, 0, 1.0)
         b = dev_normal_bf16(k * m, 1100 + i, 1, 1.0)
         c16, c32 = ca.Buffer(n * m * 2), ca.Buffer(n * m * 4)
@@ -358,10 +363,10 @@ def test_tile_gemm_paths_random():
 
 def test_attention_long_and_prefill_boundary_random():
     """Decode attention at random long caches (up to 6000 positions) and the
-    causal form around the prefill kernel's cache limit (max_len 1,088: the
-    score matrix of whole 64-key blocks fits 80 KB of LDS; the one-query
-    kernel beyond it), at the limit, one past it and at random lengths:
-    bitwise the oracle."""
+    causal form around 1,088 rows (two blocks' score matrices of whole 64-key
+    blocks share a CU up to there), at the limit, one past it and at random
+    lengths, on the one-query kernel and, laid side by side for more blocks of
+    queries, on the block kernel: bitwise the oracle."""
     D = 128
     rng = np.random.default_rng(84)
     for i in range(4):
@@ -388,21 +393,30 @@ def test_attention_long_and_prefill_boundary_random():
         lb, o = ca.Buffer.from_array(np.array(lens, np.uint32)), ca.Buffer(B * Tq * H * D * 4)
         say(f"causal attention near the prefill limit B={B} Tq={Tq} H={H} L={L} lens={lens}")
         ca.attn_causal_bf16(q, k, v, lb, o, B, Tq, H, L, D, scale, out_f32=True)
-        want = od.attn_causal(q.read(np.uint16), k.read(np.uint16, (B, H, L, D)),
-                              v.read(np.uint16, (B, H, L, D)), lens, B, Tq, H, D, scale)
+        q16, k16, v16 = q.read(np.uint16), k.read(np.uint16, (B, H, L, D)), v.read(np.uint16, (B, H, L, D))
+        want = od.attn_causal(q16, k16, v16, lens, B, Tq, H, D, scale)
         _bits_nan_aware(o.read(np.float32, (B * Tq, H * D)), want)
+        c = max(-(-65 // (B * H * -(-Tq // 16))), -(-2561 // (B * H * Tq)))  # copies: the block kernel
+        qc, kc, vc, lc = (ca.Buffer.from_array(np.tile(x.reshape(-1), c)) for x in (q16, k16, v16, np.array(lens, np.uint32)))
+        oc = ca.Buffer(c * B * Tq * H * D * 4)
+        ca.attn_causal_bf16(qc, kc, vc, lc, oc, c * B, Tq, H, L, D, scale, out_f32=True)
+        got = oc.read(np.float32, (c, B * Tq, H * D))
+        _bits_nan_aware(got[0], want)
+        assert np.array_equal(got.view(np.uint32), np.broadcast_to(got[:1].view(np.uint32), got.shape))
 
 
 def test_bf16_gemm_special_values_random():
     """NaN, +-inf and zeros at random positions of A and B (finite values of
     moderate size, so no partial sum overflows): for every path of gemm_bf16
-    (decode, tile, edge), each output is NaN exactly where the exact product
+    (decode, the tile kernels of each width and stage, general), each output is NaN exactly where the exact product
     is (a NaN input, inf * 0, or infinities of both signs in the sum),
     +-inf exactly where it is, and finite elsewhere; the bf16 output is the
     RNE of the f32 output."""
     from gpu_util import as_f32
     rng = np.random.default_rng(85)
-    shapes = [(8, 1024, 512), (16, 520, 96), (256, 256, 256), (512, 384, 192), (300, 200, 100)]
+    shapes = [(8, 1024, 512), (16, 520, 96), (256, 256, 256), (512, 384, 192), (300, 200, 100),
+              (2560, 1664, 128), (4096, 2304, 128), (2560, 2048, 64)]
+    assert all(ca.gemm_bf16_plan(*s)[2:] == (0, 0) for s in shapes[-3:])
     for i, (n, m, k) in enumerate(shapes):
         a = rng.normal(0, 1, (n, k)).astype(np.float32)
         b = rng.normal(0, 1, (k, m)).astype(np.float32)
