@@ -28,8 +28,9 @@ CATENA_DEV float bf16_to_f32(uint16_t h) { return __uint_as_float(((uint32_t)h) 
 
 // f32 -> bf16 round-to-nearest-even; NaN keeps sign and top payload and is
 // made quiet.  v_cvt_pk_bf16_f32 gives the bits of the CPU oracle's integer
-// form (or_f32_to_bf16) for each of the 2^32 inputs, in one instruction for two
-// values against eight each.
+// form (or_f32_to_bf16), signs and payloads of NaNs included (tests/
+// test_rounding.py: every high half with the low halves around the tie), in one
+// instruction for two values against eight each.
 CATENA_DEV uint32_t f32_to_bf16_bits(float x) {
   return __builtin_bit_cast(uint16_t, (__bf16)x);
 }
@@ -353,18 +354,21 @@ CATENA_DEV float serial_sum_wave_long(const float* s, uint32_t n) {
 }
 
 // Correctly rounded quotients by one divisor that many elements share, in four
-// fused steps an element and the fixup that ends every division here (the
-// compiler's takes about twelve, one of them a quarter-rate reciprocal).  hi =
+// fused steps an element (the compiler's division takes about twelve, one of
+// them a quarter-rate reciprocal) and the division fixup, which changes no value
+// here: it marks each of these divisions in the machine code, whose check
+// allows fused steps in divisions alone.  hi =
 // RN(1/b), lo = RN((1 - b hi) hi), the first remainder exact, so hi + lo = 1/b (1
 // + 2^-47); q0 = fma(a, hi, a lo) is then within one ulp of a / b, its remainder
 // fma(-b, q0, a) is exact and fma(remainder, hi, q0) is the correctly rounded
 // quotient (P. Markstein, "Computation of elementary functions on the IBM RISC
 // System/6000 processor", 1990: a faithful quotient and a correctly rounded
-// reciprocal give it).  The bounds keep every step in the normal range: b in
-// [2^-20, 2^20] and the |a| of a group in [2^-98, 2^100] give |a / b| >= 2^-118
-// and remainders that are multiples of 2^-146.  Groups outside them, zeros
-// included, take the plain division; 4.3e9 pairs, near ties and with extreme
-// mantissas among them, gave its bits.
+// reciprocal give it).  Bounds: b in [2^-20, 2^20] and the |a| of a group in
+// [2^-98, 2^100] give 2^-118 <= |a / b| <= 2^120, normal.  The remainder is a
+// multiple of 2^-146 and exact as a subnormal; a lo, subnormal below 2^-126, is
+// off by 2^-150 at most, 2^-32 of the quotient.  Both need subnormals kept, as
+// these kernels are compiled.  Groups outside the bounds, zeros included, take
+// the plain division.  tests/test_rounding.py holds the steps against it.
 struct SharedDivisor {
   float b, hi, lo;
   bool fast;
