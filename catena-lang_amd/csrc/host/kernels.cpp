@@ -68,12 +68,12 @@ uint32_t decode_kw(uint64_t n_cols, uint64_t k, bool regs_path) {
 // `alone` and `shared`: microseconds per 32-k slab of one workgroup that has
 // its CU to itself, and of each of the `fit` workgroups that share a CU;
 // `stream`: GB/s at which one CU brings a weight in from HBM (the narrower
-// the tile's rows, the less).  Fitted to 2,900 timings of five general
-// kernels and the ragged 256 x 256 one over n = 17 .. 4000, widths 256 ..
-// 11264 and depths 512 .. 11008, 1 to 16 k groups: the tile it picks is on
-// average 2.4 % from the fastest (1.22x at worst, 0.5 % without k groups).
-// The 192 x 128 and 128 x 192 rows come from 150 more; where the choice moved to
-// them, 13 of 400 drawn products, those take 10 % less on average, none longer.
+// the tile's rows, the less).  Fitted to timings over n = 17 .. 4000, widths
+// 256 .. 11264 and depths 512 .. 11008, 1 to 16 k groups.  On 110 other products
+// of n = 17 .. 4000, widths 256 .. 11008 and depths 128 .. 11008, with every tile
+// and number of groups timed, the choice takes 3.6 % more than the fastest on
+// average and 18 % at worst, of which the timing's spread is up to 10, and 6.5 %
+// less than the fastest undivided one.
 struct GemmTile {
   KernelId f32, bf16;
   uint32_t bm, bn, waves, stages, stage_k, fit;
