@@ -50,9 +50,11 @@
 //
 // What bounds it: issue on the VALU, which the f32 matrix instructions occupy
 // too (measured: 32 cycles of a SIMD per 16x16x1 instruction and about 2.4 per
-// add, added up, at four waves per SIMD; 2.6 to 4.2 per add at two).  At C5's
-// 512 keys and four workgroups per CU that is 90 % filled.  Where the score
-// buffer leaves one or two workgroups to a CU, eight waves instead of four keep
+// add, added up, at four waves per SIMD; 2.6 to 4.2 per add at two), and the
+// phases between barriers, in which fewer waves have work.  By the counters
+// issue takes 72 % of the SIMDs' cycles for 512 queries over 512 keys, four
+// workgroups to a CU, 65 % over 640-row caches, three to a CU, and 59 % for 2000
+// queries; waves wait a third of the time.  Where the score buffer leaves one or two workgroups to a CU, eight waves instead of four keep
 // the SIMDs busier, and each load, LDS read and matrix instruction is issued
 // ahead of the adds it would hold up: 2000 queries x 16 heads in a 2048-row
 // cache 1400 us (one query per workgroup) -> 583 (four waves) -> 470 (eight) ->
