@@ -65,6 +65,18 @@ def test_general_shapes(n, m, k):
     _check(n, m, k)
 
 
+# every tile, stored four or eight columns at a time and by the element
+@pytest.mark.parametrize("n,m,k,tile", [
+    (30, 79, 79, (32, 32)), (17, 248, 12, (32, 32)), (37, 4241, 80, (32, 64)), (33, 4172, 76, (32, 64)),
+    (78, 5591, 67, (64, 64)), (69, 5488, 77, (64, 64)), (2051, 109, 9, (64, 128)), (40, 4316, 15, (64, 128)),
+    (1869, 2342, 8, (128, 128)), (666, 5908, 8, (128, 128)), (2122, 5457, 43, (128, 192)), (2009, 6096, 8, (128, 192)),
+    (1483, 5917, 8, (192, 128)), (1670, 4736, 8, (192, 128)), (1745, 2398, 9, (256, 256)), (726, 5380, 9, (256, 256)),
+    (1000, 6144, 2048, (128, 128))])
+def test_each_tile(n, m, k, tile):
+    assert ca.gemm_bf16_plan(n, m, k) == (1, k) + tile
+    _check(n, m, k)
+
+
 # the 256 x 256 tile with ragged edges (the tile the host's estimate takes for
 # these): 1, 15, 16, 17 rows in the last tile; 1, 15, 17 k rows in the last slab
 # and slabs past k; B packed, A packed, both, none
