@@ -53,7 +53,7 @@ def _check(n, m, k, shift=0, special=False):
     (32, 90000, 7), (17, 90001, 8), (31, 90001, 9), (1089, 2561, 40), (1120, 2560, 41), (1121, 2562, 55),
     # 64 x 64 tiles: few k, at and past a slab of 16; 4 x 1 at 64 columns and 16 x 16 at 16, next to them
     (1280, 1025, 15), (1281, 1088, 1), (1536, 2047, 23), (2049, 1537, 31), (1537, 2048, 24), (20000, 64, 33), (20000, 65, 33),
-    (30001, 16, 48), (30001, 16, 33), (30001, 17, 48), (70000, 1, 65),
+    (30001, 16, 48), (30001, 16, 33), (30001, 17, 48), (70000, 1, 65), ((1 << 20) - 15, 3, 32), ((1 << 20) + 21, 1, 33),
     # two tiles for each of 256 CUs (three past 3 MiB of operands), 6.5 of the DPP form
     (512, 256, 17), (513, 255, 17), (522, 256, 1011), (522, 256, 1010), (769, 250, 801), (1664, 256, 16), (1665, 256, 16)])
 def test_row_forms(n, m, k):
