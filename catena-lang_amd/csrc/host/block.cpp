@@ -15,6 +15,35 @@ namespace {
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
+// Four rows of an RMSNorm to a workgroup, or one: once there are more rows than
+// one round of one-row workgroups takes, and two of the larger ones fit a CU,
+// four while their rounds, each longer than a one-row round, are fewer by more
+// than that.  A round of fours takes 1.5 of the others when the row alone is
+// read, 1.75 with an index, a table or a second output (extra 1), for which a
+// lane has fewer loads in flight, about 2 with a residual (extra 2); rows under
+// 1600 values, three or more of whose rounds go into one of fours, always win.
+// Measured, one against four, us:
+//   rows alone   4096 x 2048 24.2 / 17.3, 4096 x 3584 49 / 42, 6200 x 3584 66 / 76
+//   index        4096 x 2048 25.3 / 20.5, 4097 x 2048 25.5 / 27.0, 8192 x 3072 68 / 75
+//   residual     4096 x 2048 28.8 / 24.5, 8192 x 2048 45.1 / 46.4, 2049 x 2048 17.3 /
+//                18.2, 8192 x 1536 38 / 35, 4096 x 4096 68 / 64, 4097 x 4096 70 / 76
+// Rows of n % 4 != 0 go value by value in the four-row form: with anything
+// beside them only short ones, of more than 1024 values where that fills half a
+// round of fours or all of one (4096 x 1030 20.1 / 17.4, 6200 x 1030 28.0 / 30.6,
+// 16384 x 1030 60 / 53, 4097 x 2050 36 / 49).
+static bool rms_rows4(uint64_t rows, uint64_t n, uint32_t slot, int extra) {
+  const uint64_t cus = (unsigned)device().cu_count;
+  const uint64_t round1 = cus * std::min<uint64_t>(8, lds_fit(rmsnorm_lds_bytes(n)));
+  const uint64_t round4 = cus * 4 * std::min<uint64_t>(8, rows4_per_cu(slot));
+  if (rows <= round1 || rows4_per_cu(slot) < 2) return false;
+  if (n % 4 != 0 && extra)
+    return n <= 1024 || (n <= 1536 && (rows >= round4 || (2 * rows >= 3 * round1 && 2 * rows <= round4)));
+  if (n < 1600) return true;
+  const uint64_t c1 = ceil_div(rows, round1), c4 = ceil_div(rows, round4);
+  if (extra < 2) return extra == 0 ? 3 * c4 < 2 * c1 : 7 * c4 < 4 * c1;
+  return c4 == 1 ? n >= 2500 || 5 * rows >= 3 * round4 : n >= 3500 && 19 * c4 < 10 * c1;
+}
+
 int rmsnorm_launch(const float* x, const float* resid, const uint32_t* row_index, float* h_out,
                    float* y_f32, uint16_t* y_bf16, uint64_t rows, uint64_t n,
                    const uint32_t* tokens = nullptr, const uint16_t* table = nullptr,
@@ -46,14 +75,9 @@ int rmsnorm_launch(const float* x, const float* resid, const uint32_t* row_index
   if (resid_parts == 0 || (resid_parts > 1 && (!resid || (n % 4 == 0 && resid_stride % 4 != 0))))
     return fail(CATENA_ERR_INVALID_ARGUMENT, "rmsnorm residual partials");
   uint32_t n32 = (uint32_t)n, rows32 = (uint32_t)rows;
-  // Four rows to a workgroup (their folds then cost the VALU a quarter) once
-  // there are more rows than one round of one-row workgroups takes, and two of
-  // the larger ones fit a CU.  Measured, one against four: 2048 x 2048 14.1 / 14.9
-  // us, 4096 x 2048 25.8 / 19.1, 32001 x 2048 148 / 111, 16384 x 512 28.7 / 19.7,
-  // 1536 x 4096 28.8 / 23.1, 8192 x 6000 219 / 246.
-  const uint64_t round = (uint64_t)device().cu_count * std::min<uint64_t>(8, device().max_lds / rmsnorm_lds_bytes(n));
-  uint32_t slot = rows > round ? rows4_slot(n) : 0;
-  if (slot && rows4_per_cu(slot) < 2) slot = 0;
+  // Four rows to a workgroup (their folds then cost the VALU a quarter)?
+  uint32_t slot = rows4_slot(n);
+  if (slot && !rms_rows4(rows, n, slot, resid ? 2 : h_out || row_index || !x ? 1 : 0)) slot = 0;
   void* args[] = {&x,     &resid, &row_index,   &h_out,        &y_f32,     &y_bf16, &n32, &tokens,
                   &table, &vocab, &resid_parts, &resid_stride, &resid_out, &rows32, &slot};
   if (slot)

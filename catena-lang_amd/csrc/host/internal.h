@@ -213,10 +213,10 @@ inline uint32_t rows4_slot(uint64_t n) {
   const uint64_t n4 = (n + 3) / 4 * 4, slot = n4 + n4 / 32 * 4 + 4;
   return n4 <= 16384 && 4 * slot * sizeof(float) + 64 <= device().max_lds ? (uint32_t)slot : 0;
 }
-// such workgroups that one CU's LDS holds
-inline uint32_t rows4_per_cu(uint32_t slot) {
-  return (uint32_t)(device().max_lds / (4 * (size_t)slot * sizeof(float) + 64));
-}
+// workgroups of so many bytes that one CU's LDS, given out in pieces of 1280
+// bytes, holds
+inline uint64_t lds_fit(uint64_t bytes) { return device().max_lds / ((bytes + 1279) / 1280 * 1280); }
+inline uint32_t rows4_per_cu(uint32_t slot) { return (uint32_t)lds_fit(4 * (uint64_t)slot * sizeof(float) + 64); }
 int ensure_init();
 int fail(int status, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 void clear_error();

@@ -754,7 +754,7 @@ int catena_mi355x_softmax_f32(const float* x, float* y, uint64_t rows, uint64_t 
     return launch(vec ? KernelId::SoftmaxRows4Vec : KernelId::SoftmaxRows4, dim3((unsigned)ceil_div(rows, 4)),
                   dim3(256), 4 * (size_t)slot * sizeof(float), lds_args);
   const uint64_t row_lds = ceil_div(n, 4) * 4 * sizeof(float), cus = (unsigned)device().cu_count;
-  const uint64_t fit = device().max_lds / (row_lds + 64);
+  const uint64_t fit = lds_fit(row_lds + 64);
   if (fit >= 3 || (fit > 0 && rows <= 3 * fit * cus) || (fit == 2 && rows > 8 * cus))
     return launch(vec ? KernelId::SoftmaxRowVec : KernelId::SoftmaxRow, dim3((unsigned)rows), dim3(256),
                   row_lds, lds_args);

@@ -81,17 +81,19 @@ static int sum_launch(const float* x, float* out, uint64_t rows, uint64_t n, uin
   st = ensure_init();
   if (st) return st;
   void* args[] = {&x, &out, &n, &mean};
-  // Rows that fit LDS, four to a workgroup: while all of those run at once, or
-  // three of them fit a CU; else one wave per row, straight from memory.
+  // Rows that fit LDS, four to a workgroup: while all of those run at once, and
+  // beyond where four of them fit a CU (three, for rows that the other form would
+  // read value by value); else one wave per row, straight from memory.
   // Measured, wave against four rows: 1 x 2048 8.5 / 7.2 us, 4096 x 2048 17.0 /
   // 12.3, 4096 x 2047 32.3 / 12.9, 1000 x 8192 33.1 / 28.1, 2048 x 8192 34.5 /
-  // 54.5, 4096 x 4096 28.5 / 33.0.
+  // 54.5, 4096 x 4096 28.5 / 33.0, 2500 x 2560 17.6 / 10.3, 4096 x 2560 20.7 / 21.6,
+  // 16384 x 2816 58 / 73, 4096 x 2818 42 / 27.
   uint32_t slot = rows4_slot(n);
   const uint32_t fit = slot ? rows4_per_cu(slot) : 0;
-  if (fit >= 3 || rows <= 4ull * fit * (unsigned)device().cu_count) {
+  const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+  if (fit >= (vec ? 4 : 3) || rows <= 4ull * fit * (unsigned)device().cu_count) {
     uint32_t n32 = (uint32_t)n;
     void* args4[] = {&x, &out, &rows, &n32, &mean, &slot};
-    const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
     return launch(vec ? KernelId::SumRows4VecF32 : KernelId::SumRows4F32, dim3((unsigned)((rows + 3) / 4)), dim3(256),
                   4 * (size_t)slot * sizeof(float), args4);
   }

@@ -79,7 +79,7 @@ def test_softmax(rows, n, shift):
 
 
 @pytest.mark.parametrize("rows,n", [(1, 0), (1, 1), (7, 3), (6, 2048), (5, 513), (1025, 8192), (4099, 36), (9, 9088),
-                                    (9, 9089), (1025, 6001)])
+                                    (9, 9089), (1025, 6001), (3072, 2816), (3073, 2816), (3073, 2818), (4097, 2224), (4097, 2272)])
 @pytest.mark.parametrize("shift", [0, 4])
 def test_sum(rows, n, shift):
     say(f"sum rows {rows} n {n} shift {shift}")
@@ -110,13 +110,13 @@ def test_rmsnorm(rows, n):
         _same(got[i], oracle.rmsnorm_f32(x[i]))
 
 
-@pytest.mark.parametrize("n", [256, 260, 1024, 1030])
+@pytest.mark.parametrize("rows,n", [(2305, 256), (2305, 260), (2305, 1024), (2305, 1030), (2305, 514), (2305, 1023), (3200, 1030),
+                                    (2305, 1596), (2305, 2044), (2500, 2048), (1300, 4096), (2049, 4096)])
 @pytest.mark.parametrize("parts", ["resid", "index", "both"])
-def test_residual_rmsnorm_bf16(n, parts):
+def test_residual_rmsnorm_bf16(rows, n, parts):
     """The same norm with the residual add, the gather of rows, and both
     outputs, against the one-row form (fewer rows at a time)."""
-    rows = 2305
-    say(f"residual rmsnorm n {n} {parts}")
+    say(f"residual rmsnorm {rows} x {n} {parts}")
     x, _ = _rows(rows, n, n)
     rng = np.random.default_rng(n + 1)
     r = rng.standard_normal((rows, n)).astype(np.float32)
@@ -137,9 +137,9 @@ def test_residual_rmsnorm_bf16(n, parts):
         ca.residual_rmsnorm_bf16(xb, rb, None, h2, y2, rows, n)
         assert np.array_equal(h2.read(np.uint32).reshape(rows, n), h)
         assert np.array_equal(y2.read(np.uint16).reshape(rows, n), y)
-    for a in range(0, rows, 1024):
-        hs, ys = run(index[a:a + 1024])
-        assert np.array_equal(h[a:a + 1024], hs) and np.array_equal(y[a:a + 1024], ys)
+    for a in range(0, rows, 1000):
+        hs, ys = run(index[a:a + 1000])
+        assert np.array_equal(h[a:a + 1000], hs) and np.array_equal(y[a:a + 1000], ys)
 
 
 # whole and partial 512-value chunks, the longest rows of the bf16 form and the
