@@ -92,10 +92,11 @@ extern "C" __global__ __launch_bounds__(256) void catena_softmax_rows_f32(
 // The same for rows that fit LDS: a row is read once and written once and kept
 // in LDS between, one row to a workgroup, or (ROWS == 4) a wave to a row and
 // wave 0 folds the four denominators together (serial_sum_rows4).
-// The maximum: when a row holds no NaN, the fold's result is the largest value,
-// and its bits are the value's own unless it is a zero (of which the first one's
-// sign counts); a row with a NaN or a zero maximum takes the exact parallel form
-// over LDS.  VEC: n % 4 == 0 and 16-byte aligned rows.
+// The maximum: when a row holds no NaN, the fold's result is the largest value
+// (of zeros the first one, whose sign changes no output: x - 0 is x, and exp~ of
+// either zero is the same); a row with a NaN takes the exact parallel form over
+// LDS, all of the row's threads together.  VEC: n % 4 == 0 and 16-byte aligned
+// rows.
 // What bounds the four-row form: at 4096 x 2048 it is one round of workgroups,
 // so its phases follow one another: both passes over memory about 13 us, exp~
 // and the division (35 and 12 instructions per value) about 7, the chain of adds
@@ -110,6 +111,7 @@ CATENA_DEV void softmax_lds_body(const float* x, float* y, uint64_t rows, uint32
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float den_s[ROWS], top_s[4];
   __shared__ int nan_s[4];
+  __shared__ uint32_t at_s[4];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, tid = threadIdx.x % T;
   float* s = reinterpret_cast<float*>(smem) + (ROWS == 4 ? wave * slot : 0);
   const uint64_t row = (uint64_t)blockIdx.x * ROWS + (ROWS == 4 ? wave : 0);
@@ -146,18 +148,35 @@ CATENA_DEV void softmax_lds_body(const float* x, float* y, uint64_t rows, uint32
     mx = __builtin_fmaxf(__builtin_fmaxf(top_s[0], top_s[1]), __builtin_fmaxf(top_s[2], top_s[3]));
     anynan = (nan_s[0] | nan_s[1] | nan_s[2] | nan_s[3]) != 0;
   }
-  if (anynan || mx == 0.0f) {  // the same for every thread of the row; each wave for itself
+  if (anynan) {  // the same for every thread of the row
     int lastnan = -1;
-    for (uint32_t t = lane; t < n; t += 64)
+    for (uint32_t t = tid; t < n; t += T)
       if (s[row_at<ROWS>(t)] != s[row_at<ROWS>(t)]) lastnan = (int)t;
     lastnan = wave_max_i32(lastnan);
+    if (ROWS == 1) {
+      __syncthreads();  // top_s and nan_s have been read
+      if (lane == 0) nan_s[wave] = lastnan;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < 4; ++w) lastnan = nan_s[w] > lastnan ? nan_s[w] : lastnan;
+    }
     if (lastnan == (int)n - 1) {
       mx = s[row_at<ROWS>(n - 1)];
     } else {
       FirstMax fm{lowest, 0xFFFFFFFFu};
-      for (uint32_t t = lastnan + 1 + lane; t < n; t += 64)
+      for (uint32_t t = lastnan + 1 + tid; t < n; t += T)
         fm = first_max_combine(fm, FirstMax{s[row_at<ROWS>(t)], t});
       fm = wave_first_max(fm);
+      if (ROWS == 1) {
+        if (lane == 0) {
+          top_s[wave] = fm.v;
+          at_s[wave] = fm.i;
+        }
+        __syncthreads();
+        fm = FirstMax{top_s[0], at_s[0]};
+#pragma unroll
+        for (int w = 1; w < 4; ++w) fm = first_max_combine(fm, FirstMax{top_s[w], at_s[w]});
+      }
       mx = fm.i == 0xFFFFFFFFu ? lowest : fm.v;
     }
     if (ROWS == 1) __syncthreads();  // every wave has read the row
